@@ -361,30 +361,48 @@ __device__ __forceinline__ void place_item(int s, const uint32_t *__restrict__ k
 // In neighbour-list mode the re-sort runs only on timesteps whose gate the
 // previous step set.  Its kernels (bin, scan, place, then the list build)
 // can run as one launch, so a timestep without a rebuild costs one launch that
-// returns at once instead of four.
+// returns at once instead of four (1.8 us each).
 //
-// The phases are ordered by a work queue, not by grid barriers.  The launch's
-// work is a sequence of items -- bin chunks, scan tiles, place chunks, then
-// list-build tiles -- that blocks claim one at a time with an atomic counter,
-// in increasing order.  Before it works on an item of phase p a block waits
-// until every item of phase p - 1 is finished.  Those items were all claimed
-// before this one, so each is held by a block that is already running and
-// stays resident until it is done; phase-0 items wait for nothing.  By
-// induction over the phases every wait ends whether or not the launch's
-// blocks fit on the device at once, and whatever else runs beside it (other
-// simulations' launches on other streams).  A block that finds the queue
-// empty leaves; the last one out resets the queue for the next launch.
+// Its phases are ordered by a work queue, not by grid barriers.  The re-sort
+// is a sequence of items -- bin chunks, scan tiles, place chunks -- that blocks
+// claim one at a time with an atomic counter, in increasing order.  Before it
+// works on an item of phase p a block waits until every item of phase p - 1
+// is finished.  Those items were all claimed before this one, so each is held
+// by a block that is already running and stays resident until it is done;
+// phase-0 items wait for nothing.  By induction over the phases every wait ends
+// whether or not the launch's blocks fit on the device at once, and whatever
+// else runs beside it (other simulations' launches on other streams).  A block
+// that finds no items left waits for the last place item in the same way and
+// then builds its share of the tiles' lists, which nothing in the launch waits
+// for and which it therefore need not claim.  Timesteps use two queues in
+// turn, and each launch resets the other one.
 
-// Work-queue state of one agent type (device memory, zero between launches).
+// Work-queue state of one agent type (device memory, zero before a rebuild),
+// each counter on a cache line of its own: blocks poll one of them while others
+// add to the rest.
+constexpr int kQueueLine = 32;  // words
 struct RebuildQueue {
-  uint32_t next;     // items claimed
-  uint32_t done[4];  // items finished, per phase
-  uint32_t exited;   // blocks that found the queue empty
-  uint32_t error;    // a wait ran past its spin limit (a safety net: by the
-                     // argument above no wait can, unless the limit is forced)
-  uint32_t pad;
+  uint32_t next;  // items claimed
+  uint32_t pad0[kQueueLine - 1];
+  struct Done {
+    uint32_t n;   // items of the phase finished
+    uint32_t pad[kQueueLine - 1];
+  } done[3];
 };
-static_assert(sizeof(RebuildQueue) == 32, "the queue occupies eight words of the gate block");
+// The gate block of an agent type: words 0-15 gates, counts and the error flag
+// (a wait ran past its spin limit -- a safety net: by the argument above no
+// wait can, unless the limit is forced), from word kGateQueue on the queues of
+// the even and the odd timesteps.
+constexpr int kGateError = 8;
+constexpr int kGateQueue = kQueueLine;
+constexpr int kGateWords = kGateQueue + 2 * (int) (sizeof(RebuildQueue) / 4);
+
+// Ready for its next rebuild (one thread, of a later launch than the last one
+// that used it).
+__device__ __forceinline__ void queue_reset(RebuildQueue *q) {
+  q->next = 0u;
+  for (int p = 0; p < 3; p++) q->done[p].n = 0u;
+}
 
 // Everything the re-sort phases read and write.
 struct DeltaArgs {
@@ -403,7 +421,9 @@ struct DeltaArgs {
   GatherCols gc;              // current -> other buffers
   const int32_t *id_in;
   int32_t *id_out;
-  RebuildQueue *q;
+  RebuildQueue *q;            // this timestep's queue
+  RebuildQueue *q_other;      // the queue of the timesteps before and after
+  uint32_t *error;
   uint32_t spins;             // spin limit of one phase wait (kPhaseSpins)
   unsigned blocks;            // launch size (0: as many blocks as the CUs hold at once)
   int *launched;              // host: set to 1 when the launch function launched it
@@ -413,14 +433,20 @@ struct DeltaArgs {
 // above any phase of a rebuild.
 constexpr uint32_t kPhaseSpins = 1u << 22;
 
-// Items per phase of a launch with blocks of 256 threads.
-struct QueuePlan {
-  uint32_t end[4];  // exclusive end of each phase's items
-  __device__ __host__ int phase_of(uint32_t item) const {
-    return item < end[0] ? 0 : item < end[1] ? 1 : item < end[2] ? 2 : 3;
+// The work of one phase, `units` pieces of 256 threads each (bin and place
+// chunks, scan tiles), as items of `per` units each: about one item per block.
+// An item ends in a release at agent scope, which writes the XCD's whole L2
+// back, and is claimed with an atomic on one address, so a rebuild pays for
+// the number of items far more than for the work in them.
+struct QueuePhase {
+  uint32_t units, per, items;
+  __device__ __host__ static QueuePhase of(uint32_t units, uint32_t blocks) {
+    QueuePhase p;
+    p.units = units;
+    p.per = units > blocks ? (units + blocks - 1u) / blocks : 1u;
+    p.items = (units + p.per - 1u) / p.per;
+    return p;
   }
-  __device__ __host__ uint32_t first(int p) const { return p == 0 ? 0u : end[p - 1]; }
-  __device__ __host__ uint32_t items(int p) const { return end[p] - first(p); }
 };
 
 // Claim the block's next item (block-uniform result).
@@ -433,58 +459,49 @@ __device__ __forceinline__ uint32_t queue_claim(RebuildQueue *q) {
   return claimed;
 }
 
-// Wait until `count` items of phase p are finished.  Thread 0 waits with an
-// acquire load; after the block barrier every thread acquires at agent scope
-// too, so its reads see the finished phase's writes from every XCD.  Returns
+// Wait until `count` items of phase p are finished.  Thread 0 waits, then
+// acquires at agent scope (which drops the CU's L1 and the XCD's stale L2 lines
+// for the whole block) and the block barrier orders every thread's later reads
+// behind it, so they see the finished phase's writes from every XCD.  A block
+// waits once per phase: what it read after that wait stays cached.  Returns
 // false when the wait ran past the spin limit or another block's did.
-__device__ __forceinline__ bool queue_wait(RebuildQueue *q, int p, uint32_t count, uint32_t spins) {
+__device__ __forceinline__ bool queue_wait(RebuildQueue *q, int p, uint32_t count, uint32_t spins,
+                                           uint32_t *error) {
   __shared__ int ok;
   if (threadIdx.x == 0) {
     int good = 1;
     for (uint32_t spin = 0;; spin++) {
-      if (__hip_atomic_load(&q->done[p], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT) >= count) break;
+      if (__hip_atomic_load(&q->done[p].n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= count) break;
       if (spin >= spins ||
-          __hip_atomic_load(&q->error, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u) {
-        __hip_atomic_fetch_or(&q->error, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          __hip_atomic_load(error, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u) {
+        __hip_atomic_fetch_or(error, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         good = 0;
         break;
       }
       __builtin_amdgcn_s_sleep(4);
     }
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
     ok = good;
   }
   __syncthreads();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
   return ok != 0;
 }
 
-// Mark the block's item of phase p finished: every thread releases its writes
-// at agent scope before the block barrier, then thread 0 counts the item.
+// Mark the block's item of phase p finished: every wave waits until its
+// writes have reached the L2, the block barrier gathers them, and thread 0
+// alone releases them at agent scope and counts the item.  (A release by every
+// wave writes the L2 back four times per item.)
 __device__ __forceinline__ void queue_finish(RebuildQueue *q, int p) {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-  __syncthreads();
-  if (threadIdx.x == 0)
-    __hip_atomic_fetch_add(&q->done[p], 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// The last block out of a launch zeroes the queue for the next one.  Every
-// block leaves only after finishing the items it claimed, so when the last
-// one leaves every item is done.
-__device__ __forceinline__ void queue_exit(RebuildQueue *q) {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
   if (threadIdx.x == 0) {
-    const uint32_t e =
-        __hip_atomic_fetch_add(&q->exited, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
-    if (e == gridDim.x - 1u) {
-      __hip_atomic_store(&q->next, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      for (int p = 0; p < 4; p++)
-        __hip_atomic_store(&q->done[p], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __hip_atomic_store(&q->exited, 0u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+    __hip_atomic_fetch_add(&q->done[p].n, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 }
 
-// One item of the re-sort's phases 0-2 (blockDim.x == kScanBlock == 256):
+// One unit of the re-sort's phases 0-2 (blockDim.x == kScanBlock == 256):
 // bin chunk, scan tile, or place chunk `k` of its phase.
 template <typename P>
 __device__ __forceinline__ void delta_item(const DeltaArgs &d, int phase, uint32_t k,

@@ -186,8 +186,8 @@ struct AgentStore {
   uint4 *nl_prow0 = nullptr;    // per own slot: that agent's first list row
   double *nl_pos0 = nullptr;
   uint32_t *nl_gate = nullptr;  // [0..1] rebuild gates by timestep parity, [2] longest list,
-                                // [4] gated rebuilds run,
-                                // [8..15] work queue of the one-launch rebuild
+                                // [4] gated rebuilds run, [kGateError] a rebuild was
+                                // abandoned, from kGateQueue on: the work queues
   int nl_cap = 0;               // entries per agent
   size_t nl_ncap = 0;           // agents allocated
   // the rebuild rate of list mode (list_rate): a pinned copy of the device's
@@ -356,7 +356,7 @@ static size_t store_bytes(const AgentStore &s) {
   b += s.cap * (4 + 4 + 4 + 8 + 8);        // key, tmp_idx, tmp_id, skey x2, mover next
   const size_t tiles = (s.cells_cap + 2047) / 2048;
   b += s.cells_cap * (4 + 8 + 4 + 8) + std::max<size_t>(tiles, 1) * 4;  // count, start x2, dirty, head; bsum
-  if (s.nl_idx) b += s.nl_ncap * ((size_t) s.nl_cap * 2 + kListMetaBytes) + 16 * 4;
+  if (s.nl_idx) b += s.nl_ncap * ((size_t) s.nl_cap * 2 + kListMetaBytes) + kGateWords * 4;
   b += s.bcap * col_bytes(s);              // newborn staging
   return b;
 }
@@ -913,6 +913,11 @@ extern "C" int abl_hip_get_param(abl_sim *sim, const char *name, double *value) 
   return fail(ABL_ERR_ARG, std::string("Unknown parameter \"") + name + "\"");
 }
 
+// The error flag and the work queues of the one-launch rebuild, cleared.
+static hipError_t reset_queues(abl_sim *sim, AgentStore &s) {
+  return hipMemsetAsync(s.nl_gate + kGateError, 0, (kGateWords - kGateError) * 4, sim->stream);
+}
+
 extern "C" int abl_hip_set_config(abl_sim *sim, const char *key, const char *value) {
   CHECK_SIM(sim);
   if (!key || !value) return fail(ABL_ERR_ARG, "null argument");
@@ -970,11 +975,11 @@ extern "C" int abl_hip_set_config(abl_sim *sim, const char *key, const char *val
     else return fail(ABL_ERR_ARG, "hip.grid must be delta or full");
   } else if (k == "hip.rebuild") {
     if (v == "fused") {
-      // a fresh barrier state (an abandoned launch leaves its error flag set)
+      // fresh queues (an abandoned launch leaves its error flag set)
       for (AgentStore &s : sim->types) {
         if (s.nl_gate) {
           HIP_TRY(hipStreamSynchronize(sim->stream));
-          HIP_TRY(hipMemset(s.nl_gate + 8, 0, 8 * 4));
+          HIP_TRY(reset_queues(sim, s));
         }
       }
       sim->fused_rebuild = true;
@@ -1376,8 +1381,8 @@ static int reserve_lists(abl_sim *sim, AgentStore &s, int cap) {
   HIP_TRY(hipMalloc(&s.nl_perm, n * 4));
   HIP_TRY(hipMalloc(&s.nl_prow0, n * 16));
   if (!s.nl_gate) {
-    HIP_TRY(hipMalloc(&s.nl_gate, 16 * 4));
-    HIP_TRY(hipMemset(s.nl_gate, 0, 16 * 4));
+    HIP_TRY(hipMalloc(&s.nl_gate, kGateWords * 4));
+    HIP_TRY(hipMemsetAsync(s.nl_gate, 0, kGateWords * 4, sim->stream));
   }
   s.nl_cap = cap;
   s.nl_ncap = n;
@@ -1420,6 +1425,7 @@ static int enter_lists(abl_sim *sim, AgentStore &b, const StepDesc &st, const St
   if (rc) return rc;
   for (int attempt = 0; attempt < 2; attempt++) {
     HIP_TRY(hipMemsetAsync(b.nl_gate, 0, 4 * 4, sim->stream));
+    HIP_TRY(hipMemsetAsync(b.nl_gate + kGateQueue, 0, 2 * sizeof(RebuildQueue), sim->stream));
     NListArgs nl = list_args(sim, b, r, rl);
     StepLaunch L = Lb;
     L.nl_mode = 1;
@@ -1487,7 +1493,10 @@ static int gated_rebuild(abl_sim *sim, AgentStore &b, const StepDesc &st, const 
     d.gc = placed;
     d.id_in = b.id[b.id_cur];
     d.id_out = b.id[1 - b.id_cur];
-    d.q = reinterpret_cast<RebuildQueue *>(b.nl_gate + 8);
+    RebuildQueue *queues = reinterpret_cast<RebuildQueue *>(b.nl_gate + kGateQueue);
+    d.q = queues + (sim->timestep & 1u);
+    d.q_other = queues + (~sim->timestep & 1u);
+    d.error = b.nl_gate + kGateError;
     d.spins = sim->barrier_spins;
     d.blocks = sim->rebuild_blocks;
     d.launched = &launched;
@@ -1537,10 +1546,9 @@ static int check_rebuild(abl_sim *sim) {
   for (AgentStore &s : sim->types) {
     if (!s.nl_gate) continue;
     uint32_t err = 0;
-    HIP_TRY(hipMemcpy(&err, s.nl_gate + 8 + offsetof(RebuildQueue, error) / 4, 4,
-                      hipMemcpyDeviceToHost));
+    HIP_TRY(hipMemcpy(&err, s.nl_gate + kGateError, 4, hipMemcpyDeviceToHost));
     if (err) {
-      HIP_TRY(hipMemset(s.nl_gate + 8, 0, 8 * 4));
+      HIP_TRY(reset_queues(sim, s));
       sim->fused_rebuild = false;
       for (AgentStore &t : sim->types) {
         t.nl_ok = false;

@@ -1006,47 +1006,55 @@ template <class M>
 using policy_pos_t = typename std::conditional<policy_relative<M>::value, double, typename M::F>::type;
 
 // The gated re-sort and list build of one timestep in one launch (256
-// threads): bin, scan, place (abl_pipeline.hpp), then the copy of the new
-// cell offsets and every tile's lists, as phases of a work queue whose waits
-// end whether or not the blocks are co-resident (abl_pipeline.hpp).  Returns
-// at once when the previous step set no gate, or after a wait ran past its
-// spin limit (the host then sees q->error and rebuilds from scratch).
+// threads): bin, scan, place as phases of a work queue whose waits end whether
+// or not the blocks are co-resident (abl_pipeline.hpp), then the copy of the
+// new cell offsets and the tiles' lists, each block its share.  Returns at once
+// when the previous step set no gate, or after a wait ran past its spin limit
+// (the host then sees the error flag and rebuilds from scratch).
+//
+// Claims and releases cost more than the work: with an item per 256 agents,
+// scan tile, piece of the offsets and tile, each released by all four waves, a
+// rebuild took 1,840 us for 1,000,003 agents (the same phases as four launches
+// 125 us) and 102 us for 1,000; with one item per block and phase, released by
+// one thread, and the tiles not claimed at all it takes 310 us and 60 us.
 template <class M, int TX, int TY, int TZ, int RM>
 __global__ __launch_bounds__(256) void tiled_rebuild(typename M::Args a, NListArgs nl,
                                                       DeltaArgs d) {
   extern __shared__ __align__(16) unsigned char smem[];
+  if (blockIdx.x == 0 && threadIdx.x == 0) queue_reset(d.q_other);
   if (nl.gate[nl.parity] == 0u) return;
-  if (__hip_atomic_load(&d.q->error, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u) return;
+  if (__hip_atomic_load(d.error, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u) return;
   if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&nl.stats[2], 1u);  // rebuilds run
   __shared__ uint32_t lds[kWave + 1];
   const unsigned nt = tile_count<TX, TY, TZ, M::DIM>(a.g);
-  const uint32_t chunks = (uint32_t) (d.n + 255) / 256u;
-  const uint32_t ncopy = nl.start_dst ? (uint32_t) (nl.ncells + 1 + 255) / 256u : 0u;
-  QueuePlan plan;
-  plan.end[0] = chunks;
-  plan.end[1] = plan.end[0] + (uint32_t) d.nscan;
-  plan.end[2] = plan.end[1] + chunks;
-  plan.end[3] = plan.end[2] + ncopy + nt;
-  uint32_t longest = 0;
+  const QueuePhase agents = QueuePhase::of((uint32_t) (d.n + 255) / 256u, gridDim.x);
+  const QueuePhase scan = QueuePhase::of((uint32_t) d.nscan, gridDim.x);
+  const uint32_t end0 = agents.items, end1 = end0 + scan.items, end2 = end1 + agents.items;
+  int waited = 0;  // phases before this one are finished, as far as this block has waited
+  bool ok = true;
   for (;;) {
     const uint32_t item = queue_claim(d.q);
-    if (item >= plan.end[3]) break;
-    const int phase = plan.phase_of(item);
-    if (phase > 0 && !queue_wait(d.q, phase - 1, plan.items(phase - 1), d.spins)) break;
-    const uint32_t k = item - plan.first(phase);
-    if (phase < 3) {
-      delta_item<policy_pos_t<M>>(d, phase, k, lds);
-    } else if (k < ncopy) {
-      const int c = (int) (k * 256u + threadIdx.x);
-      if (c <= nl.ncells) nl.start_dst[c] = nl.start_src[c];
-    } else {
-      const unsigned t = k - ncopy;
-      longest = max(longest, list_build_tile<M, TX, TY, TZ, RM>(a, nl, xcd_block(t, nt), smem));
+    if (item >= end2) break;
+    const int phase = item < end0 ? 0 : item < end1 ? 1 : 2;
+    if (phase > waited) {
+      ok = queue_wait(d.q, phase - 1, phase == 1 ? agents.items : scan.items, d.spins, d.error);
+      if (!ok) break;
+      waited = phase;
     }
+    const uint32_t k = item - (phase == 0 ? 0u : phase == 1 ? end0 : end1);
+    const QueuePhase &w = phase == 1 ? scan : agents;
+    const uint32_t end = min((k + 1u) * w.per, w.units);
+    for (uint32_t u = k * w.per; u < end; u++) delta_item<policy_pos_t<M>>(d, phase, u, lds);
     queue_finish(d.q, phase);
   }
+  if (!ok || !queue_wait(d.q, 2, agents.items, d.spins, d.error)) return;
+  list_copy_starts(nl);
+  uint32_t longest = 0;
+  for (unsigned t = blockIdx.x; t < nt; t += gridDim.x) {
+    longest = max(longest, list_build_tile<M, TX, TY, TZ, RM>(a, nl, xcd_block(t, nt), smem));
+    __syncthreads();  // the next tile's tables go where this one's are read
+  }
   list_longest(nl, longest);
-  queue_exit(d.q);
 }
 
 // One timestep of the step through the lists.  An agent whose list
@@ -1288,6 +1296,8 @@ inline void launch_tiled(typename M::Args a, const GridView &g, float occupancy,
   hipLaunchKernelGGL((tiled_step<M, TX, TY, TZ, RM>), ntiles, threads, smem, stream, a);
 }
 
+constexpr unsigned kRebuildBlocks = 1024;
+
 // Launch the neighbour-list build (mode 1) or the step through the lists
 // (mode 2) for a tile shape; same tiles and LDS budget as tiled_step.
 template <class M, int TX, int TY, int TZ, int RM>
@@ -1299,14 +1309,17 @@ inline void launch_list(typename M::Args a, const GridView &g, float occupancy, 
   const int threads = block > 256 ? 256 : block;
   const unsigned ntiles = tile_count<TX, TY, TZ, M::DIM>(g);
   if (mode == 3) {
-    // as many blocks as the CUs hold at once (a multiple of the 8 XCDs); the
-    // work queue does not need them resident together, more would only
-    // find the queue empty
+    // A block per two chunks of agents and per tile, a multiple of the 8 XCDs,
+    // at most kRebuildBlocks and what the CUs hold at once (the work queue
+    // does not need them resident together, more would only wait): each block
+    // costs a claim and a release per phase.  A timestep of 1,000,003 agents
+    // that rebuilds took 457, 362, 358 and 430 us with 256, 512, 1,024 and 2,048
+    // blocks, one of 1,000 agents 84 us with 8 blocks and 110 with 2,048.
     if (!delta || delta->pos_elem != (int) sizeof(policy_pos_t<M>) || !delta->launched) return;
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return;
-    // the grid for (device, dynamic LDS) of the last launch, kept: the
-    // occupancy query costs more host time than the launch
+    // the resident blocks for (device, dynamic LDS) of the last launch, kept:
+    // the occupancy query costs more host time than the launch
     static std::atomic<uint64_t> cached{0};
     const uint64_t key = ((uint64_t) (uint32_t) dev << 40) | ((uint64_t) smem << 16);
     uint64_t got = cached.load(std::memory_order_relaxed);
@@ -1322,6 +1335,8 @@ inline void launch_list(typename M::Args a, const GridView &g, float occupancy, 
       if (grid < 8u) return;
       cached.store(key | grid, std::memory_order_relaxed);
     }
+    const unsigned chunks = (unsigned) (delta->n + 511) / 512u;
+    grid = std::min(std::min(grid, kRebuildBlocks), (std::max(chunks, ntiles) + 7u) & ~7u);
     if (delta->blocks) grid = delta->blocks;
     hipLaunchKernelGGL((tiled_rebuild<M, TX, TY, TZ, RM>), grid, 256, smem, stream, a, nl, *delta);
     *delta->launched = 1;
