@@ -1347,7 +1347,8 @@ std::string Gen::device_program() {
       << (f->near_agent ? f->near_agent->index : -1) << ", nullptr, 0.0, " << w << "u, launch_"
       << f->name << ", " << (f->uses_removal ? "true" : "false") << ", " << adds << ", "
       << (list_capable(*f) ? "true" : "false") << ", "
-      << (f->near_agent ? "radius_" + f->name : std::string("nullptr")) << "}";
+      << (f->near_agent ? "radius_" + f->name : std::string("nullptr")) << ", "
+      << (tile_capable(*f) ? "true" : "false") << "}";
   }
   o << "},\n    env,\n    nullptr,\n    nullptr,\n    nullptr,\n    false,\n    "
     << (S.simulate && S.simulate->seq_decl ? "seq_step" : "nullptr") << ",\n  };\n  return &d;\n}\n\n"

@@ -147,6 +147,9 @@ struct NListArgs {
   uint32_t *start_dst;
   int ncells;
   int gated;            // 1: build only when gate[parity] is set
+  // null, or the agents in tiles that do not fit LDS: no build at crowd_limit
+  const uint32_t *crowd;
+  uint32_t crowd_limit;
 };
 
 // Fast float reciprocal (1 ulp) for the FP32-compensated precision.

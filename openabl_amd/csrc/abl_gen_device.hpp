@@ -362,6 +362,17 @@ struct GenPolicy {
   }
 };
 
+// Count the agents of step S's tiles that do not fit LDS (tile_probe).
+template <class S>
+inline void launch_gen_probe(const StepLaunch &L) {
+  using M = GenPolicy<S>;
+  constexpr int TX = S::DIM == 3 ? 8 : 16, TY = S::DIM == 3 ? 4 : 8, TZ = S::DIM == 3 ? 4 : 1;
+  const int R = L.grid.reach;
+  if (R <= 1) launch_probe<M, TX, TY, TZ, 1>(L);
+  else if (R == 2) launch_probe<M, TX, TY, TZ, 2>(L);
+  else launch_probe<M, TX, TY, TZ, 4>(L);
+}
+
 // Launch step S on the LDS tiles of its dimension, its near loop walking
 // each agent's stencil (cell order; the grid walk's candidates in its order).
 template <class S>
@@ -371,6 +382,10 @@ inline void launch_gen_tiles(const StepLaunch &L) {
   a.rc = L.rc;
   using M = GenPolicy<S>;
   const int R = L.grid.reach;
+  if (L.nl_mode == 4) {
+    launch_gen_probe<S>(L);
+    return;
+  }
   if constexpr (S::DIM == 3) {
     if (R <= 1) launch_tiled<M, 8, 4, 4, 1>(a, L.grid, L.occupancy, L.block, L.stream, L.lds_slack);
     else if (R == 2) launch_tiled<M, 8, 4, 4, 2>(a, L.grid, L.occupancy, L.block, L.stream, L.lds_slack);
@@ -391,6 +406,10 @@ inline void launch_gen_lists(const StepLaunch &L) {
   a.rc = L.rc;
   using M = GenPolicy<S>;
   const int R = L.grid.reach;
+  if (L.nl_mode == 4) {
+    launch_gen_probe<S>(L);
+    return;
+  }
   if constexpr (S::DIM == 3) {
     if (R <= 1) launch_list<M, 8, 4, 4, 1>(a, L.grid, L.occupancy, L.block, L.stream, L.lds_slack, *L.nl, L.nl_mode, L.delta);
     else if (R == 2) launch_list<M, 8, 4, 4, 2>(a, L.grid, L.occupancy, L.block, L.stream, L.lds_slack, *L.nl, L.nl_mode, L.delta);

@@ -197,6 +197,9 @@ struct AgentStore {
   bool nl_pending = false;
   bool nl_off = false;          // lists given up for this type (rebuilt nearly every step)
   bool nl_kept = false;         // the rebuild rate was measured and the lists kept
+  // whether the agents crowd into tiles that do not fit LDS (probe_tiles),
+  // looked at once per upload, parameter or configuration change
+  bool dense = false, dense_known = false;
   uint64_t nl_t_req = 0, nl_t_prev = 0;
   uint32_t nl_c_prev = 0;
   // run-time add/remove: ids stop being 0..n-1 once agents die or are born
@@ -894,6 +897,7 @@ extern "C" int abl_hip_set_param(abl_sim *sim, const char *name, double value) {
       for (AgentStore &s : sim->types) {
         s.grid_valid = false;
         s.nl_ok = false;
+        s.dense_known = false;
       }
       return ABL_OK;
     }
@@ -927,6 +931,7 @@ extern "C" int abl_hip_set_config(abl_sim *sim, const char *key, const char *val
   for (AgentStore &s : sim->types) {
     s.nl_ok = false;
     s.grid_valid = false;
+    s.dense_known = false;
   }
   if (k == "hip.block") {
     int b = std::atoi(value);
@@ -1072,6 +1077,7 @@ extern "C" int abl_hip_upload(abl_sim *sim, int t, const void *aos, size_t count
   s.grid_valid = false;
   s.sorted = false;
   s.nl_ok = false;
+  s.dense_known = false;
   s.ids_dense = true;
   s.next_id = (int64_t) count;
   if (count == 0) return ABL_OK;
@@ -1307,6 +1313,15 @@ static int apply_births(abl_sim *sim, AgentStore &parent, AgentStore &child, int
 }
 
 // ---- neighbour lists ---------------------------------------------------------------
+
+// The gate block of an agent type.
+static int reserve_gate(abl_sim *sim, AgentStore &s) {
+  if (s.nl_gate) return ABL_OK;
+  HIP_TRY(hipMalloc(&s.nl_gate, kGateWords * 4));
+  HIP_TRY(hipMemsetAsync(s.nl_gate, 0, kGateWords * 4, sim->stream));
+  return ABL_OK;
+}
+
 // A step whose near loop runs over its own agent type, with a launcher that
 // supports them, walks per-agent neighbour lists (abl_tile.hpp) instead of
 // the stencil.  The lists are rebuilt on the device -- delta re-sort into the
@@ -1318,6 +1333,43 @@ static bool list_eligible(const abl_sim *sim, const StepDesc &st, const AgentSto
   return sim->nlist && st.nlist && st.near_agent == st.agent && sim->order == 0 && sim->tile != 0 &&
          !st.removes && !st.adds && a.n > 0 && a.pos_col >= 0 && a.n < (size_t) INT32_MAX &&
          !a.nl_off;
+}
+
+// Where a quarter of the agents or more sit in tiles whose halo does not fit
+// LDS, a few blocks that read every candidate from global memory do most of
+// the work one after another: the type then takes the launcher's kernel with
+// one thread per agent (as hip.tile=0 does), which visits the same candidates
+// in the same order.  200,003 circle3d agents in 16 Gaussian clusters: 6,900 us
+// per timestep on tiles and lists, 430 us untiled.  Counted after an upload (with
+// lists, their first build waits for the count on the device and the host's
+// wait is that build's), for populations that more than a few blocks share.
+constexpr size_t kProbeAgents = 8192;
+static uint32_t crowd_limit(const AgentStore &b) { return (uint32_t) ((b.n + 3) / 4); }
+static int launch_probe_tiles(abl_sim *sim, AgentStore &b, const StepDesc &st, const StepLaunch &Lb) {
+  NListArgs nl{};
+  nl.stats = b.nl_gate + 2;
+  StepLaunch L = Lb;
+  L.nl_mode = 4;
+  L.nl = &nl;
+  st.launch(L);
+  HIP_TRY(hipGetLastError());
+  return ABL_OK;
+}
+
+static int probe_tiles(abl_sim *sim, AgentStore &b, const StepDesc &st, const StepLaunch &L) {
+  b.dense_known = true;
+  b.dense = false;
+  if (b.n < kProbeAgents) return ABL_OK;
+  int rc = reserve_gate(sim, b);
+  if (rc) return rc;
+  HIP_TRY(hipMemsetAsync(b.nl_gate + 3, 0, 4, sim->stream));
+  rc = launch_probe_tiles(sim, b, st, L);
+  if (rc) return rc;
+  uint32_t crowd = 0;
+  HIP_TRY(hipMemcpyAsync(&crowd, b.nl_gate + 3, 4, hipMemcpyDeviceToHost, sim->stream));
+  HIP_TRY(hipStreamSynchronize(sim->stream));
+  b.dense = crowd >= crowd_limit(b);
+  return ABL_OK;
 }
 
 // With "hip.nlist" left at its default, lists are given up for an agent type
@@ -1380,10 +1432,8 @@ static int reserve_lists(abl_sim *sim, AgentStore &s, int cap) {
   HIP_TRY(hipMalloc(&s.nl_pos0, 3 * n * 8));
   HIP_TRY(hipMalloc(&s.nl_perm, n * 4));
   HIP_TRY(hipMalloc(&s.nl_prow0, n * 16));
-  if (!s.nl_gate) {
-    HIP_TRY(hipMalloc(&s.nl_gate, kGateWords * 4));
-    HIP_TRY(hipMemsetAsync(s.nl_gate, 0, kGateWords * 4, sim->stream));
-  }
+  const int rc = reserve_gate(sim, s);
+  if (rc) return rc;
   s.nl_cap = cap;
   s.nl_ncap = n;
   return ABL_OK;
@@ -1414,6 +1464,8 @@ static NListArgs list_args(const abl_sim *sim, const AgentStore &s, double r, do
 
 // Enter list mode on a fresh grid: build the lists from the current buffers,
 // grow them once if the longest list did not fit (one host wait per entry).
+// Not entered (nl_ok stays false) when the agents turn out to crowd into tiles
+// that do not fit LDS.
 static int enter_lists(abl_sim *sim, AgentStore &b, const StepDesc &st, const StepLaunch &Lb,
                        double r, double rl) {
   const double vol = b.dim == 3 ? 4.0 / 3.0 * M_PI * rl * rl * rl : M_PI * rl * rl;
@@ -1427,15 +1479,24 @@ static int enter_lists(abl_sim *sim, AgentStore &b, const StepDesc &st, const St
     HIP_TRY(hipMemsetAsync(b.nl_gate, 0, 4 * 4, sim->stream));
     HIP_TRY(hipMemsetAsync(b.nl_gate + kGateQueue, 0, 2 * sizeof(RebuildQueue), sim->stream));
     NListArgs nl = list_args(sim, b, r, rl);
+    if (!b.dense_known && b.n >= kProbeAgents && !sim->nlist_set) {
+      rc = launch_probe_tiles(sim, b, st, Lb);
+      if (rc) return rc;
+      nl.crowd = b.nl_gate + 3;
+      nl.crowd_limit = crowd_limit(b);
+    }
     StepLaunch L = Lb;
     L.nl_mode = 1;
     L.nl = &nl;
     st.launch(L);
     HIP_TRY(hipGetLastError());
-    uint32_t words[3] = {0, 0, 0};  // longest list; -; gated rebuilds run so far
+    uint32_t words[3] = {0, 0, 0};  // longest list; crowded agents; gated rebuilds run so far
     HIP_TRY(hipMemcpyAsync(words, b.nl_gate + 2, sizeof(words), hipMemcpyDeviceToHost, sim->stream));
     HIP_TRY(hipStreamSynchronize(sim->stream));
     const uint32_t longest = words[0];
+    b.dense_known = true;
+    b.dense = nl.crowd && words[1] >= nl.crowd_limit;
+    if (b.dense) return ABL_OK;
     // the rebuild rate is measured from here (list_rate)
     b.nl_c_prev = words[2];
     b.nl_t_prev = sim->timestep;
@@ -1591,7 +1652,7 @@ static int launch_step(abl_sim *sim, const StepDesc &st, uint32_t ordinal) {
     AgentStore &b = sim->types[st.near_agent];
     const double r = step_radius(sim, st);
     const double rl = r * (1.0 + sim->skin);
-    const bool want_list = list_eligible(sim, st, a);
+    bool want_list = list_eligible(sim, st, a);
     const bool gated = want_list && b.nl_ok && reach_for(b, rl) <= 4;
     if (!gated && !b.grid_valid) {
       int sp = span_open(sim, 2);
@@ -1615,6 +1676,18 @@ static int launch_step(abl_sim *sim, const StepDesc &st, uint32_t ordinal) {
     L.lds_slack = sim->lds_slack;
     L.occupancy = b.ncells ? (float) ((double) b.n / (double) b.ncells) : 0.f;
     L.rc = (float) (r / b.cell * (1.0 + 1.0 / 1048576.0));
+    // crowded tiles: one thread per agent instead (unless lists are asked for)
+    if ((st.nlist || st.tiles) && st.near_agent == st.agent && sim->order == 0 &&
+        sim->tile != 0 && !(sim->nlist_set && sim->nlist)) {
+      if (!b.dense_known && !(want_list && reach_for(b, rl) <= 4) && L.grid.reach <= 4) {
+        int rc = probe_tiles(sim, b, st, L);
+        if (rc) return rc;
+      }
+      if (b.dense_known && b.dense) {
+        want_list = false;
+        L.tile = 0;
+      }
+    }
     // lists need the list radius inside the largest tile halo (4 cells)
     if (want_list && reach_for(b, rl) <= 4) {
       L.grid.reach = reach_for(b, rl);
@@ -1626,9 +1699,14 @@ static int launch_step(abl_sim *sim, const StepDesc &st, uint32_t ordinal) {
         rc = list_rate(sim, b);
         if (rc) return rc;
       }
-      nl_step = list_args(sim, b, r, rl);
-      L.nl_mode = 2;
-      L.nl = &nl_step;
+      if (gated || b.nl_ok) {
+        nl_step = list_args(sim, b, r, rl);
+        L.nl_mode = 2;
+        L.nl = &nl_step;
+      } else if (b.dense) {
+        L.grid.reach = reach_for(b, r);
+        L.tile = 0;
+      }
     } else {
       b.nl_ok = false;
     }

@@ -91,6 +91,9 @@ struct StepDesc {
   // programs, whose constants are folded literals); when set it replaces
   // radius_scale * radius_param
   double (*radius_fn)(int precision);
+  // the launcher tiles the step (StepLaunch::nl_mode 4 probes its tiles); set
+  // for tiled steps without lists, which nlist implies it for
+  bool tiles;
 };
 
 struct ProgramDesc {
@@ -140,7 +143,8 @@ struct StepLaunch {
   float occupancy;     // near-type agents per cell (sizes the LDS tile budget)
   float lds_slack;     // LDS records per expected halo agent
   // neighbour lists: 0 = stencil walk, 1 = build the lists, 2 = step through
-  // them, 3 = gated re-sort and build in one launch (delta, abl_pipeline.hpp)
+  // them, 3 = gated re-sort and build in one launch (delta, abl_pipeline.hpp),
+  // 4 = count the agents of tiles whose halo does not fit LDS into nl->stats[1]
   int nl_mode;
   const NListArgs *nl;
   const DeltaArgs *delta;

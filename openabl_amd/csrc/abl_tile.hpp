@@ -994,6 +994,7 @@ template <class M, int TX, int TY, int TZ, int RM>
 __global__ __launch_bounds__(256) void tiled_list_build(typename M::Args a, NListArgs nl) {
   extern __shared__ __align__(16) unsigned char smem[];
   if (nl.gated && nl.gate[nl.parity] == 0u) return;
+  if (nl.crowd && *nl.crowd >= nl.crowd_limit) return;
   if (nl.gated && blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&nl.stats[2], 1u);  // rebuilds run
   list_copy_starts(nl);
   const uint32_t longest =
@@ -1285,6 +1286,37 @@ inline void tile_budget(float occupancy, int *cap, size_t *smem, float slack = 2
   *smem = head + (size_t) *cap * M::NS * sizeof(F);
 }
 
+// Adds to *agents the own agents of every tile whose halo does not fit `cap`
+// LDS records: one thread per tile, from the cell offsets alone.
+template <int DIM, int TX, int TY, int TZ, int RM>
+__global__ __launch_bounds__(256) void tile_probe(GridView g, int cap, unsigned ntiles,
+                                                  uint32_t *__restrict__ agents) {
+  using TT = TileTables<DIM, TX, TY, TZ, RM>;
+  const unsigned t = blockIdx.x * 256u + threadIdx.x;
+  if (t >= ntiles) return;
+  const typename TT::Geom G = TT::geom(g, g.reach, t);
+  uint32_t halo = 0, own = 0;
+  for (int r = 0; r < G.HN[1] * G.HN[2]; r++) {
+    halo += TT::halo_start(g, G, r, G.HN[0]) - TT::halo_start(g, G, r, 0);
+    const int y = G.H0[1] + (DIM == 3 ? r % G.HN[1] : r), z = G.H0[2] + (DIM == 3 ? r / G.HN[1] : 0);
+    if (y >= G.T0[1] && y < G.T0[1] + G.TN[1] && z >= G.T0[2] && z < G.T0[2] + G.TN[2]) {
+      const int x = G.T0[0] - G.H0[0];
+      own += TT::halo_start(g, G, r, x + G.TN[0]) - TT::halo_start(g, G, r, x);
+    }
+  }
+  if ((int) halo >= cap && own) atomicAdd(agents, own);
+}
+
+template <class M, int TX, int TY, int TZ, int RM>
+inline void launch_probe(const StepLaunch &L) {
+  int cap = 0;
+  size_t smem = 0;
+  tile_budget<M, TX, TY, TZ, RM>(L.occupancy, &cap, &smem, L.lds_slack);
+  const unsigned ntiles = tile_count<TX, TY, TZ, M::DIM>(L.grid);
+  hipLaunchKernelGGL((tile_probe<M::DIM, TX, TY, TZ, RM>), (ntiles + 255u) / 256u, 256, 0, L.stream,
+                     L.grid, cap, ntiles, L.nl->stats + 1);
+}
+
 // Launch tiled_step for a tile shape.
 template <class M, int TX, int TY, int TZ, int RM>
 inline void launch_tiled(typename M::Args a, const GridView &g, float occupancy, int block,
@@ -1353,7 +1385,11 @@ inline void launch_list(typename M::Args a, const GridView &g, float occupancy, 
 template <class M, int TX, int TY, int TZ>
 inline void launch_tiles(const StepLaunch &L, const typename M::Args &a) {
   const int R = L.grid.reach;
-  if (L.nl_mode) {
+  if (L.nl_mode == 4) {
+    if (R <= 1) launch_probe<M, TX, TY, TZ, 1>(L);
+    else if (R == 2) launch_probe<M, TX, TY, TZ, 2>(L);
+    else launch_probe<M, TX, TY, TZ, 4>(L);
+  } else if (L.nl_mode) {
     if (R <= 1) launch_list<M, TX, TY, TZ, 1>(a, L.grid, L.occupancy, L.block, L.stream, L.lds_slack, *L.nl, L.nl_mode, L.delta);
     else if (R == 2) launch_list<M, TX, TY, TZ, 2>(a, L.grid, L.occupancy, L.block, L.stream, L.lds_slack, *L.nl, L.nl_mode, L.delta);
     else launch_list<M, TX, TY, TZ, 4>(a, L.grid, L.occupancy, L.block, L.stream, L.lds_slack, *L.nl, L.nl_mode, L.delta);

@@ -233,3 +233,26 @@ def test_lists_given_up_when_rebuilt_every_step():
     c = run("circle", "f64", params, (40,), **dict(cells, **{"hip.nlist": 1}))
     assert field_bytes(c[0]) == field_bytes(run("circle", "f64", params, (40,),
                                                 **dict(cells, **{"hip.nlist": 0}))[0])
+
+
+@pytest.mark.parametrize("model,prec,params,cfg,cells", [
+    # four clusters of 5,000: nearly every agent in a tile that does not fit LDS
+    ("circle3d", "f64", circle3d_params(num_agents=20011, rho=20011 / 1e9, r=4.0, num_clusters=4,
+                                        cluster_sigma=12.0), {}, 1.05),
+    ("circle3d", "f32c", circle3d_params(num_agents=20011, rho=20011 / 1e9, r=4.0, num_clusters=4,
+                                         cluster_sigma=12.0), {"hip.cell_scale": 2}, 1.05),
+    # the 2-D tiles of a box far denser than its cells expect; without lists
+    ("boids2d", "f64", boids2d_params(num_agents=16384, agent_density=16384 / 6400.0), {"hip.nlist": 0}, 1),
+    # just below the population the tiles are counted for
+    ("circle3d", "f32", circle3d_params(num_agents=8191, rho=8191 / 1e9, r=4.0, num_clusters=1,
+                                        cluster_sigma=12.0), {}, 1.05),
+], ids=["lists-f64", "lists-f32c", "tiles-2d", "small"])
+def test_crowded_tiles_equal_untiled(model, prec, params, cfg, cells):
+    """Agents that crowd into tiles beyond LDS are stepped untiled from the
+    first timestep on: the bits of hip.tile=0 on the same cells."""
+    print(f"case nlist crowded tiles {model} {prec} {cfg}", flush=True)
+    steps = (1, 4)
+    a = run(model, prec, params, steps, **cfg)
+    b = run(model, prec, params, steps, **dict(cfg, **{"hip.tile": 0, "hip.cell_inflate": cells}))
+    for t, x, y in zip(steps, a, b):
+        assert field_bytes(x) == field_bytes(y), t
