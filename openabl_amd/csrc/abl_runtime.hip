@@ -190,11 +190,13 @@ struct AgentStore {
                                 // abandoned, from kGateQueue on: the work queues
   int nl_cap = 0;               // entries per agent
   size_t nl_ncap = 0;           // agents allocated
-  // the rebuild rate of list mode (list_rate): a pinned copy of the device's
-  // count of gated rebuilds, the event after that copy, the previous sample
+  int nl_est = 0, nl_want = 0;  // estimated entries per agent; entries asked for at the next entry
+  // list mode as the host sees it (list_watch): a pinned copy of the longest
+  // list and the count of gated rebuilds, the event after that copy, the
+  // previous sample
   uint32_t *nl_host = nullptr;
   hipEvent_t nl_ev = nullptr;
-  bool nl_pending = false;
+  bool nl_pending = false, nl_watched = false;
   bool nl_off = false;          // lists given up for this type (rebuilt nearly every step)
   bool nl_kept = false;         // the rebuild rate was measured and the lists kept
   // whether the agents crowd into tiles that do not fit LDS (probe_tiles),
@@ -1314,6 +1316,13 @@ static int apply_births(abl_sim *sim, AgentStore &parent, AgentStore &child, int
 
 // ---- neighbour lists ---------------------------------------------------------------
 
+// Capacity for lists of up to `longest` entries: a quarter more, but at most
+// four times the estimate (an agent in a dense cluster with a longer list walks
+// the stencil instead).
+static int list_room(const AgentStore &b, uint32_t longest) {
+  return (int) std::min(1.25 * (double) longest + 16.0, 4.0 * (double) b.nl_est);
+}
+
 // The gate block of an agent type.
 static int reserve_gate(abl_sim *sim, AgentStore &s) {
   if (s.nl_gate) return ABL_OK;
@@ -1372,47 +1381,63 @@ static int probe_tiles(abl_sim *sim, AgentStore &b, const StepDesc &st, const St
   return ABL_OK;
 }
 
-// With "hip.nlist" left at its default, lists are given up for an agent type
-// whose gated rebuild runs on most timesteps (its agents outrun the skin
-// every step): a re-sort and list build per timestep then costs more than
-// the stencil walk, which gives the same results.  The device counts the
-// rebuilds it runs (NListArgs::stats[2]; the list entry reads the count
-// while it waits anyway).  kListSample timesteps later the host copies the
-// count to pinned memory behind an event, and it reads the copy when it has
-// issued another kListSample timesteps (waiting for the event if need be:
-// the device still has those timesteps queued, so the wait costs it
-// nothing).  The decision is thus taken at a fixed timestep, whatever the
-// host's and the device's pace, and runs give the same bits alone, batched
-// or served.  It is taken once per type: a type that stops outrunning its
-// skin later keeps the stencil walk.
-constexpr uint64_t kListSample = 16;
-static int list_rate(abl_sim *sim, AgentStore &b) {
-  if (sim->nlist_set || b.nl_off || b.nl_kept) return ABL_OK;
+// What the host looks at while a type walks lists: the longest list built and
+// the number of rebuilds run since the lists were entered (NListArgs::stats).
+// It copies them to pinned memory behind an event, the first time kListSample
+// timesteps after entry and then every kListWatch, and reads the copy when it
+// has issued another kListSample timesteps (waiting for the event if need be:
+// the device still has those timesteps queued, so the wait costs it nothing).
+// What follows from them is thus decided at a fixed timestep, whatever the
+// host's and the device's pace, and runs give the same bits alone, batched or
+// served.
+//
+// Lists given up: with "hip.nlist" left at its default, a type whose gated
+// rebuild ran on most of the first timesteps (its agents outrun the skin every
+// step) goes back to the stencil walk, which gives the same results without a
+// list build per timestep.  Taken once per type: a type that stops outrunning
+// its skin later keeps the stencil walk.
+//
+// Lists grown: where the agents draw together, lists get longer than their
+// capacity, and an overflowed list sends its agent to the stencil and sets the
+// gate, so one such agent makes every timestep rebuild.  The type then enters
+// list mode anew, with room for the longest list (list_room's bound).  boids2d,
+// 65,536 agents at ten times the time step, 300 timesteps: 29 us per timestep,
+// 54 without growing.
+constexpr uint64_t kListSample = 8, kListWatch = 64;
+static int list_watch(abl_sim *sim, AgentStore &b) {
+  if (b.nl_off) return ABL_OK;
   if (!b.nl_host) {
-    HIP_TRY(hipHostMalloc((void **) &b.nl_host, 4, hipHostMallocDefault));
+    HIP_TRY(hipHostMalloc((void **) &b.nl_host, 3 * 4, hipHostMallocDefault));
     HIP_TRY(hipEventCreateWithFlags(&b.nl_ev, hipEventDisableTiming));
   }
   if (b.nl_pending) {
     if (sim->timestep - b.nl_t_req < kListSample) return ABL_OK;
     HIP_TRY(hipEventSynchronize(b.nl_ev));
-    const uint32_t c = *b.nl_host;
+    b.nl_pending = false;
+    const uint32_t longest = b.nl_host[0], c = b.nl_host[2];
     const uint64_t dt = b.nl_t_req - b.nl_t_prev;
-    if (dt >= kListSample && 2 * (uint64_t) (c - b.nl_c_prev) > dt) {
-      b.nl_off = true;
-      b.sorted = false;  // the stencil walk starts from a full sort
-    } else {
+    if (!sim->nlist_set && !b.nl_kept) {
+      if (2 * (uint64_t) (c - b.nl_c_prev) > dt) {
+        b.nl_off = true;
+        b.sorted = false;  // the stencil walk starts from a full sort
+        return ABL_OK;
+      }
       b.nl_kept = true;
     }
     b.nl_c_prev = c;
     b.nl_t_prev = b.nl_t_req;
-    b.nl_pending = false;
+    if (!sim->list_cap && (int64_t) longest > b.nl_cap && list_room(b, longest) > b.nl_cap) {
+      b.nl_want = list_room(b, longest);
+      b.nl_ok = false;
+      b.sorted = false;
+    }
     return ABL_OK;
   }
-  if (sim->timestep - b.nl_t_prev >= kListSample) {
-    HIP_TRY(hipMemcpyAsync(b.nl_host, b.nl_gate + 4, 4, hipMemcpyDeviceToHost, sim->stream));
+  if (sim->timestep - b.nl_t_prev >= (b.nl_watched ? kListWatch : kListSample)) {
+    HIP_TRY(hipMemcpyAsync(b.nl_host, b.nl_gate + 2, 3 * 4, hipMemcpyDeviceToHost, sim->stream));
     HIP_TRY(hipEventRecord(b.nl_ev, sim->stream));
     b.nl_t_req = sim->timestep;
-    b.nl_pending = true;
+    b.nl_pending = b.nl_watched = true;
   }
   return ABL_OK;
 }
@@ -1462,16 +1487,24 @@ static NListArgs list_args(const abl_sim *sim, const AgentStore &s, double r, do
   return nl;
 }
 
+// List entries of an agent: half again the expected population of the list
+// radius rl.
+static int list_estimate(const AgentStore &b, double rl) {
+  const double vol = b.dim == 3 ? 4.0 / 3.0 * M_PI * rl * rl * rl : M_PI * rl * rl;
+  const double env = (double) b.ncells * std::pow(b.cell, (double) b.dim);
+  const double expect = env > 0 ? vol * (double) b.n / env : 0.0;
+  return (int) (1.5 * expect) + 16;
+}
+
 // Enter list mode on a fresh grid: build the lists from the current buffers,
 // grow them once if the longest list did not fit (one host wait per entry).
 // Not entered (nl_ok stays false) when the agents turn out to crowd into tiles
 // that do not fit LDS.
 static int enter_lists(abl_sim *sim, AgentStore &b, const StepDesc &st, const StepLaunch &Lb,
                        double r, double rl) {
-  const double vol = b.dim == 3 ? 4.0 / 3.0 * M_PI * rl * rl * rl : M_PI * rl * rl;
-  const double env = (double) b.ncells * std::pow(b.cell, (double) b.dim);
-  const double expect = env > 0 ? vol * (double) b.n / env : 0.0;
-  const int want = sim->list_cap ? sim->list_cap : std::max(b.nl_cap, (int) (1.5 * expect) + 16);
+  b.nl_est = list_estimate(b, rl);
+  const int want = sim->list_cap ? sim->list_cap : std::max(std::max(b.nl_cap, b.nl_est), b.nl_want);
+  b.nl_want = 0;
   if (sim->list_cap && b.nl_cap != ((sim->list_cap + 7) & ~7)) b.nl_cap = 0;  // size requested
   int rc = reserve_lists(sim, b, want);
   if (rc) return rc;
@@ -1497,13 +1530,11 @@ static int enter_lists(abl_sim *sim, AgentStore &b, const StepDesc &st, const St
     b.dense_known = true;
     b.dense = nl.crowd && words[1] >= nl.crowd_limit;
     if (b.dense) return ABL_OK;
-    // the rebuild rate is measured from here (list_rate)
+    // watched from here on (list_watch)
     b.nl_c_prev = words[2];
     b.nl_t_prev = sim->timestep;
-    b.nl_pending = false;
-    // grow to the longest list, but to at most four times the estimate: an
-    // agent in a dense cluster with a longer list walks the stencil instead
-    const int grow = std::min((int) (1.25 * longest) + 16, 4 * want);
+    b.nl_pending = b.nl_watched = false;
+    const int grow = list_room(b, longest);
     if ((int) longest <= b.nl_cap || grow <= b.nl_cap || b.nl_cap >= 65528 || sim->list_cap) break;
     rc = reserve_lists(sim, b, grow);
     if (rc) return rc;
@@ -1696,7 +1727,7 @@ static int launch_step(abl_sim *sim, const StepDesc &st, uint32_t ordinal) {
       span_close(sim, sp);
       if (rc) return rc;
       if (gated) {
-        rc = list_rate(sim, b);
+        rc = list_watch(sim, b);
         if (rc) return rc;
       }
       if (gated || b.nl_ok) {

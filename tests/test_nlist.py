@@ -256,3 +256,19 @@ def test_crowded_tiles_equal_untiled(model, prec, params, cfg, cells):
     b = run(model, prec, params, steps, **dict(cfg, **{"hip.tile": 0, "hip.cell_inflate": cells}))
     for t, x, y in zip(steps, a, b):
         assert field_bytes(x) == field_bytes(y), t
+
+
+@pytest.mark.parametrize("prec", ["f64", "f32"])
+def test_lists_grown_while_agents_draw_together(prec):
+    """Boids pulled together until their lists outgrow the capacity they were
+    entered with: entered anew with room (at a fixed timestep), and with a
+    vanishing skin, where every timestep rebuilds, still the stencil walk's
+    bits."""
+    print(f"case nlist growing {prec}", flush=True)
+    params = dict(boids2d_params(num_agents=3001), time_scale=0.05, steer_scale=3.0)
+    steps = (60, 200)
+    a = run("boids2d", prec, params, steps,
+            **{"hip.nlist": 1, "hip.skin": 1e-9, "hip.cell_inflate": 1})
+    b = run("boids2d", prec, params, steps, **{"hip.nlist": 0})
+    for t, x, y in zip(steps, a, b):
+        assert field_bytes(x) == field_bytes(y), t
