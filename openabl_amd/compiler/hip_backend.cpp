@@ -1236,6 +1236,7 @@ std::string Gen::device_program() {
       << "  const unsigned blk = xcd_block(blockIdx.x, gridDim.x);\n"
       << "  const int i = (int) (blk * blockDim.x + threadIdx.x);\n"
       << "  if (i >= a.n) return;\n"
+      << (f->uses_removal ? "  a.dead[i] = 0;\n" : "") << (f->added_agent ? "  a.born[i] = 0;\n" : "")
       << "  Ctx<F, BY_ID> c_(a, i);\n"
       << "  const " << ag->name << "<F> in_ = load_" << ag->name << "<F>(a.in, i);\n"
       << "  " << ag->name << "<F> out_ = in_;\n"

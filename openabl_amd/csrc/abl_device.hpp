@@ -306,6 +306,72 @@ __device__ __forceinline__ void for_each_candidate_row(const GridView &g, double
   }
 }
 
+// Visit the candidates of an agent's stencil, narrowed to the cells within rc
+// cell units of (px, py, pz), in the order of for_each_candidate:
+// visit(j, q), q the candidate's position, until it returns false.
+//
+// A lane's walk is a chain of reads, each waited for before the next test, so
+// AHEAD positions of a row are read together, and the next row's cell offsets
+// while this one is visited.  For small populations, whose few waves wait on
+// each read, and near radii well below the cell size, where most of the stencil
+// is out of reach (predator_prey: 3,200 agents, near loops 6 to 26 us before, 6
+// to 22 us after; 250,000 agents, 26 to 38 us before, 15 to 31 us after); a
+// million boids with cells of the radius walk plainly 10% faster.
+template <int AHEAD, typename F, typename Visit>
+__device__ __forceinline__ void for_each_candidate_pos(const GridView &g, const F *const *p, double px,
+                                                       double py, double pz, float rc,
+                                                       Visit &&visit) {
+  const int cx = cell_coord(px, g.lo[0], g.inv_cell, g.n[0]);
+  const int cy = cell_coord(py, g.lo[1], g.inv_cell, g.n[1]);
+  const int cz = g.dim == 3 ? cell_coord(pz, g.lo[2], g.inv_cell, g.n[2]) : 0;
+  const float ux = (float) ((px - g.lo[0]) * g.inv_cell - (double) cx);
+  const float uy = (float) ((py - g.lo[1]) * g.inv_cell - (double) cy);
+  const float uz = g.dim == 3 ? (float) ((pz - g.lo[2]) * g.inv_cell - (double) cz) : 0.f;
+  const int R = g.reach;
+  const int zr = g.dim == 3 ? R : 0;
+  // the slots [a, b) of the stencil row (dy, dz), none past the last row
+  auto fetch = [&](int dy, int dz, uint32_t *a, uint32_t *b) {
+    *a = *b = 0u;
+    const int y = cy + dy, z = cz + dz;
+    int xa, xb;
+    if (dz > zr || y < 0 || y >= g.n[1] || z < 0 || (g.dim == 3 && z >= g.n[2]) ||
+        !row_interval(ux, uy, uz, dy, dz, rc, R, &xa, &xb))
+      return;
+    const int x0 = max(cx + xa, 0), x1 = min(cx + xb, g.n[0] - 1);
+    if (x0 > x1) return;
+    const uint32_t base = ((uint32_t) z * (uint32_t) g.n[1] + (uint32_t) y) * (uint32_t) g.n[0];
+    *a = g.start[base + (uint32_t) x0];
+    *b = g.start[base + (uint32_t) x1 + 1u];
+  };
+  int dy = -R, dz = -zr;
+  uint32_t a, b;
+  fetch(dy, dz, &a, &b);
+  bool go = true;
+  while (go && dz <= zr) {
+    if (++dy > R) {
+      dy = -R;
+      dz++;
+    }
+    uint32_t a1, b1;
+    fetch(dy, dz, &a1, &b1);
+    for (uint32_t j = a; go && j < b; j += AHEAD) {
+      F q[AHEAD][3];
+#pragma unroll
+      for (int u = 0; u < AHEAD; u++) {
+        const uint32_t k = j + u < b ? j + u : b - 1;
+        q[u][0] = p[0][k];
+        q[u][1] = p[1][k];
+        q[u][2] = g.dim == 3 ? p[2][k] : (F) 0;
+      }
+#pragma unroll
+      for (int u = 0; u < AHEAD; u++)
+        if (go && j + u < b) go = visit(j + u, q[u]);
+    }
+    a = a1;
+    b = b1;
+  }
+}
+
 // A column read through a buffer resource: the column's base address is
 // scalar and each lane supplies a 32-bit byte offset, so one offset serves
 // every column of a record (the record's columns are at the same offset) and

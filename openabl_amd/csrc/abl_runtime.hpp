@@ -151,8 +151,10 @@ struct StepLaunch {
   float rc;            // near radius in cell units, widened by 2^-20
   // run-time add()/removeCurrent() and random() inside steps
   const int32_t *self_id;  // ids of the stepping agents
-  uint8_t *dead;           // removeCurrent() flags, per stepping agent
-  uint8_t *born;           // add() flags, per stepping agent
+  // removeCurrent() and add() flags: a step that removes, or adds, writes 0 or 1
+  // for each of its agents
+  uint8_t *dead;
+  uint8_t *born;
   ColSet birth;            // newborn columns (the added type), per parent slot
   uint64_t seed;
   uint64_t timestep;

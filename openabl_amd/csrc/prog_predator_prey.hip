@@ -48,7 +48,7 @@ struct Args {
   uint8_t *dead;
   uint8_t *born;
   GridView g;
-  float near_t;
+  float near_t, rc;
   int n;
   uint64_t seed, t;
   uint32_t ordinal;
@@ -75,10 +75,25 @@ __device__ __forceinline__ F bound(F v, F env) {
   return v < (F) 0 ? (F) 0 : (v > env ? env : v);
 }
 
-template <bool BY_ID, typename Body>
-__device__ __forceinline__ void near_loop(const GridView &g, const int32_t *ids, int3 c, Body &&b) {
-  if (BY_ID) for_each_candidate_by_id(g, c.x, c.y, 0, g.reach, ids, b);
-  else for_each_candidate(g, c.x, c.y, 0, g.reach, b);
+// The near loop around (x, y) over the type with position columns qx, qy:
+// body(j, nx, ny, f) for each neighbour, f the float square distance.
+template <bool BY_ID, typename F, typename Body>
+__device__ __forceinline__ void near_loop(const Args<F> &a, F x, F y, const F *qx, const F *qy, Body &&b) {
+  auto visit = [&](uint32_t j, F nx, F ny) {
+    const float f = dist_sq_f32<F>(nx, ny, x, y);
+    if (!(f > a.near_t)) b(j, nx, ny, f);
+  };
+  if (BY_ID) {
+    const int3 c = cell_of<F>(a.g, x, y, (F) 0);
+    for_each_candidate_by_id(a.g, c.x, c.y, 0, a.g.reach, a.nb_id,
+                             [&](uint32_t j) { visit(j, qx[j], qy[j]); });
+  } else {
+    const F *const p[3] = {qx, qy, nullptr};
+    for_each_candidate_pos<8, F>(a.g, p, (double) x, (double) y, 0.0, a.rc, [&](uint32_t j, const F *q) {
+      visit(j, q[0], q[1]);
+      return true;
+    });
+  }
 }
 
 #define PROLOGUE                                                   \
@@ -98,13 +113,11 @@ __global__ __launch_bounds__(1024) void pred_follow_prey(Args<F> a) {
   F cx = 0, cy = 0;
   F closest = a.R_interact;
   bool can_see = false;
-  near_loop<BY_ID>(a.g, a.nb_id, cell_of<F>(a.g, x, y, (F) 0), [&](uint32_t j) {
-    const float f = dist_sq_f32<F>(qx[j], qy[j], x, y);
-    if (f > a.near_t) return;
+  near_loop<BY_ID>(a, x, y, qx, qy, [&](uint32_t, F nx, F ny, float f) {
     const F separation = dist_of<F>(f);
     if (separation < closest) {
-      cx = qx[j];
-      cy = qy[j];
+      cx = nx;
+      cy = ny;
       closest = separation;
       can_see = true;
     }
@@ -122,15 +135,13 @@ __global__ __launch_bounds__(1024) void pred_avoid(Args<F> a) {
   PROLOGUE
   const F *qx = COL(nb, C_PX, const F), *qy = COL(nb, C_PY, const F);
   F ax = 0, ay = 0;
-  near_loop<BY_ID>(a.g, a.nb_id, cell_of<F>(a.g, x, y, (F) 0), [&](uint32_t j) {
-    const float f = dist_sq_f32<F>(qx[j], qy[j], x, y);
-    if (f > a.near_t) return;
+  near_loop<BY_ID>(a, x, y, qx, qy, [&](uint32_t, F nx, F ny, float f) {
     const F separation = dist_of<F>(f);
-    if (separation < a.R_avoid && (qx[j] != x || qy[j] != y)) {
+    if (separation < a.R_avoid && (nx != x || ny != y)) {
       if ((double) separation > 0.0) {
         const F s = a.R_avoid / separation;
-        ax = ax + (x - qx[j]) * s;
-        ay = ay + (y - qy[j]) * s;
+        ax = ax + (x - nx) * s;
+        ay = ay + (y - ny) * s;
       }
     }
   });
@@ -170,12 +181,11 @@ __global__ __launch_bounds__(1024) void pred_eat_or_starve(Args<F> a) {
   PROLOGUE
   const F *qx = COL(nb, C_PX, const F), *qy = COL(nb, C_PY, const F);
   int life = COL(in, C_LIFE, const int32_t)[i];
-  near_loop<BY_ID>(a.g, a.nb_id, cell_of<F>(a.g, x, y, (F) 0), [&](uint32_t j) {
-    if (dist_sq_f32<F>(qx[j], qy[j], x, y) > a.near_t) return;
+  near_loop<BY_ID>(a, x, y, qx, qy, [&](uint32_t j, F, F, float) {
     life += a.gain_pred;
   });
   COL(out, C_LIFE, int32_t)[i] = life;
-  if (life < 1) a.dead[i] = 1;
+  a.dead[i] = life < 1;
 }
 
 // pred_reproduction / prey_reproduction: with probability p, add a copy at
@@ -187,8 +197,9 @@ __global__ __launch_bounds__(1024) void reproduction(Args<F> a) {
   const F p = PRED ? a.prob_pred : a.prob_prey;
   const uint64_t bits = counter_bits(a.seed, a.t, a.ordinal, (uint64_t) a.self_id[i], 0);
   int out_life = life;
-  if (counter_random<F>((F) 0, (F) 1.0, bits) < p) {
-    a.born[i] = 1;
+  const bool born = counter_random<F>((F) 0, (F) 1.0, bits) < p;
+  a.born[i] = born;
+  if (born) {
     COL(birth, C_PX, F)[i] = x;
     COL(birth, C_PY, F)[i] = y;
     COL(birth, C_DX, F)[i] = COL(in, C_DX, const F)[i] * (F) (-1.0);
@@ -208,15 +219,13 @@ __global__ __launch_bounds__(1024) void prey_avoid_pred(Args<F> a) {
   PROLOGUE
   const F *qx = COL(nb, C_PX, const F), *qy = COL(nb, C_PY, const F);
   F ax = 0, ay = 0;
-  near_loop<BY_ID>(a.g, a.nb_id, cell_of<F>(a.g, x, y, (F) 0), [&](uint32_t j) {
-    const float f = dist_sq_f32<F>(qx[j], qy[j], x, y);
-    if (f > a.near_t) return;
+  near_loop<BY_ID>(a, x, y, qx, qy, [&](uint32_t, F nx, F ny, float f) {
     const F separation = dist_of<F>(f);
     if (separation < a.R_interact) {
       if ((double) separation > 0.0) {
         const F s = a.R_interact / separation;
-        ax = ax + (x - qx[j]) * s;
-        ay = ay + (y - qy[j]) * s;
+        ax = ax + (x - nx) * s;
+        ay = ay + (y - ny) * s;
       }
     }
   });
@@ -230,18 +239,16 @@ __global__ __launch_bounds__(1024) void prey_flock(Args<F> a) {
   const F *qx = COL(nb, C_PX, const F), *qy = COL(nb, C_PY, const F);
   F gcx = 0, gcy = 0, gvx = 0, gvy = 0, ax = 0, ay = 0;
   int count = 0;
-  near_loop<BY_ID>(a.g, a.nb_id, cell_of<F>(a.g, x, y, (F) 0), [&](uint32_t j) {
-    const float f = dist_sq_f32<F>(qx[j], qy[j], x, y);
-    if (f > a.near_t) return;
+  near_loop<BY_ID>(a, x, y, qx, qy, [&](uint32_t, F nx, F ny, float f) {
     const F separation = dist_of<F>(f);
-    gcx = gcx + qx[j];
-    gcy = gcy + qy[j];
+    gcx = gcx + nx;
+    gcy = gcy + ny;
     count += 1;
-    if (separation < a.R_avoid && (qx[j] != x || qy[j] != y)) {
+    if (separation < a.R_avoid && (nx != x || ny != y)) {
       if ((double) separation > 0.0) {
         const F s = a.R_avoid / separation;
-        ax = ax + (x - qx[j]) * s;
-        ay = ay + (y - qy[j]) * s;
+        ax = ax + (x - nx) * s;
+        ay = ay + (y - ny) * s;
       }
     }
   });
@@ -261,12 +268,11 @@ __global__ __launch_bounds__(1024) void prey_eat_or_starve(Args<F> a) {
   const F *qx = COL(nb, G_PX, const F), *qy = COL(nb, G_PY, const F);
   const uint8_t *avail = COL(nb, G_AVAIL, const uint8_t);
   int life = COL(in, C_LIFE, const int32_t)[i];
-  near_loop<BY_ID>(a.g, a.nb_id, cell_of<F>(a.g, x, y, (F) 0), [&](uint32_t j) {
-    if (dist_sq_f32<F>(qx[j], qy[j], x, y) > a.near_t) return;
+  near_loop<BY_ID>(a, x, y, qx, qy, [&](uint32_t j, F, F, float) {
     if (avail[j]) life += a.gain_prey;
   });
   COL(out, C_LIFE, int32_t)[i] = life;
-  if (life < 1) a.dead[i] = 1;
+  a.dead[i] = life < 1;
 }
 
 template <typename F, bool BY_ID>
@@ -275,16 +281,14 @@ __global__ __launch_bounds__(1024) void prey_eaten(Args<F> a) {
   const F *qx = COL(nb, C_PX, const F), *qy = COL(nb, C_PY, const F);
   bool eaten = false;
   F closest = a.R_kill;
-  near_loop<BY_ID>(a.g, a.nb_id, cell_of<F>(a.g, x, y, (F) 0), [&](uint32_t j) {
-    const float f = dist_sq_f32<F>(qx[j], qy[j], x, y);
-    if (f > a.near_t) return;
+  near_loop<BY_ID>(a, x, y, qx, qy, [&](uint32_t, F nx, F ny, float f) {
     const F distance = dist_of<F>(f);
     if (distance < closest) {
       closest = distance;
       eaten = true;
     }
   });
-  if (eaten) a.dead[i] = 1;
+  a.dead[i] = eaten;
 }
 
 // ---- Grass steps ---------------------------------------------------------------------
@@ -300,9 +304,7 @@ __global__ __launch_bounds__(1024) void grass_eaten(Args<F> a) {
   const bool in_avail = COL(in, G_AVAIL, const uint8_t)[i] != 0;
   F closest = a.R_grass;
   bool eaten = false;
-  near_loop<BY_ID>(a.g, a.nb_id, cell_of<F>(a.g, x, y, (F) 0), [&](uint32_t j) {
-    const float f = dist_sq_f32<F>(qx[j], qy[j], x, y);
-    if (f > a.near_t) return;
+  near_loop<BY_ID>(a, x, y, qx, qy, [&](uint32_t, F nx, F ny, float f) {
     const F distance = dist_of<F>(f);
     if (distance < closest && in_avail) {
       closest = distance;
@@ -354,6 +356,7 @@ Args<F> make_args(const StepLaunch &L) {
   a.born = L.born;
   a.g = L.grid;
   a.near_t = L.near_t;
+  a.rc = L.rc;
   a.n = L.n;
   a.seed = L.seed;
   a.t = L.timestep;
