@@ -362,63 +362,50 @@ struct GenPolicy {
   }
 };
 
-// Count the agents of step S's tiles that do not fit LDS (tile_probe).
-template <class S>
-inline void launch_gen_probe(const StepLaunch &L) {
+// Launch step S on the LDS tiles of its dimension: its near loop walking each
+// agent's stencil (cell order; the grid walk's candidates in its order), or
+// what StepLaunch::nl_mode says.  LISTS: programs generated with lists.
+template <class S, bool LISTS, int TX, int TY, int TZ, int RM>
+inline void launch_gen_tile(const StepLaunch &L, const GenTileArgs &a) {
   using M = GenPolicy<S>;
-  constexpr int TX = S::DIM == 3 ? 8 : 16, TY = S::DIM == 3 ? 4 : 8, TZ = S::DIM == 3 ? 4 : 1;
-  const int R = L.grid.reach;
-  if (R <= 1) launch_probe<M, TX, TY, TZ, 1>(L);
-  else if (R == 2) launch_probe<M, TX, TY, TZ, 2>(L);
-  else launch_probe<M, TX, TY, TZ, 4>(L);
+  if (L.nl_mode == 4) {
+    launch_probe<M, TX, TY, TZ, RM>(L);
+  } else if constexpr (LISTS) {
+    if (L.nl_mode)
+      launch_list<M, TX, TY, TZ, RM>(a, L.grid, L.occupancy, L.block, L.stream, L.lds_slack, *L.nl,
+                                     L.nl_mode, L.delta);
+    else launch_tiled<M, TX, TY, TZ, RM>(a, L.grid, L.occupancy, L.block, L.stream, L.lds_slack);
+  } else {
+    launch_tiled<M, TX, TY, TZ, RM>(a, L.grid, L.occupancy, L.block, L.stream, L.lds_slack);
+  }
 }
-
-// Launch step S on the LDS tiles of its dimension, its near loop walking
-// each agent's stencil (cell order; the grid walk's candidates in its order).
-template <class S>
+template <class S, bool LISTS, int TX, int TY, int TZ>
+inline void launch_gen_reach(const StepLaunch &L, const GenTileArgs &a) {
+  if (L.grid.reach <= 1) launch_gen_tile<S, LISTS, TX, TY, TZ, 1>(L, a);
+  else if (L.grid.reach == 2) launch_gen_tile<S, LISTS, TX, TY, TZ, 2>(L, a);
+  else launch_gen_tile<S, LISTS, TX, TY, TZ, 4>(L, a);
+}
+template <class S, bool LISTS = false>
 inline void launch_gen_tiles(const StepLaunch &L) {
   GenTileArgs a{};
   static_cast<GenArgs &>(a) = make_args(L);
   a.rc = L.rc;
-  using M = GenPolicy<S>;
-  const int R = L.grid.reach;
-  if (L.nl_mode == 4) {
-    launch_gen_probe<S>(L);
-    return;
-  }
   if constexpr (S::DIM == 3) {
-    if (R <= 1) launch_tiled<M, 8, 4, 4, 1>(a, L.grid, L.occupancy, L.block, L.stream, L.lds_slack);
-    else if (R == 2) launch_tiled<M, 8, 4, 4, 2>(a, L.grid, L.occupancy, L.block, L.stream, L.lds_slack);
-    else launch_tiled<M, 8, 4, 4, 4>(a, L.grid, L.occupancy, L.block, L.stream, L.lds_slack);
+    launch_gen_reach<S, LISTS, 8, 4, 4>(L, a);
   } else {
-    if (R <= 1) launch_tiled<M, 16, 8, 1, 1>(a, L.grid, L.occupancy, L.block, L.stream, L.lds_slack);
-    else if (R == 2) launch_tiled<M, 16, 8, 1, 2>(a, L.grid, L.occupancy, L.block, L.stream, L.lds_slack);
-    else launch_tiled<M, 16, 8, 1, 4>(a, L.grid, L.occupancy, L.block, L.stream, L.lds_slack);
+    // as tile_cells, with the 8 x 8 tiles for wide reaches only
+    const int t = tile_cells(L);
+    if (t == 2 && L.grid.reach > 1) launch_gen_reach<S, LISTS, 8, 8, 1>(L, a);
+    else if (t == 2 || t == 4) launch_gen_tile<S, LISTS, 8, 4, 1, 1>(L, a);
+    else launch_gen_reach<S, LISTS, 16, 8, 1>(L, a);
   }
 }
 
-// Launch the list build (mode 1), the step through the lists (2) or the
-// one-launch gated rebuild (3) of step S on the tiles of its dimension.
+// The same for programs with lists: the list build (mode 1), the step through
+// the lists (2) or the one-launch gated rebuild (3).
 template <class S>
 inline void launch_gen_lists(const StepLaunch &L) {
-  GenTileArgs a{};
-  static_cast<GenArgs &>(a) = make_args(L);
-  a.rc = L.rc;
-  using M = GenPolicy<S>;
-  const int R = L.grid.reach;
-  if (L.nl_mode == 4) {
-    launch_gen_probe<S>(L);
-    return;
-  }
-  if constexpr (S::DIM == 3) {
-    if (R <= 1) launch_list<M, 8, 4, 4, 1>(a, L.grid, L.occupancy, L.block, L.stream, L.lds_slack, *L.nl, L.nl_mode, L.delta);
-    else if (R == 2) launch_list<M, 8, 4, 4, 2>(a, L.grid, L.occupancy, L.block, L.stream, L.lds_slack, *L.nl, L.nl_mode, L.delta);
-    else launch_list<M, 8, 4, 4, 4>(a, L.grid, L.occupancy, L.block, L.stream, L.lds_slack, *L.nl, L.nl_mode, L.delta);
-  } else {
-    if (R <= 1) launch_list<M, 16, 8, 1, 1>(a, L.grid, L.occupancy, L.block, L.stream, L.lds_slack, *L.nl, L.nl_mode, L.delta);
-    else if (R == 2) launch_list<M, 16, 8, 1, 2>(a, L.grid, L.occupancy, L.block, L.stream, L.lds_slack, *L.nl, L.nl_mode, L.delta);
-    else launch_list<M, 16, 8, 1, 4>(a, L.grid, L.occupancy, L.block, L.stream, L.lds_slack, *L.nl, L.nl_mode, L.delta);
-  }
+  launch_gen_tiles<S, true>(L);
 }
 template <typename T>
 __device__ __forceinline__ void col_put(void *const *cols, int c, int i, T v) {

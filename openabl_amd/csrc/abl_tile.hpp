@@ -1381,6 +1381,14 @@ inline void launch_list(typename M::Args a, const GridView &g, float occupancy, 
   }
 }
 
+// Dispatch on the list mode for a stencil reach of one cell.
+template <class M, int TX, int TY, int TZ>
+inline void launch_tiles_near(const StepLaunch &L, const typename M::Args &a) {
+  if (L.nl_mode == 4) launch_probe<M, TX, TY, TZ, 1>(L);
+  else if (L.nl_mode) launch_list<M, TX, TY, TZ, 1>(a, L.grid, L.occupancy, L.block, L.stream, L.lds_slack, *L.nl, L.nl_mode, L.delta);
+  else launch_tiled<M, TX, TY, TZ, 1>(a, L.grid, L.occupancy, L.block, L.stream, L.lds_slack);
+}
+
 // Dispatch on the stencil reach (RM = 1, 2 or 4 cells) and on the list mode.
 template <class M, int TX, int TY, int TZ>
 inline void launch_tiles(const StepLaunch &L, const typename M::Args &a) {
@@ -1397,6 +1405,32 @@ inline void launch_tiles(const StepLaunch &L, const typename M::Args &a) {
     if (R <= 1) launch_tiled<M, TX, TY, TZ, 1>(a, L.grid, L.occupancy, L.block, L.stream, L.lds_slack);
     else if (R == 2) launch_tiled<M, TX, TY, TZ, 2>(a, L.grid, L.occupancy, L.block, L.stream, L.lds_slack);
     else launch_tiled<M, TX, TY, TZ, 4>(a, L.grid, L.occupancy, L.block, L.stream, L.lds_slack);
+  }
+}
+
+// The cells of a 2-D tile for hip.tile=1: as many as hold about one agent per
+// lane of a block (16 x 8, 8 x 8 or 8 x 4), since a block works its own agents
+// off 256 at a time and a fuller tile waits for its second and third round while
+// CUs have no tile at all.  (Reaches beyond one cell stop at 8 x 8: the halo of a
+// smaller tile is three times its own cells.)  boids2d through the lists, cells of
+// the radius, 7.2 agents each, FP64: 1,000 agents 18.4 us per timestep on 16 x 8
+// cells, 13.4 on 8 x 8, 9.4 on 8 x 4; 65,536 agents 24.6, 18.8 and 14.6 us;
+// 1,048,576 agents 69.0, 60.1 and 56.7 us (the stencil walk 152, 124 and 107); with
+// half the cell size, 1.8 agents each, 55.6 on 16 x 8 and 59.2 on 8 x 8.
+inline int tile_cells(const StepLaunch &L) {
+  constexpr float kOwn = 240.f;
+  if (L.tile != 1 || L.occupancy * 128.f <= kOwn) return L.tile;
+  return L.occupancy * 64.f <= kOwn || L.grid.reach > 1 ? 2 : 4;
+}
+
+// Launch policy M on the 2-D tiles of hip.tile (2: 8 x 8, 3: 32 x 8 cells).
+template <class M>
+inline void launch_tiles_2d(const StepLaunch &L, const typename M::Args &a) {
+  switch (tile_cells(L)) {
+    case 2: launch_tiles<M, 8, 8, 1>(L, a); break;
+    case 3: launch_tiles<M, 32, 8, 1>(L, a); break;
+    case 4: launch_tiles_near<M, 8, 4, 1>(L, a); break;
+    default: launch_tiles<M, 16, 8, 1>(L, a);
   }
 }
 

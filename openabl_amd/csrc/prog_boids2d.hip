@@ -343,12 +343,8 @@ void launch_c(const StepLaunch &L) {
   a.max_pos = L.params[P_MAX_POS];
   if (L.order == 1) {
     hipLaunchKernelGGL((boids_step_c<true>), grid_blocks(L.n, L.block), L.block, 0, L.stream, a);
-  } else if (L.tile == 1 && L.grid.reach <= 4) {
-    launch_tiles<BoidPolicyC, 16, 8, 1>(L, a);
-  } else if (L.tile == 2 && L.grid.reach <= 4) {
-    launch_tiles<BoidPolicyC, 8, 8, 1>(L, a);
-  } else if (L.tile == 3 && L.grid.reach <= 4) {
-    launch_tiles<BoidPolicyC, 32, 8, 1>(L, a);
+  } else if (L.tile != 0 && L.grid.reach <= 4) {
+    launch_tiles_2d<BoidPolicyC>(L, a);
   } else {
     hipLaunchKernelGGL((boids_step_c<false>), grid_blocks(L.n, L.block), L.block, 0, L.stream, a);
   }
@@ -380,12 +376,8 @@ void launch_typed(const StepLaunch &L) {
   a.max_pos = (F) L.params[P_MAX_POS];
   if (L.order == 1) {
     hipLaunchKernelGGL((boids_step<F, true>), grid_blocks(L.n, L.block), L.block, 0, L.stream, a);
-  } else if (L.tile == 1 && L.grid.reach <= 4) {
-    launch_tiles<BoidPolicy<F>, 16, 8, 1>(L, a);
-  } else if (L.tile == 2 && L.grid.reach <= 4) {
-    launch_tiles<BoidPolicy<F>, 8, 8, 1>(L, a);
-  } else if (L.tile == 3 && L.grid.reach <= 4) {
-    launch_tiles<BoidPolicy<F>, 32, 8, 1>(L, a);
+  } else if (L.tile != 0 && L.grid.reach <= 4) {
+    launch_tiles_2d<BoidPolicy<F>>(L, a);
   } else {
     hipLaunchKernelGGL((boids_step<F, false>), grid_blocks(L.n, L.block), L.block, 0, L.stream, a);
   }

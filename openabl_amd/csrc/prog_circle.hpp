@@ -339,7 +339,6 @@ struct CirclePolicyC {
   }
 };
 
-
 template <int DIM>
 void launch_c(const StepLaunch &L) {
   CircleArgsC<DIM> a{};
@@ -362,10 +361,8 @@ void launch_c(const StepLaunch &L) {
   if (L.order == 1) {
     hipLaunchKernelGGL((circle_step_c<DIM, true>), nb, L.block, 0, L.stream, a);
   } else if (L.tile != 0 && L.grid.reach <= 4) {
-    if (DIM == 3) launch_tiles<M, 8, 4, 4>(L, a);
-    else if (L.tile == 2) launch_tiles<M, 8, 8, 1>(L, a);
-    else if (L.tile == 3) launch_tiles<M, 32, 8, 1>(L, a);
-    else launch_tiles<M, 16, 8, 1>(L, a);
+    if constexpr (DIM == 3) launch_tiles<M, 8, 4, 4>(L, a);
+    else launch_tiles_2d<M>(L, a);
   } else if ((size_t) L.n * 8u < ((size_t) 1 << 31)) {
     hipLaunchKernelGGL((circle_step_c<DIM, false>), nb, L.block, 0, L.stream, a);
   } else {
@@ -397,10 +394,8 @@ void launch_typed(const StepLaunch &L) {
   if (L.order == 1) {
     hipLaunchKernelGGL((circle_step<F, DIM, true>), nb, L.block, 0, L.stream, a);
   } else if (L.tile != 0 && L.grid.reach <= 4) {
-    if (DIM == 3) launch_tiles<CirclePolicy<F, DIM>, 8, 4, 4>(L, a);
-    else if (L.tile == 2) launch_tiles<CirclePolicy<F, DIM>, 8, 8, 1>(L, a);
-    else if (L.tile == 3) launch_tiles<CirclePolicy<F, DIM>, 32, 8, 1>(L, a);
-    else launch_tiles<CirclePolicy<F, DIM>, 16, 8, 1>(L, a);
+    if constexpr (DIM == 3) launch_tiles<CirclePolicy<F, DIM>, 8, 4, 4>(L, a);
+    else launch_tiles_2d<CirclePolicy<F, DIM>>(L, a);
   } else if (untiled_ok) {
     hipLaunchKernelGGL((circle_step<F, DIM, false>), nb, L.block, 0, L.stream, a);
   } else {

@@ -272,3 +272,28 @@ def test_lists_grown_while_agents_draw_together(prec):
     b = run("boids2d", prec, params, steps, **{"hip.nlist": 0})
     for t, x, y in zip(steps, a, b):
         assert field_bytes(x) == field_bytes(y), t
+
+
+@pytest.mark.parametrize("prec", ["f64", "f32"])
+@pytest.mark.parametrize("n,density,cfg", [
+    (3001, 1, {}),                      # 7.2 agents per cell: tiles of 8 x 4 cells
+    (3001, 0.4, {}),                    # 2.9: 8 x 8
+    (3001, 0.2, {}),                    # 1.4: 16 x 8
+    (3001, 4, {"hip.cell_scale": 2}),   # reach 2, 7.2: 8 x 8
+    (1, 1, {}),
+])
+def test_tile_shapes_equal(n, density, cfg, prec):
+    """hip.tile=1 takes its cells per tile from the cells' occupancy: on the
+    same cells, bits of the fixed shapes (through lists rebuilt every step) and
+    of the untiled kernel."""
+    print(f"case nlist tile shapes {n} {density} {cfg} {prec}", flush=True)
+    p = boids2d_params(num_agents=n)
+    p["agent_density"] *= density
+    steps = (1, 6)
+    same = dict(cfg, **{"hip.cell_inflate": 1})
+    runs = [run("boids2d", prec, p, steps, **dict(same, **{"hip.tile": t, **extra}))
+            for t, extra in ((1, {"hip.skin": 1e-9}), (1, {"hip.nlist": 0}),
+                             (2, {"hip.skin": 1e-9}), (3, {"hip.nlist": 0}), (0, {}))]
+    for b in runs[1:]:
+        for t, x, y in zip(steps, runs[0], b):
+            assert field_bytes(x) == field_bytes(y), t
