@@ -152,6 +152,27 @@ struct NListArgs {
   uint32_t crowd_limit;
 };
 
+// The tiles and slots of an ensemble's members in one launch (abl_ensemble.hip).
+struct EnsTiles {
+  const uint2 *tile_of;       // per tile: its member, and that member's first tile
+  const uint32_t *off;        // [members + 1] first slots
+  const uint32_t *cell_base;  // [members + 1] first cells
+  const GridView *grids;      // [members]
+  uint32_t *mgate;            // [2][members] rebuild flags by timestep parity (lists)
+  int members;
+  unsigned total;             // tiles
+};
+
+// member of slot i (binary search over the slot offsets)
+__device__ __forceinline__ int member_of(const uint32_t *off, int members, uint32_t i) {
+  int lo = 0, hi = members - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (off[mid] <= i) lo = mid; else hi = mid - 1;
+  }
+  return lo;
+}
+
 // Fast float reciprocal (1 ulp) for the FP32-compensated precision.
 __device__ __forceinline__ float rcp_f32(float x) { return __builtin_amdgcn_rcpf(x); }
 

@@ -17,10 +17,10 @@
 // and walked while no agent of the member has moved more than skin / 2 since
 // (abl_tile.hpp).  Each member has its own rebuild gate, set by its own
 // agents, so it rebuilds on exactly the timesteps a run of it alone would.
-// The sort runs when some member is due; a member that is not keeps its
-// stored cell keys, so the sort leaves its agents where they are.  The sort
-// gathers into the other buffers and the list build copies the agents of the
-// rebuilt members back, so the step always reads the current buffers.
+// Re-sort and list build are one launch that returns at once when no member is
+// due (tiled_rebuild_multi); it re-sorts the agents of the members due by the
+// delta method into the other buffers, and the list build copies them back, so
+// the step always reads the current buffers.
 //
 // With static populations every timestep issues the same kernels on the same
 // buffers (without lists the grid gather and the step each flip the columns;
@@ -31,6 +31,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -67,54 +68,28 @@ struct Member {
   float near_t = 0.f, rc = 0.f;
 };
 
-// member of slot i (binary search over the slot offsets)
-__device__ __forceinline__ int member_of(const uint32_t *off, int members, uint32_t i) {
-  int lo = 0, hi = members - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (off[mid] <= i) lo = mid; else hi = mid - 1;
-  }
-  return lo;
-}
-
-// Every slot's cell key.  With a gate: only while *gate is set, and a member
-// whose own gate (mgate[m]) is clear keeps the key of the slot's cell at the
-// last sort (skey), so the sort leaves its agents in place.
+// Every slot's cell key.
 template <typename P>
-__global__ void k_ens_bin(const P *__restrict__ px, const P *__restrict__ py,
-                          const uint32_t *__restrict__ off, const GridView *__restrict__ grids,
-                          const uint32_t *__restrict__ cell_base, int members,
-                          uint32_t *__restrict__ key, uint32_t *__restrict__ count, int n,
-                          const uint32_t *__restrict__ gate = nullptr,
-                          const uint32_t *__restrict__ mgate = nullptr,
-                          const uint32_t *__restrict__ skey = nullptr) {
-  if (gate && *gate == 0u) return;
+__global__ void k_ens_bin(const P *__restrict__ px, const P *__restrict__ py, EnsTiles e,
+                          uint32_t *__restrict__ key, uint32_t *__restrict__ count, int n) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  const int m = member_of(off, members, (uint32_t) i);
-  uint32_t k;
-  if (mgate && mgate[m] == 0u) {
-    k = skey[i];
-  } else {
-    const GridView &g = grids[m];
-    const int3 c = cell_of<P>(g, px[i], py[i], (P) 0);
-    k = cell_base[m] + (uint32_t) c.y * (uint32_t) g.n[0] + (uint32_t) c.x;
-  }
+  const int m = member_of(e.off, e.members, (uint32_t) i);
+  const uint32_t k = e.cell_base[m] + cell_key<P>(e.grids[m], px, py, (const P *) nullptr, i);
   key[i] = k;
   atomicAdd(&count[k], 1u);
 }
 
 // slot s of member m back to record id within that member's output block
-__global__ void k_ens_unpermute(char *__restrict__ aos, const void *const *__restrict__ cols,
-                                int elem, int ncols, const int32_t *__restrict__ id, uint32_t begin,
-                                int n) {
+__global__ void k_ens_unpermute(char *__restrict__ aos, ColSet cols, int elem, int ncols,
+                                const int32_t *__restrict__ id, uint32_t begin, int n) {
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= n) return;
   const uint32_t s = begin + (uint32_t) k;
   char *rec = aos + (size_t) id[s] * (size_t) (elem * ncols);
   for (int c = 0; c < ncols; c++) {
-    if (elem == 8) ((double *) rec)[c] = ((const double *) cols[c])[s];
-    else ((float *) rec)[c] = ((const float *) cols[c])[s];
+    if (elem == 8) ((double *) rec)[c] = ((const double *) cols.c[c])[s];
+    else ((float *) rec)[c] = ((const float *) cols.c[c])[s];
   }
 }
 
@@ -131,9 +106,11 @@ struct abl_ensemble {
   int cur = 0;
   int32_t *id[2] = {nullptr, nullptr};
   int id_cur = 0;
-  uint32_t *d_off = nullptr, *d_cell_base = nullptr, *d_tile_base = nullptr;
+  uint32_t *d_off = nullptr, *d_cell_base = nullptr;
+  uint2 *d_tile_of = nullptr;
   GridView *d_grids = nullptr;
   void *d_args[2] = {nullptr, nullptr};  // member arguments for cur = 0 / cur = 1
+  void *d_build[2] = {nullptr, nullptr};  // lists: the same on the rebuild's cell offsets
   uint32_t *key = nullptr, *count = nullptr, *start = nullptr, *bsum = nullptr, *tmp_idx = nullptr;
   int32_t *tmp_id = nullptr;
   size_t ncells = 0;
@@ -155,9 +132,18 @@ struct abl_ensemble {
   uint32_t *nl_perm = nullptr;
   uint4 *nl_prow0 = nullptr;
   double *nl_pos0 = nullptr;
-  uint32_t *nl_gate = nullptr;   // [0..1] some member due, by parity; [2] longest list
+  uint32_t *nl_gate = nullptr;   // [0..1] some member due, by parity; [2] longest list;
+                                 // error flag, generation and queues (abl_pipeline.hpp)
   uint32_t *nl_mgate = nullptr;  // [2][members] member due, by parity
-  uint32_t *skey = nullptr;      // each slot's cell key at the last sort
+  uint32_t *skey[2] = {nullptr, nullptr};  // each slot's cell key at the last sort; the rebuild's
+  uint32_t *start_new = nullptr;           // the rebuild's cell offsets
+  uint32_t *dirty = nullptr;               // MoverLists
+  unsigned long long *mhead = nullptr, *mnext = nullptr;
+  uint32_t *h_error = nullptr;   // pinned copy of the error flag, as of the last simulate()
+  // download workspace: one member's records, grown to the largest asked for
+  std::mutex dl_lock;
+  void *dl = nullptr;
+  size_t dl_bytes = 0;
   hipStream_t stream = nullptr;
   hipGraphExec_t exec = nullptr;
   hipGraph_t graph = nullptr;
@@ -263,23 +249,41 @@ static void free_all(abl_ensemble *e) {
     }
     if (e->id[b]) (void) hipFree(e->id[b]);
     if (e->d_args[b]) (void) hipFree(e->d_args[b]);
+    if (e->d_build[b]) (void) hipFree(e->d_build[b]);
     e->id[b] = nullptr;
-    e->d_args[b] = nullptr;
+    e->d_args[b] = e->d_build[b] = nullptr;
   }
-  void *p[] = {e->d_off, e->d_cell_base, e->d_tile_base, e->d_grids, e->key, e->count,
-               e->start, e->bsum, e->tmp_idx, e->tmp_id, e->nl_idx, e->nl_len, e->nl_perm,
-               e->nl_prow0, e->nl_pos0, e->nl_gate, e->nl_mgate, e->skey};
-  for (void *q : p) {
+  auto drop = [](auto &q) {
     if (q) (void) hipFree(q);
-  }
-  e->nl_idx = e->nl_len = nullptr;
-  e->nl_perm = e->nl_gate = e->nl_mgate = e->skey = nullptr;
-  e->nl_prow0 = nullptr;
-  e->nl_pos0 = nullptr;
-  e->d_off = e->d_cell_base = e->d_tile_base = e->key = e->count = e->start = e->bsum = nullptr;
-  e->tmp_idx = nullptr;
-  e->tmp_id = nullptr;
-  e->d_grids = nullptr;
+    q = nullptr;
+  };
+  drop(e->d_off);
+  drop(e->d_cell_base);
+  drop(e->d_tile_of);
+  drop(e->d_grids);
+  drop(e->key);
+  drop(e->count);
+  drop(e->start);
+  drop(e->bsum);
+  drop(e->tmp_idx);
+  drop(e->tmp_id);
+  drop(e->nl_idx);
+  drop(e->nl_len);
+  drop(e->nl_perm);
+  drop(e->nl_prow0);
+  drop(e->nl_pos0);
+  drop(e->nl_gate);
+  drop(e->nl_mgate);
+  drop(e->skey[0]);
+  drop(e->skey[1]);
+  drop(e->start_new);
+  drop(e->dirty);
+  drop(e->mhead);
+  drop(e->mnext);
+  drop(e->dl);
+  e->dl_bytes = 0;
+  if (e->h_error) (void) hipHostFree(e->h_error);
+  e->h_error = nullptr;
   if (e->exec) (void) hipGraphExecDestroy(e->exec);
   if (e->graph) (void) hipGraphDestroy(e->graph);
   e->exec = nullptr;
@@ -309,69 +313,104 @@ static NListArgs ens_list_args(const abl_ensemble *e) {
   return nl;
 }
 
-// The gated rebuild of the current timestep: the sort of every slot into the
-// other buffers (members not due keep their places), then the lists of the
-// members due, which copy their agents back to the current buffers.
-static void issue_rebuild(abl_ensemble *e) {
-  const int n = (int) e->n;
-  const int M = (int) e->mem.size();
-  hipStream_t st = e->stream;
-  const int b = e->cur;
-  const uint32_t par = (uint32_t) (e->timestep & 1u);
-  const uint32_t *gate = e->nl_gate + par;
-  const uint32_t *mg = e->nl_mgate + (size_t) par * (size_t) M;
-  if (e->elem == 8) {
-    hipLaunchKernelGGL(k_ens_bin<double>, grid_blocks(n, 256), 256, 0, st,
-                       (const double *) e->col[b][0], (const double *) e->col[b][1], e->d_off,
-                       e->d_grids, e->d_cell_base, M, e->key, e->count, n, gate, mg, e->skey);
-  } else {
-    hipLaunchKernelGGL(k_ens_bin<float>, grid_blocks(n, 256), 256, 0, st,
-                       (const float *) e->col[b][0], (const float *) e->col[b][1], e->d_off,
-                       e->d_grids, e->d_cell_base, M, e->key, e->count, n, gate, mg, e->skey);
-  }
-  const int nc = (int) e->ncells;
-  const int ntiles = (nc + kScanTile - 1) / kScanTile;
-  hipLaunchKernelGGL((k_scan_tiles<uint32_t, false>), ntiles, kScanBlock, 0, st, e->count, e->start,
-                     e->bsum, nc, gate);
-  hipLaunchKernelGGL(k_scan_totals, 1, 1024, 0, st, e->bsum, ntiles, e->start, nc, gate);
-  hipLaunchKernelGGL(k_scan_add, grid_blocks(nc, 256), 256, 0, st, e->start, e->bsum, nc, gate);
-  hipLaunchKernelGGL(k_scatter, grid_blocks(n, 256), 256, 0, st, e->key, e->count, e->start,
-                     e->id[e->id_cur], e->tmp_idx, e->tmp_id, n, gate);
+static EnsTiles ens_tiles(const abl_ensemble *e) {
+  EnsTiles t{};
+  t.tile_of = e->d_tile_of;
+  t.off = e->d_off;
+  t.cell_base = e->d_cell_base;
+  t.grids = e->d_grids;
+  t.mgate = e->nl_mgate;
+  t.members = (int) e->mem.size();
+  t.total = e->total_tiles;
+  return t;
+}
+
+static GatherCols ens_gather(const abl_ensemble *e, int from) {
   GatherCols gc{};
   gc.ncols = e->ncols;
   for (int c = 0; c < e->ncols; c++) {
-    gc.src[c] = e->col[b][c];
-    gc.dst[c] = e->col[1 - b][c];
+    gc.src[c] = e->col[from][c];
+    gc.dst[c] = e->col[1 - from][c];
     gc.elem[c] = e->elem;
   }
-  hipLaunchKernelGGL(k_rank_gather, grid_blocks(n, 256), 256, 0, st, e->tmp_idx, e->tmp_id,
-                     e->key, e->start, gc, e->id[1 - e->id_cur], n, e->skey, nullptr, gate);
-  NListArgs nl = ens_list_args(e);
-  nl.gated = 1;
-  nl.copy.ncols = e->ncols;
-  for (int c = 0; c < e->ncols; c++) {
-    nl.copy.src[c] = e->col[1 - b][c];
-    nl.copy.dst[c] = e->col[b][c];
-    nl.copy.elem[c] = e->elem;
-  }
-  nl.id_src = e->id[1 - e->id_cur];
-  nl.id_dst = e->id[e->id_cur];
-  nl.skey_src = e->skey;
-  nl.skey_dst = e->skey;
-  // the build reads the sorted buffers: the arguments whose input is 1 - b
-  e->hooks->launch_multi_list(e->precision, e->d_args[b], e->d_tile_base, M, e->total_tiles,
-                              e->reach, e->occupancy, e->tile, e->block, st, nl, e->nl_mgate, 1);
+  return gc;
 }
 
-// Every member due a rebuild at this parity (p) and none at the other.
-static int set_gates(abl_ensemble *e, uint32_t p) {
-  const size_t M = e->mem.size();
-  std::vector<uint32_t> g(16, 0u), mg(2 * M, 0u);
-  g[p] = 1u;
-  for (size_t m = 0; m < M; m++) mg[p * M + m] = 1u;
-  ENS_TRY(hipMemcpy(e->nl_gate, g.data(), 16 * 4, hipMemcpyHostToDevice));
-  ENS_TRY(hipMemcpy(e->nl_mgate, mg.data(), 2 * M * 4, hipMemcpyHostToDevice));
-  return ABL_OK;
+// The full sort of every slot into the other buffers: cell offsets to `start`;
+// keys and restored counts where asked for.
+static void issue_sort(abl_ensemble *e, uint32_t *start, uint32_t *skey_out, uint32_t *count_out) {
+  const int n = (int) e->n;
+  const int nc = (int) e->ncells;
+  hipStream_t st = e->stream;
+  const int b = e->cur;
+  const EnsTiles t = ens_tiles(e);
+  if (n > 0) {
+    if (e->elem == 8)
+      hipLaunchKernelGGL(k_ens_bin<double>, grid_blocks(n, 256), 256, 0, st,
+                         (const double *) e->col[b][0], (const double *) e->col[b][1], t, e->key,
+                         e->count, n);
+    else
+      hipLaunchKernelGGL(k_ens_bin<float>, grid_blocks(n, 256), 256, 0, st,
+                         (const float *) e->col[b][0], (const float *) e->col[b][1], t, e->key,
+                         e->count, n);
+  }
+  const int ntiles = (nc + kScanTile - 1) / kScanTile;
+  hipLaunchKernelGGL(k_scan_tiles, ntiles, kScanBlock, 0, st, e->count, start, e->bsum, nc);
+  hipLaunchKernelGGL(k_scan_totals, 1, 1024, 0, st, e->bsum, ntiles, start, nc);
+  hipLaunchKernelGGL(k_scan_add, grid_blocks(nc, 256), 256, 0, st, start, e->bsum, nc);
+  if (n > 0) {
+    hipLaunchKernelGGL(k_scatter, grid_blocks(n, 256), 256, 0, st, e->key, e->count, start,
+                       e->id[e->id_cur], e->tmp_idx, e->tmp_id, n);
+    hipLaunchKernelGGL(k_rank_gather, grid_blocks(n, 256), 256, 0, st, e->tmp_idx, e->tmp_id,
+                       e->key, start, ens_gather(e, b), e->id[1 - e->id_cur], n, skey_out,
+                       count_out);
+  }
+}
+
+// The list build's arguments: from the rebuild's buffers, its agents copied back
+// to the current ones.
+static NListArgs ens_build_args(const abl_ensemble *e) {
+  NListArgs nl = ens_list_args(e);
+  nl.copy = ens_gather(e, 1 - e->cur);
+  nl.id_src = e->id[1 - e->id_cur];
+  nl.id_dst = e->id[e->id_cur];
+  nl.skey_src = e->skey[1];
+  nl.skey_dst = e->skey[0];
+  nl.start_src = e->start_new;
+  nl.start_dst = e->start;
+  return nl;
+}
+
+// The gated rebuild of the current timestep (tiled_rebuild_multi).
+static int issue_rebuild(abl_ensemble *e) {
+  DeltaArgs d{};
+  const int b = e->cur;
+  d.px = e->col[b][0];
+  d.py = e->col[b][1];
+  d.pos_elem = e->elem;
+  d.skey = e->skey[0];
+  d.key = e->key;
+  d.count = e->count;
+  d.bsum = e->bsum;
+  d.ml = MoverLists{e->dirty, e->mhead, e->mnext};
+  d.n = (int) e->n;
+  d.start_old = e->start;
+  d.start_new = e->start_new;
+  d.ncells = (int) e->ncells;
+  d.nscan = ((int) e->ncells + kScanTile - 1) / kScanTile;
+  d.skey_out = e->skey[1];
+  d.gc = ens_gather(e, b);
+  d.id_in = e->id[e->id_cur];
+  d.id_out = e->id[1 - e->id_cur];
+  RebuildQueue *queues = reinterpret_cast<RebuildQueue *>(e->nl_gate + kGateQueue);
+  d.q = queues + (e->timestep & 1u);
+  d.q_other = queues + (~e->timestep & 1u);
+  d.error = e->nl_gate + kGateError;
+  d.spins = kPhaseSpins;
+  const int rc = e->hooks->launch_multi_list(e->precision, e->d_build[b], ens_tiles(e), e->reach,
+                                             e->occupancy, e->tile, e->block, e->stream,
+                                             ens_build_args(e), &d, 3);
+  return rc ? ens_fail(rc, "list rebuild: no launch size") : ABL_OK;
 }
 
 // List buffers, and every member's first sort and lists (as a run alone
@@ -393,17 +432,35 @@ static int init_lists(abl_ensemble *e) {
   ENS_TRY(hipMalloc(&e->nl_perm, N * 4));
   ENS_TRY(hipMalloc(&e->nl_prow0, N * 16));
   ENS_TRY(hipMalloc(&e->nl_pos0, 2 * N * 8));
-  ENS_TRY(hipMalloc(&e->nl_gate, 16 * 4));
+  ENS_TRY(hipMalloc(&e->nl_gate, kGateWords * 4));
   ENS_TRY(hipMalloc(&e->nl_mgate, 2 * M * 4));
-  ENS_TRY(hipMalloc(&e->skey, N * 4));
+  for (uint32_t *&k : e->skey) ENS_TRY(hipMalloc(&k, N * 4));
+  ENS_TRY(hipMalloc(&e->dirty, e->ncells * 4));
+  ENS_TRY(hipMalloc(&e->mhead, e->ncells * 8));
+  ENS_TRY(hipMalloc(&e->mnext, N * 8));
+  ENS_TRY(hipMemsetAsync(e->dirty, 0, e->ncells * 4, e->stream));
+  ENS_TRY(hipMemsetAsync(e->mhead, 0, e->ncells * 8, e->stream));
+  ENS_TRY(hipHostMalloc((void **) &e->h_error, 4, hipHostMallocDefault));
+  *e->h_error = 0u;
+  // The lists below are those of the initial state: no member is due at the
+  // first timestep (an overflowed list sets its member's gate at that step).
+  std::vector<uint32_t> words(kGateWords, 0u), none(2 * M, 0u);
+  words[kGateGen] = 1u;
+  ENS_TRY(hipMemcpy(e->nl_mgate, none.data(), 2 * M * 4, hipMemcpyHostToDevice));
+  const int ntiles = ((int) e->ncells + kScanTile - 1) / kScanTile;
   for (int attempt = 0;; attempt++) {
     if (e->nl_idx) ENS_TRY(hipFree(e->nl_idx));
     e->nl_idx = nullptr;
     ENS_TRY(hipMalloc(&e->nl_idx, (size_t) cap * N * 2));
     e->nl_cap = cap;
-    int rc = set_gates(e, 0u);
-    if (rc) return rc;
-    issue_rebuild(e);
+    ENS_TRY(hipMemcpy(e->nl_gate, words.data(), kGateWords * 4, hipMemcpyHostToDevice));
+    ENS_TRY(hipMemsetAsync(e->count, 0, (e->ncells + 1) * 4, e->stream));
+    issue_sort(e, e->start_new, e->skey[1], e->count);
+    hipLaunchKernelGGL(k_tile_totals, ntiles, kScanBlock, 0, e->stream, e->count, e->bsum,
+                       (int) e->ncells);
+    e->hooks->launch_multi_list(e->precision, e->d_build[e->cur], ens_tiles(e), e->reach,
+                                e->occupancy, e->tile, e->block, e->stream, ens_build_args(e),
+                                nullptr, 1);
     ENS_TRY(hipGetLastError());
     ENS_TRY(hipStreamSynchronize(e->stream));
     uint32_t longest = 0;
@@ -412,11 +469,6 @@ static int init_lists(abl_ensemble *e) {
     if (attempt > 0 || (int) longest <= cap || grow <= cap || cap >= 65528 || e->list_cap) break;
     cap = std::min((grow + 7) & ~7, 65528);
   }
-  // the lists are those of the initial state: no member is due at the first
-  // timestep (an overflowed list sets its member's gate at that step)
-  std::vector<uint32_t> zero(std::max<size_t>(16, 2 * M), 0u);
-  ENS_TRY(hipMemcpy(e->nl_gate, zero.data(), 16 * 4, hipMemcpyHostToDevice));
-  ENS_TRY(hipMemcpy(e->nl_mgate, zero.data(), 2 * M * 4, hipMemcpyHostToDevice));
   return ABL_OK;
 }
 
@@ -543,43 +595,51 @@ extern "C" int abl_ens_init(abl_ensemble *e, uint64_t s0, uint64_t s1) {
   e->cur = 0;
   e->id_cur = 0;
   // device tables
-  std::vector<uint32_t> off(M + 1), cb(M + 1), tb(M + 1);
+  std::vector<uint32_t> off(M + 1), cb(M + 1);
+  std::vector<uint2> tile_of;
   std::vector<GridView> grids(M);
   for (int m = 0; m < M; m++) {
     off[m] = e->mem[m].off;
     cb[m] = e->mem[m].cell_base;
-    tb[m] = e->mem[m].tile_base;
+    tile_of.insert(tile_of.end(), e->mem[m].ntiles, make_uint2((uint32_t) m, e->mem[m].tile_base));
     grids[m] = e->mem[m].g;
   }
   off[M] = (uint32_t) total;
   cb[M] = (uint32_t) cells;
-  tb[M] = tiles;
   ENS_TRY(hipMalloc(&e->d_off, (M + 1) * 4));
   ENS_TRY(hipMalloc(&e->d_cell_base, (M + 1) * 4));
-  ENS_TRY(hipMalloc(&e->d_tile_base, (M + 1) * 4));
+  ENS_TRY(hipMalloc(&e->d_tile_of, tile_of.size() * sizeof(uint2)));
   ENS_TRY(hipMalloc(&e->d_grids, M * sizeof(GridView)));
   ENS_TRY(hipMemcpy(e->d_off, off.data(), (M + 1) * 4, hipMemcpyHostToDevice));
   ENS_TRY(hipMemcpy(e->d_cell_base, cb.data(), (M + 1) * 4, hipMemcpyHostToDevice));
-  ENS_TRY(hipMemcpy(e->d_tile_base, tb.data(), (M + 1) * 4, hipMemcpyHostToDevice));
+  ENS_TRY(hipMemcpy(e->d_tile_of, tile_of.data(), tile_of.size() * sizeof(uint2),
+                    hipMemcpyHostToDevice));
   ENS_TRY(hipMemcpy(e->d_grids, grids.data(), M * sizeof(GridView), hipMemcpyHostToDevice));
   // member kernel arguments: after the grid gather the columns sit in buffer
   // 1 - cur; the step reads them and writes buffer cur
   const size_t asz = e->hooks->args_size(e->precision);
+  if (e->lists) ENS_TRY(hipMalloc(&e->start_new, (cells + 1) * 4));
   for (int b = 0; b < 2; b++) {
-    std::vector<char> args((size_t) M * asz);
-    for (int m = 0; m < M; m++) {
-      ColSet in{}, outc{};
-      for (int c = 0; c < e->ncols; c++) {
-        in.c[c] = e->col[1 - b][c];
-        outc.c[c] = e->col[b][c];
+    auto args_on = [&](const uint32_t *start, void **d_args) -> int {
+      std::vector<char> args((size_t) M * asz);
+      for (int m = 0; m < M; m++) {
+        ColSet in{}, outc{};
+        for (int c = 0; c < e->ncols; c++) {
+          in.c[c] = e->col[1 - b][c];
+          outc.c[c] = e->col[b][c];
+        }
+        GridView g = e->mem[m].g;
+        g.start = start + e->mem[m].cell_base;
+        e->hooks->fill_args(e->precision, &args[(size_t) m * asz], e->mem[m].params.data(), in, outc,
+                            g, e->mem[m].near_t, e->mem[m].rc, e->mem[m].n, e->occupancy, e->tile);
       }
-      GridView g = e->mem[m].g;
-      g.start = e->start + e->mem[m].cell_base;
-      e->hooks->fill_args(e->precision, &args[(size_t) m * asz], e->mem[m].params.data(), in, outc,
-                          g, e->mem[m].near_t, e->mem[m].rc, e->mem[m].n, e->occupancy, e->tile);
-    }
-    ENS_TRY(hipMalloc(&e->d_args[b], args.size()));
-    ENS_TRY(hipMemcpy(e->d_args[b], args.data(), args.size(), hipMemcpyHostToDevice));
+      ENS_TRY(hipMalloc(d_args, args.size()));
+      ENS_TRY(hipMemcpy(*d_args, args.data(), args.size(), hipMemcpyHostToDevice));
+      return ABL_OK;
+    };
+    int rc = args_on(e->start, &e->d_args[b]);
+    if (!rc && e->lists) rc = args_on(e->start_new, &e->d_build[b]);
+    if (rc) return rc;
   }
   e->timestep = 0;
   if (e->lists && total > 0) {
@@ -597,17 +657,15 @@ extern "C" int abl_ens_init(abl_ensemble *e, uint64_t s0, uint64_t s1) {
 // other ones.
 static int issue_step(abl_ensemble *e) {
   const int n = (int) e->n;
-  const int M = (int) e->mem.size();
-  hipStream_t st = e->stream;
   const int b = e->cur;
   if (e->lists) {
     if (n > 0) {
-      issue_rebuild(e);
-      NListArgs nl = ens_list_args(e);
+      const int rc = issue_rebuild(e);
+      if (rc) return rc;
       // the step reads buffer b: the arguments whose input is 1 - (1 - b)
-      e->hooks->launch_multi_list(e->precision, e->d_args[1 - b], e->d_tile_base, M,
-                                  e->total_tiles, e->reach, e->occupancy, e->tile, e->block, st,
-                                  nl, e->nl_mgate, 2);
+      e->hooks->launch_multi_list(e->precision, e->d_args[1 - b], ens_tiles(e), e->reach,
+                                  e->occupancy, e->tile, e->block, e->stream, ens_list_args(e),
+                                  nullptr, 2);
       e->cur ^= 1;
     }
     e->timestep += 1;
@@ -615,39 +673,12 @@ static int issue_step(abl_ensemble *e) {
     return ABL_OK;
   }
   e->timestep += 1;
+  issue_sort(e, e->start, nullptr, nullptr);
   if (n > 0) {
-    if (e->elem == 8) {
-      hipLaunchKernelGGL(k_ens_bin<double>, grid_blocks(n, 256), 256, 0, st,
-                         (const double *) e->col[b][0], (const double *) e->col[b][1], e->d_off,
-                         e->d_grids, e->d_cell_base, M, e->key, e->count, n);
-    } else {
-      hipLaunchKernelGGL(k_ens_bin<float>, grid_blocks(n, 256), 256, 0, st,
-                         (const float *) e->col[b][0], (const float *) e->col[b][1], e->d_off,
-                         e->d_grids, e->d_cell_base, M, e->key, e->count, n);
-    }
-  }
-  const int nc = (int) e->ncells;
-  const int ntiles = (nc + kScanTile - 1) / kScanTile;
-  hipLaunchKernelGGL((k_scan_tiles<uint32_t, false>), ntiles, kScanBlock, 0, st, e->count, e->start,
-                     e->bsum, nc);
-  hipLaunchKernelGGL(k_scan_totals, 1, 1024, 0, st, e->bsum, ntiles, e->start, nc);
-  hipLaunchKernelGGL(k_scan_add, grid_blocks(nc, 256), 256, 0, st, e->start, e->bsum, nc);
-  if (n > 0) {
-    hipLaunchKernelGGL(k_scatter, grid_blocks(n, 256), 256, 0, st, e->key, e->count, e->start,
-                       e->id[e->id_cur], e->tmp_idx, e->tmp_id, n);
-    GatherCols gc{};
-    gc.ncols = e->ncols;
-    for (int c = 0; c < e->ncols; c++) {
-      gc.src[c] = e->col[b][c];
-      gc.dst[c] = e->col[1 - b][c];
-      gc.elem[c] = e->elem;
-    }
-    hipLaunchKernelGGL(k_rank_gather, grid_blocks(n, 256), 256, 0, st, e->tmp_idx, e->tmp_id,
-                       e->key, e->start, gc, e->id[1 - e->id_cur], n);
     e->id_cur ^= 1;
     // the step reads buffer 1 - b and writes buffer b: columns end where they began
-    e->hooks->launch_multi(e->precision, e->d_args[b], e->d_tile_base, M, e->total_tiles,
-                           e->reach, e->occupancy, e->tile, e->block, st);
+    e->hooks->launch_multi(e->precision, e->d_args[b], ens_tiles(e), e->reach, e->occupancy, e->tile,
+                           e->block, e->stream);
   }
   ENS_TRY(hipGetLastError());
   return ABL_OK;
@@ -688,6 +719,15 @@ extern "C" int abl_ens_simulate(abl_ensemble *e, int steps) {
     if (rc) return rc;
   }
   ENS_TRY(hipEventRecord(e->ev1, e->stream));
+  if (e->h_error)
+    ENS_TRY(hipMemcpyAsync(e->h_error, e->nl_gate + kGateError, 4, hipMemcpyDeviceToHost, e->stream));
+  return ABL_OK;
+}
+
+// After a synchronisation: no rebuild of the timesteps so far gave up waiting.
+static int ens_check(const abl_ensemble *e) {
+  if (e->h_error && *(const volatile uint32_t *) e->h_error)
+    return ens_fail(ABL_ERR_DEVICE, "list rebuild: a phase did not finish");
   return ABL_OK;
 }
 
@@ -697,7 +737,7 @@ extern "C" int abl_ens_synchronize(abl_ensemble *e, double *ms) {
   float f = 0.f;
   if (hipEventElapsedTime(&f, e->ev0, e->ev1) == hipSuccess) e->last_ms = f;
   if (ms) *ms = e->last_ms;
-  return ABL_OK;
+  return ens_check(e);
 }
 
 extern "C" int abl_ens_member_count(abl_ensemble *e, int member, size_t *count) {
@@ -717,21 +757,26 @@ extern "C" int abl_ens_download(abl_ensemble *e, int member, void *aos, size_t c
   if (mb.n == 0) return ABL_OK;
   if (!aos || capacity < (size_t) mb.n) return ens_fail(ABL_ERR_ARG, "buffer too small");
   const size_t rec = (size_t) e->ncols * (size_t) e->elem;
-  void *dst = nullptr, **dcols = nullptr;
-  ENS_TRY(hipStreamSynchronize(e->stream));
-  ENS_TRY(hipMalloc(&dst, (size_t) mb.n * rec));
-  ENS_TRY(hipMalloc((void **) &dcols, kMaxCols * sizeof(void *)));
-  void *hcols[kMaxCols] = {};
-  for (int c = 0; c < e->ncols; c++) hcols[c] = e->col[e->cur][c];
-  ENS_TRY(hipMemcpy(dcols, hcols, sizeof hcols, hipMemcpyHostToDevice));
-  hipLaunchKernelGGL(k_ens_unpermute, grid_blocks(mb.n, 256), 256, 0, e->stream, (char *) dst,
-                     (const void *const *) dcols, e->elem, e->ncols, e->id[e->id_cur], mb.off, mb.n);
+  const size_t bytes = (size_t) mb.n * rec;
+  std::lock_guard<std::mutex> hold(e->dl_lock);
+  if (e->dl_bytes < bytes) {
+    ENS_TRY(hipStreamSynchronize(e->stream));
+    if (e->dl) ENS_TRY(hipFree(e->dl));
+    e->dl = nullptr;
+    e->dl_bytes = 0;
+    size_t most = 0;
+    for (const Member &k : e->mem) most = std::max(most, (size_t) k.n * rec);
+    ENS_TRY(hipMalloc(&e->dl, most));
+    e->dl_bytes = most;
+  }
+  ColSet cols{};
+  for (int c = 0; c < e->ncols; c++) cols.c[c] = e->col[e->cur][c];
+  hipLaunchKernelGGL(k_ens_unpermute, grid_blocks(mb.n, 256), 256, 0, e->stream, (char *) e->dl,
+                     cols, e->elem, e->ncols, e->id[e->id_cur], mb.off, mb.n);
   ENS_TRY(hipGetLastError());
-  ENS_TRY(hipMemcpyAsync(aos, dst, (size_t) mb.n * rec, hipMemcpyDeviceToHost, e->stream));
+  ENS_TRY(hipMemcpyAsync(aos, e->dl, bytes, hipMemcpyDeviceToHost, e->stream));
   ENS_TRY(hipStreamSynchronize(e->stream));
-  ENS_TRY(hipFree(dst));
-  ENS_TRY(hipFree(dcols));
-  return ABL_OK;
+  return ens_check(e);
 }
 
 extern "C" int abl_ens_agents(abl_ensemble *e, size_t *total) {

@@ -61,19 +61,18 @@ struct EnsembleHooks {
                     const ColSet &out, const GridView &g, float near_t, float rc, int n,
                     float occupancy, int tile);
   // one launch over every member's tiles
-  void (*launch_multi)(int precision, const void *d_args, const uint32_t *d_tile_base,
-                       int members, unsigned total_tiles, int reach, float occupancy, int tile,
-                       int block, hipStream_t stream);
+  void (*launch_multi)(int precision, const void *d_args, const EnsTiles &tiles, int reach,
+                       float occupancy, int tile, int block, hipStream_t stream);
   // main()'s agent records for these parameters (generator already seeded)
   int (*host_records)(const double *params, int precision, std::vector<char> &out,
                       size_t *count);
-  // the gated list build (mode 1) or the step through the lists (mode 2)
-  // over every member's tiles, with the members' own rebuild gates (null:
-  // the program has no list form)
-  void (*launch_multi_list)(int precision, const void *d_args, const uint32_t *d_tile_base,
-                            int members, unsigned total_tiles, int reach, float occupancy,
-                            int tile, int block, hipStream_t stream, const NListArgs &nl,
-                            uint32_t *mgate, int mode);
+  // the first list build (mode 1), the step through the lists (mode 2) or the
+  // one-launch gated rebuild (mode 3, delta) over every member's tiles, with
+  // the members' own rebuild gates (null: the program has no list form); 0, or
+  // an error
+  int (*launch_multi_list)(int precision, const void *d_args, const EnsTiles &tiles, int reach,
+                           float occupancy, int tile, int block, hipStream_t stream,
+                           const NListArgs &nl, const DeltaArgs *delta, int mode);
 };
 
 struct StepDesc {

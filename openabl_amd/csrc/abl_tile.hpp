@@ -301,21 +301,15 @@ __global__ __launch_bounds__(256) void tiled_step(typename M::Args a) {
 }
 
 // Ensemble form: the tiles of many independent members in one launch.
-// Member m owns tiles [tile_base[m], tile_base[m+1]) and has its own
-// arguments (grid, parameters); the block's member is uniform, so its
-// arguments are read through the scalar cache.
+// Each member has its own arguments (grid, parameters); the block's member is
+// uniform, so its arguments are read through the scalar cache.
 template <class M, int TX, int TY, int TZ, int RM>
 __global__ __launch_bounds__(256) void tiled_step_multi(const typename M::Args *__restrict__ args,
-                                                        const uint32_t *__restrict__ tile_base,
-                                                        int members) {
+                                                        const uint2 *__restrict__ tile_of) {
   extern __shared__ __align__(16) unsigned char smem[];
   const unsigned t = xcd_block(blockIdx.x, gridDim.x);
-  int lo = 0, hi = members - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (tile_base[mid] <= t) lo = mid; else hi = mid - 1;
-  }
-  tiled_body<M, TX, TY, TZ, RM>(args[lo], t - tile_base[lo], smem);
+  const uint2 of = tile_of[t];
+  tiled_body<M, TX, TY, TZ, RM>(args[uniform((int) of.x)], t - (unsigned) uniform((int) of.y), smem);
 }
 
 // A coordinate whose square overflows to +inf in F.
@@ -1006,6 +1000,26 @@ __global__ __launch_bounds__(256) void tiled_list_build(typename M::Args a, NLis
 template <class M>
 using policy_pos_t = typename std::conditional<policy_relative<M>::value, double, typename M::F>::type;
 
+// The re-sort's phases as items of the work queue; true when all are finished
+// and seen by this block.
+template <class Unit>
+__device__ __forceinline__ bool rebuild_phases(const DeltaArgs &d, uint32_t chunks, Unit unit) {
+  const QueuePhase agents = QueuePhase::of(chunks, gridDim.x);
+  const QueuePhase scan = QueuePhase::of((uint32_t) d.nscan, gridDim.x);
+  for (int phase = 0; phase < 3; phase++) {
+    const QueuePhase &w = phase == 1 ? scan : agents;
+    for (bool again = false;; again = true) {
+      const QueueItem it = queue_claim(d.q, phase, w, again);
+      if (it.item == ~0u) break;
+      const uint32_t end = min((it.item + 1u) * w.per, w.units);
+      for (uint32_t u = it.item * w.per; u < end; u++) unit(phase, u);
+      queue_finish(d.q, phase, it.shard);
+    }
+    if (!queue_wait(d.q, phase, w, d.spins, d.error)) return false;
+  }
+  return true;
+}
+
 // The gated re-sort and list build of one timestep in one launch (256
 // threads): bin, scan, place as phases of a work queue whose waits end whether
 // or not the blocks are co-resident (abl_pipeline.hpp), then the copy of the
@@ -1022,33 +1036,16 @@ template <class M, int TX, int TY, int TZ, int RM>
 __global__ __launch_bounds__(256) void tiled_rebuild(typename M::Args a, NListArgs nl,
                                                       DeltaArgs d) {
   extern __shared__ __align__(16) unsigned char smem[];
-  if (blockIdx.x == 0 && threadIdx.x == 0) queue_reset(d.q_other);
+  if (blockIdx.x == 0) queue_reset(d.q_other);
   if (nl.gate[nl.parity] == 0u) return;
   if (__hip_atomic_load(d.error, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u) return;
   if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&nl.stats[2], 1u);  // rebuilds run
   __shared__ uint32_t lds[kWave + 1];
   const unsigned nt = tile_count<TX, TY, TZ, M::DIM>(a.g);
-  const QueuePhase agents = QueuePhase::of((uint32_t) (d.n + 255) / 256u, gridDim.x);
-  const QueuePhase scan = QueuePhase::of((uint32_t) d.nscan, gridDim.x);
-  const uint32_t end0 = agents.items, end1 = end0 + scan.items, end2 = end1 + agents.items;
-  int waited = 0;  // phases before this one are finished, as far as this block has waited
-  bool ok = true;
-  for (;;) {
-    const uint32_t item = queue_claim(d.q);
-    if (item >= end2) break;
-    const int phase = item < end0 ? 0 : item < end1 ? 1 : 2;
-    if (phase > waited) {
-      ok = queue_wait(d.q, phase - 1, phase == 1 ? agents.items : scan.items, d.spins, d.error);
-      if (!ok) break;
-      waited = phase;
-    }
-    const uint32_t k = item - (phase == 0 ? 0u : phase == 1 ? end0 : end1);
-    const QueuePhase &w = phase == 1 ? scan : agents;
-    const uint32_t end = min((k + 1u) * w.per, w.units);
-    for (uint32_t u = k * w.per; u < end; u++) delta_item<policy_pos_t<M>>(d, phase, u, lds);
-    queue_finish(d.q, phase);
-  }
-  if (!ok || !queue_wait(d.q, 2, agents.items, d.spins, d.error)) return;
+  if (!rebuild_phases(d, (uint32_t) (d.n + 255) / 256u, [&](int phase, uint32_t u) {
+        delta_item<policy_pos_t<M>>(d, phase, u, lds);
+      }))
+    return;
   list_copy_starts(nl);
   uint32_t longest = 0;
   for (unsigned t = blockIdx.x; t < nt; t += gridDim.x) {
@@ -1220,45 +1217,75 @@ __global__ __launch_bounds__(256, policy_list_waves<M>::value) void tiled_step_l
 // members + m].  A member rebuilds exactly when a run of it alone would: when
 // one of its own agents strayed or overflowed.
 
-__device__ __forceinline__ int tile_member(const uint32_t *__restrict__ tile_base, int members,
-                                           unsigned t) {
-  int lo = 0, hi = members - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (tile_base[mid] <= t) lo = mid; else hi = mid - 1;
-  }
-  return lo;
-}
-
-// The lists of the tiles of members due a rebuild, after the gated sort
-// (records in the sorted buffers args point at; copied back as in
-// tiled_list_build).
+// Every member's first lists, after the full sort (records in the sorted buffers
+// args point at; copied back as in tiled_list_build).
 template <class M, int TX, int TY, int TZ, int RM>
 __global__ __launch_bounds__(256) void tiled_list_build_multi(const typename M::Args *__restrict__ args,
-                                                              const uint32_t *__restrict__ tile_base,
-                                                              int members, NListArgs nl,
-                                                              const uint32_t *__restrict__ mgate) {
+                                                              const uint2 *__restrict__ tile_of,
+                                                              NListArgs nl) {
   extern __shared__ __align__(16) unsigned char smem[];
-  if (nl.gate[nl.parity] == 0u) return;
+  list_copy_starts(nl);
   const unsigned t = xcd_block(blockIdx.x, gridDim.x);
-  const int m = tile_member(tile_base, members, t);
-  if (mgate[nl.parity * members + m] == 0u) return;
-  const uint32_t longest = list_build_tile<M, TX, TY, TZ, RM>(args[m], nl, t - tile_base[m], smem);
+  const uint2 of = tile_of[t];
+  const uint32_t longest = list_build_tile<M, TX, TY, TZ, RM>(
+      args[uniform((int) of.x)], nl, t - (unsigned) uniform((int) of.y), smem);
+  list_longest(nl, longest);
+}
+
+// The gated re-sort and list build of the members due, in one launch
+// (tiled_rebuild), over the chunks of those members only.  30 members of 1,000 to
+// 65,536 boids: a timestep with no member due 37 us (of it 4.6 us for this launch
+// that returns) against 48 us with seven gated launches for the full sort and the list
+// build; with one to a few members due each step 64 against 69 us, with every
+// member due 230 us against 143: a skin that small is not worth its lists.
+template <class M, int TX, int TY, int TZ, int RM>
+__global__ __launch_bounds__(256) void tiled_rebuild_multi(const typename M::Args *__restrict__ args,
+                                                            EnsTiles e, NListArgs nl, DeltaArgs d) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  if (blockIdx.x == 0) queue_reset(d.q_other);
+  if (nl.gate[nl.parity] == 0u) return;
+  if (__hip_atomic_load(d.error, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u) return;
+  __shared__ uint32_t lds[kWave + 1];
+  const uint32_t gen = nl.gate[kGateGen];
+  const uint32_t *due = e.mgate + nl.parity * e.members;
+  __shared__ uint32_t before[kScanBlock];
+  DueChunks chunks{due, before, 0u, 0u};
+  chunks.count(e, lds);
+  if (!rebuild_phases(d, chunks.total, [&](int phase, uint32_t u) {
+        ens_delta_item<policy_pos_t<M>>(d, e, chunks, gen, phase, u, lds);
+      }))
+    return;
+  list_copy_starts(nl);
+  uint32_t longest = 0;
+  for (unsigned t = blockIdx.x; t < e.total; t += gridDim.x) {
+    const unsigned tile = xcd_block(t, e.total);
+    const uint2 of = e.tile_of[tile];
+    const int m = uniform((int) of.x);
+    if (due[m] == 0u) continue;
+    longest = max(longest, list_build_tile<M, TX, TY, TZ, RM>(
+                               args[m], nl, tile - (unsigned) uniform((int) of.y), smem));
+    __syncthreads();  // the next tile's tables go where this one's are read
+  }
   list_longest(nl, longest);
 }
 
 // One timestep of every member through the lists; clears this parity's gates
-// and sets the next parity's for the members that strayed.
+// (and moves to the next generation where they were set) and sets the next
+// parity's for the members that strayed.
 template <class M, int TX, int TY, int TZ, int RM>
 __global__ __launch_bounds__(256, policy_list_waves<M>::value) void tiled_step_list_multi(
-    const typename M::Args *__restrict__ args, const uint32_t *__restrict__ tile_base,
-    int members, NListArgs nl, uint32_t *__restrict__ mgate) {
+    const typename M::Args *__restrict__ args, const uint2 *__restrict__ tile_of, int members,
+    NListArgs nl, uint32_t *__restrict__ mgate) {
   extern __shared__ __align__(16) unsigned char smem[];
   const unsigned t = xcd_block(blockIdx.x, gridDim.x);
-  const int m = tile_member(tile_base, members, t);
-  const unsigned first = tile_base[m];
+  const uint2 of = tile_of[t];
+  const int m = uniform((int) of.x);
+  const unsigned first = (unsigned) uniform((int) of.y);
   if (threadIdx.x == 0) {
-    if (blockIdx.x == 0) nl.gate[nl.parity] = 0u;
+    if (blockIdx.x == 0 && nl.gate[nl.parity] != 0u) {
+      nl.gate[nl.parity] = 0u;
+      nl.gate[kGateGen] += 1u;
+    }
     if (t == first) mgate[nl.parity * members + m] = 0u;
   }
   if (step_list_tile<M, TX, TY, TZ, RM>(args[m], nl, t - first, smem)) {
@@ -1332,6 +1359,35 @@ constexpr unsigned kRebuildBlocks = 1024;
 
 // Launch the neighbour-list build (mode 1) or the step through the lists
 // (mode 2) for a tile shape; same tiles and LDS budget as tiled_step.
+// Blocks of a one-launch rebuild, 0 if the device cannot tell: a block per two
+// chunks of agents and per tile, a multiple of the 8 XCDs, at most kRebuildBlocks
+// and what the CUs hold at once (the work queue does not need them resident
+// together, more would only wait): each block costs a claim and a release per
+// phase.  A timestep of 1,000,003 agents that rebuilds took 457, 362, 358 and 430
+// us with 256, 512, 1,024 and 2,048 blocks, one of 1,000 agents 84 us with 8 blocks
+// and 110 with 2,048.  `cached`: the kernel's resident blocks for (device, dynamic
+// LDS) of the last launch, since the occupancy query costs more host time than
+// the launch.
+inline unsigned rebuild_grid(const void *kernel, size_t smem, int n, unsigned ntiles,
+                             std::atomic<uint64_t> &cached) {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return 0;
+  const uint64_t key = ((uint64_t) (uint32_t) dev << 40) | ((uint64_t) smem << 16);
+  const uint64_t got = cached.load(std::memory_order_relaxed);
+  unsigned grid = (got & ~0xFFFFull) == key ? (unsigned) (got & 0xFFFFu) : 0u;
+  if (!grid) {
+    int per_cu = 0, cus = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, 256, smem) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+      return 0;
+    grid = std::min(((unsigned) per_cu * (unsigned) cus) & ~7u, 0xFFF8u);
+    if (grid < 8u) return 0;
+    cached.store(key | grid, std::memory_order_relaxed);
+  }
+  const unsigned chunks = (unsigned) (n + 511) / 512u;
+  return std::min(std::min(grid, kRebuildBlocks), (std::max(chunks, ntiles) + 7u) & ~7u);
+}
+
 template <class M, int TX, int TY, int TZ, int RM>
 inline void launch_list(typename M::Args a, const GridView &g, float occupancy, int block,
                         hipStream_t stream, float slack, const NListArgs &nl, int mode,
@@ -1341,34 +1397,11 @@ inline void launch_list(typename M::Args a, const GridView &g, float occupancy, 
   const int threads = block > 256 ? 256 : block;
   const unsigned ntiles = tile_count<TX, TY, TZ, M::DIM>(g);
   if (mode == 3) {
-    // A block per two chunks of agents and per tile, a multiple of the 8 XCDs,
-    // at most kRebuildBlocks and what the CUs hold at once (the work queue
-    // does not need them resident together, more would only wait): each block
-    // costs a claim and a release per phase.  A timestep of 1,000,003 agents
-    // that rebuilds took 457, 362, 358 and 430 us with 256, 512, 1,024 and 2,048
-    // blocks, one of 1,000 agents 84 us with 8 blocks and 110 with 2,048.
     if (!delta || delta->pos_elem != (int) sizeof(policy_pos_t<M>) || !delta->launched) return;
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return;
-    // the resident blocks for (device, dynamic LDS) of the last launch, kept:
-    // the occupancy query costs more host time than the launch
     static std::atomic<uint64_t> cached{0};
-    const uint64_t key = ((uint64_t) (uint32_t) dev << 40) | ((uint64_t) smem << 16);
-    uint64_t got = cached.load(std::memory_order_relaxed);
-    unsigned grid = (got & ~0xFFFFull) == key ? (unsigned) (got & 0xFFFFu) : 0u;
-    if (!grid) {
-      int per_cu = 0, cus = 0;
-      if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-              &per_cu, reinterpret_cast<const void *>(&tiled_rebuild<M, TX, TY, TZ, RM>), 256,
-              smem) != hipSuccess ||
-          hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-        return;
-      grid = std::min(((unsigned) per_cu * (unsigned) cus) & ~7u, 0xFFF8u);
-      if (grid < 8u) return;
-      cached.store(key | grid, std::memory_order_relaxed);
-    }
-    const unsigned chunks = (unsigned) (delta->n + 511) / 512u;
-    grid = std::min(std::min(grid, kRebuildBlocks), (std::max(chunks, ntiles) + 7u) & ~7u);
+    unsigned grid = rebuild_grid(reinterpret_cast<const void *>(&tiled_rebuild<M, TX, TY, TZ, RM>),
+                                 smem, delta->n, ntiles, cached);
+    if (!grid) return;
     if (delta->blocks) grid = delta->blocks;
     hipLaunchKernelGGL((tiled_rebuild<M, TX, TY, TZ, RM>), grid, 256, smem, stream, a, nl, *delta);
     *delta->launched = 1;

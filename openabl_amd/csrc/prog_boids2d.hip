@@ -494,77 +494,86 @@ void ens_fill_args(int precision, void *dst, const double *p, const ColSet &in, 
 }
 
 template <typename F, int TX, int TY, int RM>
-void ens_launch(const void *args, const uint32_t *tile_base, int members, unsigned total,
-                float occupancy, int block, hipStream_t st) {
+void ens_launch(const void *args, const EnsTiles &e, float occupancy, int block, hipStream_t st) {
   int cap = 0;
   size_t smem = 0;
   ens_cap<F, TX, TY, RM>(occupancy, &cap, &smem);
   const int threads = block > 256 ? 256 : block;
-  hipLaunchKernelGGL((tiled_step_multi<BoidPolicy<F>, TX, TY, 1, RM>), total, threads, smem, st,
-                     (const BoidArgs<F> *) args, tile_base, members);
+  hipLaunchKernelGGL((tiled_step_multi<BoidPolicy<F>, TX, TY, 1, RM>), e.total, threads, smem, st,
+                     (const BoidArgs<F> *) args, e.tile_of);
 }
 
 template <typename F, int TX, int TY>
-void ens_launch_r(const void *args, const uint32_t *tb, int m, unsigned total, int reach,
-                  float occ, int block, hipStream_t st) {
-  if (reach <= 1) ens_launch<F, TX, TY, 1>(args, tb, m, total, occ, block, st);
-  else if (reach == 2) ens_launch<F, TX, TY, 2>(args, tb, m, total, occ, block, st);
-  else ens_launch<F, TX, TY, 4>(args, tb, m, total, occ, block, st);
+void ens_launch_r(const void *args, const EnsTiles &e, int reach, float occ, int block,
+                  hipStream_t st) {
+  if (reach <= 1) ens_launch<F, TX, TY, 1>(args, e, occ, block, st);
+  else if (reach == 2) ens_launch<F, TX, TY, 2>(args, e, occ, block, st);
+  else ens_launch<F, TX, TY, 4>(args, e, occ, block, st);
 }
 
 template <typename F>
-void ens_launch_t(const void *args, const uint32_t *tb, int m, unsigned total, int reach,
-                  float occ, int tile, int block, hipStream_t st) {
-  if (tile == 2) ens_launch_r<F, 8, 8>(args, tb, m, total, reach, occ, block, st);
-  else if (tile == 3) ens_launch_r<F, 32, 8>(args, tb, m, total, reach, occ, block, st);
-  else ens_launch_r<F, 16, 8>(args, tb, m, total, reach, occ, block, st);
+void ens_launch_t(const void *args, const EnsTiles &e, int reach, float occ, int tile, int block,
+                  hipStream_t st) {
+  if (tile == 2) ens_launch_r<F, 8, 8>(args, e, reach, occ, block, st);
+  else if (tile == 3) ens_launch_r<F, 32, 8>(args, e, reach, occ, block, st);
+  else ens_launch_r<F, 16, 8>(args, e, reach, occ, block, st);
 }
 
-void ens_launch_multi(int precision, const void *args, const uint32_t *tb, int m, unsigned total,
-                      int reach, float occ, int tile, int block, hipStream_t st) {
-  if (precision == 0) ens_launch_t<double>(args, tb, m, total, reach, occ, tile, block, st);
-  else ens_launch_t<float>(args, tb, m, total, reach, occ, tile, block, st);
+void ens_launch_multi(int precision, const void *args, const EnsTiles &e, int reach, float occ,
+                      int tile, int block, hipStream_t st) {
+  if (precision == 0) ens_launch_t<double>(args, e, reach, occ, tile, block, st);
+  else ens_launch_t<float>(args, e, reach, occ, tile, block, st);
 }
 
 template <typename F, int TX, int TY, int RM>
-void ens_launch_list(const void *args, const uint32_t *tile_base, int members, unsigned total,
-                     float occupancy, int block, hipStream_t st, const NListArgs &nl,
-                     uint32_t *mgate, int mode) {
+int ens_launch_list(const void *args, const EnsTiles &e, float occupancy, int block, hipStream_t st,
+                    const NListArgs &nl, const DeltaArgs *delta, int mode) {
+  using M = BoidPolicy<F>;
   int cap = 0;
   size_t smem = 0;
   ens_cap<F, TX, TY, RM>(occupancy, &cap, &smem);
   const int threads = block > 256 ? 256 : block;
-  if (mode == 1)
-    hipLaunchKernelGGL((tiled_list_build_multi<BoidPolicy<F>, TX, TY, 1, RM>), total, threads, smem,
-                       st, (const BoidArgs<F> *) args, tile_base, members, nl, mgate);
-  else
-    hipLaunchKernelGGL((tiled_step_list_multi<BoidPolicy<F>, TX, TY, 1, RM>), total, threads, smem,
-                       st, (const BoidArgs<F> *) args, tile_base, members, nl, mgate);
+  const BoidArgs<F> *ma = (const BoidArgs<F> *) args;
+  if (mode == 1) {
+    hipLaunchKernelGGL((tiled_list_build_multi<M, TX, TY, 1, RM>), e.total, threads, smem, st, ma,
+                       e.tile_of, nl);
+  } else if (mode == 2) {
+    hipLaunchKernelGGL((tiled_step_list_multi<M, TX, TY, 1, RM>), e.total, threads, smem, st, ma,
+                       e.tile_of, e.members, nl, e.mgate);
+  } else {
+    static std::atomic<uint64_t> cached{0};
+    const unsigned grid =
+        rebuild_grid(reinterpret_cast<const void *>(&tiled_rebuild_multi<M, TX, TY, 1, RM>), smem,
+                     delta->n, e.total, cached);
+    if (!grid) return ABL_ERR_DEVICE;
+    hipLaunchKernelGGL((tiled_rebuild_multi<M, TX, TY, 1, RM>), grid, 256, smem, st, ma, e, nl,
+                       *delta);
+  }
+  return ABL_OK;
 }
 
 template <typename F, int TX, int TY>
-void ens_launch_list_r(const void *args, const uint32_t *tb, int m, unsigned total, int reach,
-                       float occ, int block, hipStream_t st, const NListArgs &nl, uint32_t *mg,
-                       int mode) {
-  if (reach <= 1) ens_launch_list<F, TX, TY, 1>(args, tb, m, total, occ, block, st, nl, mg, mode);
-  else if (reach == 2) ens_launch_list<F, TX, TY, 2>(args, tb, m, total, occ, block, st, nl, mg, mode);
-  else ens_launch_list<F, TX, TY, 4>(args, tb, m, total, occ, block, st, nl, mg, mode);
+int ens_launch_list_r(const void *args, const EnsTiles &e, int reach, float occ, int block,
+                      hipStream_t st, const NListArgs &nl, const DeltaArgs *delta, int mode) {
+  if (reach <= 1) return ens_launch_list<F, TX, TY, 1>(args, e, occ, block, st, nl, delta, mode);
+  if (reach == 2) return ens_launch_list<F, TX, TY, 2>(args, e, occ, block, st, nl, delta, mode);
+  return ens_launch_list<F, TX, TY, 4>(args, e, occ, block, st, nl, delta, mode);
 }
 
 template <typename F>
-void ens_launch_list_t(const void *args, const uint32_t *tb, int m, unsigned total, int reach,
-                       float occ, int tile, int block, hipStream_t st, const NListArgs &nl,
-                       uint32_t *mg, int mode) {
-  if (tile == 2) ens_launch_list_r<F, 8, 8>(args, tb, m, total, reach, occ, block, st, nl, mg, mode);
-  else if (tile == 3) ens_launch_list_r<F, 32, 8>(args, tb, m, total, reach, occ, block, st, nl, mg, mode);
-  else ens_launch_list_r<F, 16, 8>(args, tb, m, total, reach, occ, block, st, nl, mg, mode);
+int ens_launch_list_t(const void *args, const EnsTiles &e, int reach, float occ, int tile, int block,
+                      hipStream_t st, const NListArgs &nl, const DeltaArgs *delta, int mode) {
+  if (tile == 2) return ens_launch_list_r<F, 8, 8>(args, e, reach, occ, block, st, nl, delta, mode);
+  if (tile == 3) return ens_launch_list_r<F, 32, 8>(args, e, reach, occ, block, st, nl, delta, mode);
+  return ens_launch_list_r<F, 16, 8>(args, e, reach, occ, block, st, nl, delta, mode);
 }
 
-void ens_launch_multi_list(int precision, const void *args, const uint32_t *tb, int m,
-                           unsigned total, int reach, float occ, int tile, int block,
-                           hipStream_t st, const NListArgs &nl, uint32_t *mgate, int mode) {
-  if (precision == 0) ens_launch_list_t<double>(args, tb, m, total, reach, occ, tile, block, st, nl, mgate, mode);
-  else ens_launch_list_t<float>(args, tb, m, total, reach, occ, tile, block, st, nl, mgate, mode);
+int ens_launch_multi_list(int precision, const void *args, const EnsTiles &e, int reach, float occ,
+                          int tile, int block, hipStream_t st, const NListArgs &nl,
+                          const DeltaArgs *delta, int mode) {
+  if (precision == 0)
+    return ens_launch_list_t<double>(args, e, reach, occ, tile, block, st, nl, delta, mode);
+  return ens_launch_list_t<float>(args, e, reach, occ, tile, block, st, nl, delta, mode);
 }
 
 const EnsembleHooks ensemble_hooks = {ens_args_size, ens_tile_shape, ens_fill_args,

@@ -84,3 +84,30 @@ def test_lists_follow_each_members_own_rebuilds():
         assert field_bytes(ens.download(m)) == field_bytes(sim.download(dt)), m
         sim.close()
     ens.close()
+
+
+@pytest.mark.parametrize("graph", [0, 1])
+@pytest.mark.parametrize("count,most", [(1, 700), (255, 3), (256, 40), (300, 40), (520, 9)])
+def test_rebuild_chunks_of_many_members(count, most, graph):
+    """The one-launch rebuild numbers the chunks of the members due in groups of
+    members (one per thread of a block; from 257 members on two or more each):
+    members of no more than one chunk, of several, of a single agent."""
+    from openabl_amd import MEMBERS, Simulation, load_library, record_dtype
+    from openabl_amd.ensemble import Ensemble, member_seed
+    print(f"case ensemble rebuild chunks {count} {most} graph={graph}", flush=True)
+    rng = np.random.default_rng(count)
+    ms = [{"num_agents": int(n), "agent_density": 0.065, "max_pos": fold6(math.sqrt(n / 0.065)),
+           "time_scale": 0.01} for n in rng.integers(1, most + 1, count)]
+    cfg = {"hip.cell_scale": 2, "hip.tile": 1, "hip.nlist": 1, "hip.list_cap": 96, "hip.skin": 0.001}
+    ens = Ensemble("boids2d", "f64", ms, config=dict(cfg, **{"hip.graph": graph}))
+    ens.init(0x1234, 0x5678)
+    ens.simulate(9)
+    dt = record_dtype(MEMBERS["boids2d"], "f64")
+    for m in sorted({0, count // 2, count - 1, *rng.integers(0, count, 3).tolist()}):
+        load_library().abl_rng_seed(*member_seed(0x1234, 0x5678, m))
+        sim = Simulation("boids2d", "f64", params=ms[m], config=cfg)
+        sim.init_agents()
+        sim.simulate(9)
+        assert field_bytes(ens.download(m)) == field_bytes(sim.download(dt)), m
+        sim.close()
+    ens.close()
