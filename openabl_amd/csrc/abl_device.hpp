@@ -147,10 +147,16 @@ struct NListArgs {
   uint32_t *start_dst;
   int ncells;
   int gated;            // 1: build only when gate[parity] is set
-  // null, or the agents in tiles that do not fit LDS: no build at crowd_limit
+  // null, or the agents in tiles that do not fit LDS: no build, and no step on
+  // tiles, at crowd_limit
   const uint32_t *crowd;
   uint32_t crowd_limit;
+  // tile_probe: null, or the pinned word the count goes to
+  uint32_t *publish;
 };
+// tile_probe's words of `stats` where it publishes: the blocks' ticket and sum
+// (zero again when it is done) and the count
+constexpr int kProbeTicket = 8, kProbeSum = 9, kProbeCount = 10;
 
 // The tiles and slots of an ensemble's members in one launch (abl_ensemble.hip).
 struct EnsTiles {

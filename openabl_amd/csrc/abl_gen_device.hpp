@@ -374,9 +374,9 @@ inline void launch_gen_tile(const StepLaunch &L, const GenTileArgs &a) {
     if (L.nl_mode)
       launch_list<M, TX, TY, TZ, RM>(a, L.grid, L.occupancy, L.block, L.stream, L.lds_slack, *L.nl,
                                      L.nl_mode, L.delta);
-    else launch_tiled<M, TX, TY, TZ, RM>(a, L.grid, L.occupancy, L.block, L.stream, L.lds_slack);
+    else launch_tiled<M, TX, TY, TZ, RM>(a, L);
   } else {
-    launch_tiled<M, TX, TY, TZ, RM>(a, L.grid, L.occupancy, L.block, L.stream, L.lds_slack);
+    launch_tiled<M, TX, TY, TZ, RM>(a, L);
   }
 }
 template <class S, bool LISTS, int TX, int TY, int TZ>
@@ -393,10 +393,9 @@ inline void launch_gen_tiles(const StepLaunch &L) {
   if constexpr (S::DIM == 3) {
     launch_gen_reach<S, LISTS, 8, 4, 4>(L, a);
   } else {
-    // as tile_cells, with the 8 x 8 tiles for wide reaches only
     const int t = tile_cells(L);
-    if (t == 2 && L.grid.reach > 1) launch_gen_reach<S, LISTS, 8, 8, 1>(L, a);
-    else if (t == 2 || t == 4) launch_gen_tile<S, LISTS, 8, 4, 1, 1>(L, a);
+    if (t == 2) launch_gen_reach<S, LISTS, 8, 8, 1>(L, a);
+    else if (t == 4) launch_gen_tile<S, LISTS, 8, 4, 1, 1>(L, a);
     else launch_gen_reach<S, LISTS, 16, 8, 1>(L, a);
   }
 }

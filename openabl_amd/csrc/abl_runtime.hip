@@ -1416,10 +1416,15 @@ extern "C" int abl_hip_init_agents(abl_sim *sim) {
 
 // ---- run-time add()/removeCurrent() ------------------------------------------------
 
+static int reserve_counts(abl_sim *sim) {
+  if (!sim->hcount)
+    HIP_TRY(hipHostMalloc((void **) &sim->hcount, sim->types.size() * 8, hipHostMallocDefault));
+  return ABL_OK;
+}
+
 static int reserve_flags(abl_sim *sim, size_t n) {
-  if (!sim->hcount) {
-    HIP_TRY(hipHostMalloc((void **) &sim->hcount, sim->types.size() * 4, hipHostMallocDefault));
-  }
+  const int rc = reserve_counts(sim);
+  if (rc) return rc;
   if (n <= sim->fcap && sim->dead) return ABL_OK;
   size_t cap = std::max<size_t>(n + n / 8, 1024);
   void *ptrs[] = {sim->dead, sim->born, sim->fbsum, sim->bl_pid, sim->bl_slot};
@@ -1436,21 +1441,25 @@ static int reserve_flags(abl_sim *sim, size_t n) {
   return ABL_OK;
 }
 
-// The pinned word of agent type s, armed for a count.
+// The pinned words of agent type s: its population's count, its crowded agents.
+static uint32_t *count_word(abl_sim *sim, const AgentStore &s) {
+  return sim->hcount + (&s - sim->types.data());
+}
+static uint32_t *crowd_word(abl_sim *sim, const AgentStore &s) {
+  return count_word(sim, s) + sim->types.size();
+}
 constexpr uint32_t kNoCount = 0xFFFFFFFFu;
-static uint32_t *arm_count(abl_sim *sim, const AgentStore &s) {
-  uint32_t *w = sim->hcount + (&s - sim->types.data());
+static uint32_t *arm_word(uint32_t *w) {
   __atomic_store_n(w, kNoCount, __ATOMIC_SEQ_CST);
   return w;
 }
+static uint32_t *arm_count(abl_sim *sim, const AgentStore &s) { return arm_word(count_word(sim, s)); }
 
-// Read the count of the removal or births pending on a type.  The device writes
-// it to pinned memory, where the host looks for it (a stream wait costs the
-// host ten times as long); if it does not come within some hundred
-// microseconds the host waits for the stream.
-static int settle(abl_sim *sim, AgentStore &s) {
-  if (s.pending == AgentStore::kSettled) return ABL_OK;
-  const uint32_t *w = sim->hcount + (&s - sim->types.data());
+// Read the count an armed word is to receive.  The device writes it to pinned
+// memory, where the host looks for it (a stream wait costs the host ten times
+// as long); if it does not come within some hundred microseconds the host waits
+// for the stream.
+static int read_count(abl_sim *sim, const uint32_t *w, uint32_t *out) {
   uint32_t c = kNoCount;
   for (int k = 0; k < 20000 && (c = __atomic_load_n(w, __ATOMIC_ACQUIRE)) == kNoCount; k++)
     __builtin_ia32_pause();
@@ -1459,6 +1468,16 @@ static int settle(abl_sim *sim, AgentStore &s) {
     c = __atomic_load_n(w, __ATOMIC_ACQUIRE);
     if (c == kNoCount) return fail(ABL_ERR_DEVICE, "no count from the device");
   }
+  *out = c;
+  return ABL_OK;
+}
+
+// Take in the removal or births pending on a type.
+static int settle(abl_sim *sim, AgentStore &s) {
+  if (s.pending == AgentStore::kSettled) return ABL_OK;
+  uint32_t c = 0;
+  const int rc = read_count(sim, count_word(sim, s), &c);
+  if (rc) return rc;
   const bool removed = s.pending == AgentStore::kRemoved;
   s.pending = AgentStore::kSettled;
   if (removed ? c == s.n : c == 0) return ABL_OK;  // nothing removed, nothing born
@@ -1583,13 +1602,16 @@ static bool list_eligible(const abl_sim *sim, const StepDesc &st, const AgentSto
 // the work one after another: the type then takes the launcher's kernel with
 // one thread per agent (as hip.tile=0 does), which visits the same candidates
 // in the same order.  200,003 circle3d agents in 16 Gaussian clusters: 6,900 us
-// per timestep on tiles and lists, 430 us untiled.  Counted after an upload (with
-// lists, their first build waits for the count on the device and the host's
-// wait is that build's), for populations that more than a few blocks share.
+// per timestep on tiles and lists, 430 us untiled.  Counted after an upload, for
+// populations that more than a few blocks share.  The first build of the lists, or
+// the first step on tiles, waits for the count on the device and does nothing
+// if it says untiled; the host reads it while that build or step runs.
 constexpr size_t kProbeAgents = 8192;
 static uint32_t crowd_limit(const AgentStore &b) { return (uint32_t) ((b.n + 3) / 4); }
-static int launch_probe_tiles(abl_sim *sim, AgentStore &b, const StepDesc &st, const StepLaunch &Lb) {
+static int launch_probe_tiles(AgentStore &b, const StepDesc &st, const StepLaunch &Lb,
+                              uint32_t *publish) {
   NListArgs nl{};
+  nl.publish = publish;
   nl.stats = b.nl_gate + 2;
   StepLaunch L = Lb;
   L.nl_mode = 4;
@@ -1599,18 +1621,23 @@ static int launch_probe_tiles(abl_sim *sim, AgentStore &b, const StepDesc &st, c
   return ABL_OK;
 }
 
-static int probe_tiles(abl_sim *sim, AgentStore &b, const StepDesc &st, const StepLaunch &L) {
-  b.dense_known = true;
-  b.dense = false;
-  if (b.n < kProbeAgents) return ABL_OK;
+// The count for a first step on tiles: *nl holds back the step that L launches
+// (read_crowd).
+static int probe_tiles(abl_sim *sim, AgentStore &b, const StepDesc &st, const StepLaunch &L,
+                       NListArgs *nl) {
   int rc = reserve_gate(sim, b);
+  if (!rc) rc = reserve_counts(sim);
   if (rc) return rc;
-  HIP_TRY(hipMemsetAsync(b.nl_gate + 3, 0, 4, sim->stream));
-  rc = launch_probe_tiles(sim, b, st, L);
-  if (rc) return rc;
+  nl->crowd = b.nl_gate + 2 + kProbeCount;
+  nl->crowd_limit = crowd_limit(b);
+  return launch_probe_tiles(b, st, L, arm_word(crowd_word(sim, b)));
+}
+
+static int read_crowd(abl_sim *sim, AgentStore &b) {
   uint32_t crowd = 0;
-  HIP_TRY(hipMemcpyAsync(&crowd, b.nl_gate + 3, 4, hipMemcpyDeviceToHost, sim->stream));
-  HIP_TRY(hipStreamSynchronize(sim->stream));
+  const int rc = read_count(sim, crowd_word(sim, b), &crowd);
+  if (rc) return rc;
+  b.dense_known = true;
   b.dense = crowd >= crowd_limit(b);
   return ABL_OK;
 }
@@ -1744,10 +1771,9 @@ static int enter_lists(abl_sim *sim, AgentStore &b, const StepDesc &st, const St
   if (rc) return rc;
   for (int attempt = 0; attempt < 2; attempt++) {
     HIP_TRY(hipMemsetAsync(b.nl_gate, 0, 4 * 4, sim->stream));
-    HIP_TRY(hipMemsetAsync(b.nl_gate + kGateQueue, 0, 2 * sizeof(RebuildQueue), sim->stream));
     NListArgs nl = list_args(sim, b, r, rl);
     if (!b.dense_known && b.n >= kProbeAgents && !sim->nlist_set) {
-      rc = launch_probe_tiles(sim, b, st, Lb);
+      rc = launch_probe_tiles(b, st, Lb, nullptr);
       if (rc) return rc;
       nl.crowd = b.nl_gate + 3;
       nl.crowd_limit = crowd_limit(b);
@@ -1920,6 +1946,7 @@ static int launch_step(abl_sim *sim, const StepDesc &st, uint32_t ordinal) {
     L.out.c[c] = (st.writes >> c) & 1u ? col_other(a, (int) c) : nullptr;
   }
   NListArgs nl_step{};
+  AgentStore *probed = nullptr;  // type whose crowded tiles are counted and not yet read
   if (st.near_agent >= 0) {
     AgentStore &b = sim->types[st.near_agent];
     const double r = step_radius(sim, st);
@@ -1952,8 +1979,14 @@ static int launch_step(abl_sim *sim, const StepDesc &st, uint32_t ordinal) {
     if ((st.nlist || st.tiles) && st.near_agent == st.agent && sim->order == 0 &&
         sim->tile != 0 && !(sim->nlist_set && sim->nlist)) {
       if (!b.dense_known && !(want_list && reach_for(b, rl) <= 4) && L.grid.reach <= 4) {
-        int rc = probe_tiles(sim, b, st, L);
-        if (rc) return rc;
+        b.dense = false;
+        b.dense_known = b.n < kProbeAgents;
+        if (!b.dense_known) {
+          int rc = probe_tiles(sim, b, st, L, &nl_step);
+          if (rc) return rc;
+          L.nl = &nl_step;
+          probed = &b;
+        }
       }
       if (b.dense_known && b.dense) {
         want_list = false;
@@ -2004,6 +2037,15 @@ static int launch_step(abl_sim *sim, const StepDesc &st, uint32_t ordinal) {
   if (L.n > 0) {
     int sp = span_open(sim, 1);
     st.launch(L);
+    if (probed) {
+      int rc = read_crowd(sim, *probed);
+      if (rc) return rc;
+      if (probed->dense) {
+        L.tile = 0;
+        L.nl = nullptr;
+        st.launch(L);
+      }
+    }
     span_close(sim, sp);
     HIP_TRY(hipGetLastError());
   }

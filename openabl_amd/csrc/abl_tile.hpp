@@ -295,8 +295,10 @@ __device__ __forceinline__ void tiled_body(const typename M::Args &a, unsigned t
                                            unsigned char *smem);
 
 template <class M, int TX, int TY, int TZ, int RM>
-__global__ __launch_bounds__(256) void tiled_step(typename M::Args a) {
+__global__ __launch_bounds__(256) void tiled_step(typename M::Args a, const uint32_t *crowd,
+                                                   uint32_t crowd_limit) {
   extern __shared__ __align__(16) unsigned char smem[];
+  if (crowd && *crowd >= crowd_limit) return;
   tiled_body<M, TX, TY, TZ, RM>(a, xcd_block(blockIdx.x, gridDim.x), smem);
 }
 
@@ -990,6 +992,11 @@ __global__ __launch_bounds__(256) void tiled_list_build(typename M::Args a, NLis
   if (nl.gated && nl.gate[nl.parity] == 0u) return;
   if (nl.crowd && *nl.crowd >= nl.crowd_limit) return;
   if (nl.gated && blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&nl.stats[2], 1u);  // rebuilds run
+  if (!nl.gated && blockIdx.x == 0) {  // entering list mode: fresh queues
+    RebuildQueue *q = reinterpret_cast<RebuildQueue *>(nl.gate + kGateQueue);
+    queue_reset(q);
+    queue_reset(q + 1);
+  }
   list_copy_starts(nl);
   const uint32_t longest =
       list_build_tile<M, TX, TY, TZ, RM>(a, nl, xcd_block(blockIdx.x, gridDim.x), smem);
@@ -1313,25 +1320,46 @@ inline void tile_budget(float occupancy, int *cap, size_t *smem, float slack = 2
   *smem = head + (size_t) *cap * M::NS * sizeof(F);
 }
 
-// Adds to *agents the own agents of every tile whose halo does not fit `cap`
-// LDS records: one thread per tile, from the cell offsets alone.
+// Adds up the own agents of every tile whose halo does not fit `cap` LDS records:
+// kProbeLanes threads per tile, a halo row each, from the cell offsets alone.  The
+// last block done hands the sum to the host where it looks for it
+// (NListArgs::publish).
+constexpr unsigned kProbeLanes = 16;
 template <int DIM, int TX, int TY, int TZ, int RM>
 __global__ __launch_bounds__(256) void tile_probe(GridView g, int cap, unsigned ntiles,
-                                                  uint32_t *__restrict__ agents) {
+                                                  uint32_t *stats, uint32_t *publish) {
   using TT = TileTables<DIM, TX, TY, TZ, RM>;
-  const unsigned t = blockIdx.x * 256u + threadIdx.x;
-  if (t >= ntiles) return;
-  const typename TT::Geom G = TT::geom(g, g.reach, t);
+  const unsigned t = (blockIdx.x * 256u + threadIdx.x) / kProbeLanes;
+  const int lane = (int) (threadIdx.x % kProbeLanes);
   uint32_t halo = 0, own = 0;
-  for (int r = 0; r < G.HN[1] * G.HN[2]; r++) {
-    halo += TT::halo_start(g, G, r, G.HN[0]) - TT::halo_start(g, G, r, 0);
-    const int y = G.H0[1] + (DIM == 3 ? r % G.HN[1] : r), z = G.H0[2] + (DIM == 3 ? r / G.HN[1] : 0);
-    if (y >= G.T0[1] && y < G.T0[1] + G.TN[1] && z >= G.T0[2] && z < G.T0[2] + G.TN[2]) {
-      const int x = G.T0[0] - G.H0[0];
-      own += TT::halo_start(g, G, r, x + G.TN[0]) - TT::halo_start(g, G, r, x);
+  if (t < ntiles) {
+    const typename TT::Geom G = TT::geom(g, g.reach, t);
+    for (int r = lane; r < G.HN[1] * G.HN[2]; r += (int) kProbeLanes) {
+      halo += TT::halo_start(g, G, r, G.HN[0]) - TT::halo_start(g, G, r, 0);
+      const int y = G.H0[1] + (DIM == 3 ? r % G.HN[1] : r), z = G.H0[2] + (DIM == 3 ? r / G.HN[1] : 0);
+      if (y >= G.T0[1] && y < G.T0[1] + G.TN[1] && z >= G.T0[2] && z < G.T0[2] + G.TN[2]) {
+        const int x = G.T0[0] - G.H0[0];
+        own += TT::halo_start(g, G, r, x + G.TN[0]) - TT::halo_start(g, G, r, x);
+      }
     }
   }
-  if ((int) halo >= cap && own) atomicAdd(agents, own);
+#pragma unroll
+  for (int d = 1; d < (int) kProbeLanes; d <<= 1) {
+    halo += (uint32_t) __shfl_xor((int) halo, d, kWave);
+    own += (uint32_t) __shfl_xor((int) own, d, kWave);
+  }
+  if (lane == 0 && (int) halo >= cap && own) atomicAdd(&stats[publish ? kProbeSum : 1], own);
+  if (!publish) return;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    __threadfence();
+    if (atomicAdd(&stats[kProbeTicket], 1u) == gridDim.x - 1u) {
+      const uint32_t sum = atomicExch(&stats[kProbeSum], 0u);
+      stats[kProbeTicket] = 0u;
+      stats[kProbeCount] = sum;
+      __hip_atomic_store(publish, sum, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+  }
 }
 
 template <class M, int TX, int TY, int TZ, int RM>
@@ -1340,19 +1368,19 @@ inline void launch_probe(const StepLaunch &L) {
   size_t smem = 0;
   tile_budget<M, TX, TY, TZ, RM>(L.occupancy, &cap, &smem, L.lds_slack);
   const unsigned ntiles = tile_count<TX, TY, TZ, M::DIM>(L.grid);
-  hipLaunchKernelGGL((tile_probe<M::DIM, TX, TY, TZ, RM>), (ntiles + 255u) / 256u, 256, 0, L.stream,
-                     L.grid, cap, ntiles, L.nl->stats + 1);
+  hipLaunchKernelGGL((tile_probe<M::DIM, TX, TY, TZ, RM>), (ntiles * kProbeLanes + 255u) / 256u, 256, 0,
+                     L.stream, L.grid, cap, ntiles, L.nl->stats, L.nl->publish);
 }
 
 // Launch tiled_step for a tile shape.
 template <class M, int TX, int TY, int TZ, int RM>
-inline void launch_tiled(typename M::Args a, const GridView &g, float occupancy, int block,
-                         hipStream_t stream, float slack = 2.0f) {
+inline void launch_tiled(typename M::Args a, const StepLaunch &L) {
   size_t smem = 0;
-  tile_budget<M, TX, TY, TZ, RM>(occupancy, &a.cap, &smem, slack);
-  const int threads = block > 256 ? 256 : block;
-  const unsigned ntiles = tile_count<TX, TY, TZ, M::DIM>(g);
-  hipLaunchKernelGGL((tiled_step<M, TX, TY, TZ, RM>), ntiles, threads, smem, stream, a);
+  tile_budget<M, TX, TY, TZ, RM>(L.occupancy, &a.cap, &smem, L.lds_slack);
+  const int threads = L.block > 256 ? 256 : L.block;
+  const unsigned ntiles = tile_count<TX, TY, TZ, M::DIM>(L.grid);
+  hipLaunchKernelGGL((tiled_step<M, TX, TY, TZ, RM>), ntiles, threads, smem, L.stream, a,
+                     L.nl ? L.nl->crowd : nullptr, L.nl ? L.nl->crowd_limit : 0u);
 }
 
 constexpr unsigned kRebuildBlocks = 1024;
@@ -1419,7 +1447,7 @@ template <class M, int TX, int TY, int TZ>
 inline void launch_tiles_near(const StepLaunch &L, const typename M::Args &a) {
   if (L.nl_mode == 4) launch_probe<M, TX, TY, TZ, 1>(L);
   else if (L.nl_mode) launch_list<M, TX, TY, TZ, 1>(a, L.grid, L.occupancy, L.block, L.stream, L.lds_slack, *L.nl, L.nl_mode, L.delta);
-  else launch_tiled<M, TX, TY, TZ, 1>(a, L.grid, L.occupancy, L.block, L.stream, L.lds_slack);
+  else launch_tiled<M, TX, TY, TZ, 1>(a, L);
 }
 
 // Dispatch on the stencil reach (RM = 1, 2 or 4 cells) and on the list mode.
@@ -1435,9 +1463,9 @@ inline void launch_tiles(const StepLaunch &L, const typename M::Args &a) {
     else if (R == 2) launch_list<M, TX, TY, TZ, 2>(a, L.grid, L.occupancy, L.block, L.stream, L.lds_slack, *L.nl, L.nl_mode, L.delta);
     else launch_list<M, TX, TY, TZ, 4>(a, L.grid, L.occupancy, L.block, L.stream, L.lds_slack, *L.nl, L.nl_mode, L.delta);
   } else {
-    if (R <= 1) launch_tiled<M, TX, TY, TZ, 1>(a, L.grid, L.occupancy, L.block, L.stream, L.lds_slack);
-    else if (R == 2) launch_tiled<M, TX, TY, TZ, 2>(a, L.grid, L.occupancy, L.block, L.stream, L.lds_slack);
-    else launch_tiled<M, TX, TY, TZ, 4>(a, L.grid, L.occupancy, L.block, L.stream, L.lds_slack);
+    if (R <= 1) launch_tiled<M, TX, TY, TZ, 1>(a, L);
+    else if (R == 2) launch_tiled<M, TX, TY, TZ, 2>(a, L);
+    else launch_tiled<M, TX, TY, TZ, 4>(a, L);
   }
 }
 
