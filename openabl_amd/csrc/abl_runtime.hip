@@ -179,6 +179,13 @@ struct AgentStore {
   bool sorted = false;
   GridView sgv{};
   size_t sorted_n = 0;
+  // neighbours that stay (StepDesc::fixed), for the stored order, radius and reach
+  uint4 *fx_nb = nullptr;
+  uint8_t *fx_len = nullptr;
+  size_t fx_cap = 0;
+  bool fx_ok = false;
+  float fx_t = 0.f;
+  int fx_reach = 0;
   // neighbour lists (abl_tile.hpp): valid for the stored order while nl_ok
   bool nl_ok = false;
   uint16_t *nl_idx = nullptr, *nl_len = nullptr;
@@ -323,7 +330,12 @@ static void free_store(AgentStore &s) {
   s.skey[0] = s.skey[1] = s.dirty = nullptr;
   s.mhead = s.mnext = nullptr;
   s.sorted = false;
-  void *nl_ptrs[] = {s.nl_idx, s.nl_len, s.nl_pos0, s.nl_gate, s.nl_perm, s.nl_prow0};
+  void *nl_ptrs[] = {s.nl_idx, s.nl_len, s.nl_pos0, s.nl_gate, s.nl_perm, s.nl_prow0,
+                     s.fx_nb, s.fx_len};
+  s.fx_nb = nullptr;
+  s.fx_len = nullptr;
+  s.fx_cap = 0;
+  s.fx_ok = false;
   for (void *p : nl_ptrs) {
     if (p) (void) hipFree(p);
   }
@@ -370,6 +382,7 @@ static size_t store_bytes(const AgentStore &s) {
   const size_t tiles = (s.cells_cap + 2047) / 2048;
   b += s.cells_cap * (4 + 8 + 4 + 8) + std::max<size_t>(tiles, 1) * 4;  // count, start x2, dirty, head; bsum
   if (s.nl_idx) b += s.nl_ncap * ((size_t) s.nl_cap * 2 + kListMetaBytes) + kGateWords * 4;
+  b += s.fx_cap * (16 + 1);                // kept neighbours
   b += s.bcap * col_bytes(s);              // newborn staging
   return b;
 }
@@ -915,6 +928,7 @@ static int build_grid(abl_sim *sim, AgentStore &s) {
   const int n = (int) s.n;
   const int nc = (int) s.ncells;
   hipStream_t st = sim->stream;
+  s.fx_ok = false;
   const bool delta = sim->grid_delta && n > 0 && s.mnext && s.sorted && s.sorted_n == s.n &&
                      same_grid(s.gv, s.sgv);
   s.gen += 1;
@@ -1642,6 +1656,35 @@ static int read_crowd(abl_sim *sim, AgentStore &b) {
   return ABL_OK;
 }
 
+// Room for the neighbours of type b that L's step keeps; without it the launcher
+// walks the stencil.
+static void keep_neighbours(AgentStore &b, StepLaunch &L) {
+  if (b.fx_cap < b.n) {
+    void *old[] = {b.fx_nb, b.fx_len};
+    b.fx_nb = nullptr;
+    b.fx_len = nullptr;
+    b.fx_cap = 0;
+    b.fx_ok = false;
+    for (void *p : old) {
+      if (p && hipFree(p) != hipSuccess) return;
+    }
+    if (hipMalloc(&b.fx_nb, b.cap * sizeof(uint4)) != hipSuccess ||
+        hipMalloc(&b.fx_len, b.cap) != hipSuccess) {
+      (void) hipGetLastError();
+      if (b.fx_nb) (void) hipFree(b.fx_nb);
+      b.fx_nb = nullptr;
+      b.fx_len = nullptr;
+      return;
+    }
+    b.fx_cap = b.cap;
+  }
+  L.fixed = FixedNeighbours{b.fx_nb, b.fx_len,
+                            !b.fx_ok || b.fx_t != L.near_t || b.fx_reach != L.grid.reach};
+  b.fx_ok = true;
+  b.fx_t = L.near_t;
+  b.fx_reach = L.grid.reach;
+}
+
 // What the host looks at while a type walks lists: the longest list built and
 // the number of rebuilds run since the lists were entered (NListArgs::stats).
 // It copies them to pinned memory behind an event, the first time kListSample
@@ -1975,6 +2018,8 @@ static int launch_step(abl_sim *sim, const StepDesc &st, uint32_t ordinal) {
     L.lds_slack = sim->lds_slack;
     L.occupancy = b.ncells ? (float) ((double) b.n / (double) b.ncells) : 0.f;
     L.rc = (float) (r / b.cell * (1.0 + 1.0 / 1048576.0));
+    if (st.fixed && st.near_agent == st.agent && sim->order == 0 && sim->tile != 0 && L.n > 0)
+      keep_neighbours(b, L);
     // crowded tiles: one thread per agent instead (unless lists are asked for)
     if ((st.nlist || st.tiles) && st.near_agent == st.agent && sim->order == 0 &&
         sim->tile != 0 && !(sim->nlist_set && sim->nlist)) {

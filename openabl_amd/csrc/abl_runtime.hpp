@@ -93,6 +93,9 @@ struct StepDesc {
   // the launcher tiles the step (StepLaunch::nl_mode 4 probes its tiles); set
   // for tiled steps without lists, which nlist implies it for
   bool tiles;
+  // the near loop visits its own type, whose positions no step writes: the
+  // launcher keeps each agent's neighbours between two sorts (StepLaunch::fixed)
+  bool fixed;
 };
 
 struct ProgramDesc {
@@ -124,6 +127,14 @@ struct ColSet {
   void *c[kMaxCols];
 };
 
+// Neighbours kept for as long as the stored order stands (launchers of steps with
+// StepDesc::fixed say what the words hold).
+struct FixedNeighbours {
+  uint4 *nb;     // [n], or null: none kept
+  uint8_t *len;  // [n]
+  bool build;    // not built yet for this order, radius and reach
+};
+
 struct StepLaunch {
   hipStream_t stream;
   int precision;       // abl_precision
@@ -148,6 +159,7 @@ struct StepLaunch {
   const NListArgs *nl;
   const DeltaArgs *delta;
   float rc;            // near radius in cell units, widened by 2^-20
+  FixedNeighbours fixed;
   // run-time add()/removeCurrent() and random() inside steps
   const int32_t *self_id;  // ids of the stepping agents
   // removeCurrent() and add() flags: a step that removes, or adds, writes 0 or 1

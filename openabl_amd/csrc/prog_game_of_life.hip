@@ -14,7 +14,7 @@
 #include <vector>
 
 #include "abl_runtime.hpp"
-#include "abl_tile.hpp"
+#include "abl_pipeline.hpp"
 
 namespace abl {
 namespace {
@@ -28,9 +28,8 @@ struct LifeArgs {
   uint8_t *out_alive;
   GridView g;
   float near_t;
-  float rc;
-  int cap;
   int n;
+  FixedNeighbours fx;
 };
 
 __device__ __forceinline__ uint8_t life_rule(bool alive, int living) {
@@ -44,11 +43,9 @@ __device__ __forceinline__ uint8_t life_rule(bool alive, int living) {
   return out ? 1 : 0;
 }
 
+// Cells within the radius of agent i that are alive, by the stencil.
 template <typename F>
-__global__ __launch_bounds__(1024) void life_step(LifeArgs<F> a) {
-  const unsigned blk = xcd_block(blockIdx.x, gridDim.x);
-  const int i = (int) (blk * blockDim.x + threadIdx.x);
-  if (i >= a.n) return;
+__device__ __forceinline__ int life_walk(const LifeArgs<F> &a, int i) {
   const F x = a.px[i], y = a.py[i];
   const int3 c = cell_of<F>(a.g, x, y, (F) 0);
   int living = 0;
@@ -57,32 +54,84 @@ __global__ __launch_bounds__(1024) void life_step(LifeArgs<F> a) {
     if (f > a.near_t) return;
     living += a.alive[j] ? 1 : 0;
   });
-  a.out_alive[i] = life_rule(a.alive[i] != 0, living);
+  return living;
 }
 
-// LDS-tiled policy (abl_tile.hpp): records {x, y, alive as 0/1}.
-template <typename F_>
-struct LifePolicy {
-  using F = F_;
-  static constexpr int DIM = 2, NS = 3;
-  using Args = LifeArgs<F>;
-  __device__ static void load(const Args &a, uint32_t j, F *r) {
-    r[0] = a.px[j];
-    r[1] = a.py[j];
-    r[2] = a.alive[j] ? (F) 1 : (F) 0;
-  }
-  struct Acc {
-    int living;
-    __device__ void visit(const Args &a, const F *own, const F *nb) {
-      if (dist_sq_f32<F>(nb[0], nb[1], own[0], own[1]) > a.near_t) return;
-      living += nb[2] != (F) 0 ? 1 : 0;
+template <typename F>
+__global__ __launch_bounds__(1024) void life_step(LifeArgs<F> a) {
+  const unsigned blk = xcd_block(blockIdx.x, gridDim.x);
+  const int i = (int) (blk * blockDim.x + threadIdx.x);
+  if (i >= a.n) return;
+  a.out_alive[i] = life_rule(a.alive[i] != 0, life_walk(a, i));
+}
+
+// Positions never change, so neither does who is whose neighbour: up to eight of
+// them, as signed 16-bit distances in slots, are kept for as long as the stored
+// order stands, with their number and whether the agent counts itself
+// (kLifeSelf).  An agent with more neighbours, or one further off, walks the
+// stencil.  A timestep is then 19 bytes per agent and eight reads of a byte, where
+// the walk tests some 20 candidates (1,048,576 cells, FP64: 8.9 us per timestep
+// against 31.8 with the walk by a thread per agent and 38.7 on LDS tiles; FP32 8.6,
+// 25.8 and 29.2).
+constexpr int kLifeKept = 8;
+constexpr uint8_t kLifeSelf = 0x80, kLifeWalk = 0x7F;
+
+template <typename F>
+__global__ __launch_bounds__(1024) void life_neighbours(LifeArgs<F> a) {
+  const unsigned blk = xcd_block(blockIdx.x, gridDim.x);
+  const int i = (int) (blk * blockDim.x + threadIdx.x);
+  if (i >= a.n) return;
+  const F x = a.px[i], y = a.py[i];
+  const int3 c = cell_of<F>(a.g, x, y, (F) 0);
+  uint64_t lo = 0, hi = 0;
+  uint32_t count = 0;
+  uint8_t self = 0;
+  bool fits = true;
+  for_each_candidate(a.g, c.x, c.y, 0, a.g.reach, [&](uint32_t j) {
+    const float f = dist_sq_f32<F>(a.px[j], a.py[j], x, y);
+    if (f > a.near_t) return;
+    if ((int) j == i) {
+      self = kLifeSelf;
+      return;
     }
-  };
-  __device__ static void begin(const Args &, Acc &s, const F *) { s.living = 0; }
-  __device__ static void finish(const Args &a, Acc &s, const F *own, uint32_t i, double *) {
-    a.out_alive[i] = life_rule(own[2] != (F) 0, s.living);
+    const int d = (int) j - i;
+    fits = fits && d >= -32768 && d <= 32767;
+    const uint64_t v = (uint64_t) ((uint32_t) d & 0xFFFFu) << (16u * (count & 3u));
+    if (count < 4u) lo |= v;
+    else if (count < (uint32_t) kLifeKept) hi |= v;
+    count++;
+  });
+  fits = fits && count <= (uint32_t) kLifeKept;
+  a.fx.len[i] = fits ? (uint8_t) (count | self) : kLifeWalk;
+  a.fx.nb[i] = make_uint4((uint32_t) lo, (uint32_t) (lo >> 32), (uint32_t) hi, (uint32_t) (hi >> 32));
+}
+
+template <typename F>
+__global__ __launch_bounds__(1024) void life_step_fixed(LifeArgs<F> a) {
+  const unsigned blk = xcd_block(blockIdx.x, gridDim.x);
+  const int i = (int) (blk * blockDim.x + threadIdx.x);
+  if (i >= a.n) return;
+  const uint8_t len = a.fx.len[i];
+  const bool alive = a.alive[i] != 0;
+  int living;
+  if (len == kLifeWalk) {
+    living = life_walk(a, i);
+  } else {
+    const uint4 e = a.fx.nb[i];
+    const uint32_t w[4] = {e.x, e.y, e.z, e.w};
+    const int count = len & 0x0F;
+    uint8_t v[kLifeKept];
+#pragma unroll
+    for (int k = 0; k < kLifeKept; k++) {  // all in flight; unused entries read the agent's own
+      const int d = (int) (int16_t) (w[k / 2] >> (16 * (k & 1)));
+      v[k] = a.alive[k < count ? i + d : i];
+    }
+    living = (len & kLifeSelf) && alive ? 1 : 0;
+#pragma unroll
+    for (int k = 0; k < kLifeKept; k++) living += k < count && v[k] ? 1 : 0;
   }
-};
+  a.out_alive[i] = life_rule(alive, living);
+}
 
 template <typename F>
 void launch_typed(const StepLaunch &L) {
@@ -93,16 +142,15 @@ void launch_typed(const StepLaunch &L) {
   a.out_alive = (uint8_t *) L.out.c[2];
   a.g = L.grid;
   a.near_t = L.near_t;
-  a.rc = L.rc;
   a.n = L.n;
-  using M = LifePolicy<F>;
-  if (L.tile != 0 && L.grid.reach == 1) {
-    launch_tiled<M, 16, 8, 1, 1>(a, L);
-  } else if (L.tile != 0 && L.grid.reach == 2) {
-    launch_tiled<M, 16, 8, 1, 2>(a, L);
-  } else {
-    hipLaunchKernelGGL(life_step<F>, grid_blocks(L.n, L.block), L.block, 0, L.stream, a);
+  a.fx = L.fixed;
+  const unsigned nb = grid_blocks(L.n, L.block);
+  if (!L.fixed.nb) {
+    hipLaunchKernelGGL(life_step<F>, nb, L.block, 0, L.stream, a);
+    return;
   }
+  if (L.fixed.build) hipLaunchKernelGGL(life_neighbours<F>, nb, L.block, 0, L.stream, a);
+  hipLaunchKernelGGL(life_step_fixed<F>, nb, L.block, 0, L.stream, a);
 }
 
 // main() of game_of_life.abl before simulate:
@@ -162,7 +210,8 @@ const ProgramDesc *program_game_of_life() {
       {{"Cell", {{"pos", K_FLOAT2, true}, {"alive", K_BOOL, false}}}},
       {{"radius", 1.5}, {"debug", 0}, {"alive_fraction", 0.1}, {"num_agents", 400},
        {"num_timesteps", 100}, {"size", 20}},
-      {{"step_move", 0, 0, "radius", 1.0, 0x4u, launch_step_move}},
+      {{"step_move", 0, 0, "radius", 1.0, 0x4u, launch_step_move, false, 0, false,
+        nullptr, false, true}},
       env,
       host_init,
   };

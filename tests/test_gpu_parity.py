@@ -291,3 +291,42 @@ def test_boids_radius_boundary(prec, order):
     sim.upload(recs)
     sim.simulate(1)
     assert field_bytes(state(sim, "boids2d", prec)) == field_bytes(o.agents())
+
+
+@pytest.mark.parametrize("prec", ["f64", "f32"])
+@pytest.mark.parametrize("case", ["one", "lattice", "crowded", "far"])
+def test_life_kept_neighbours_equal_walk(case, prec):
+    """game_of_life keeps up to eight neighbours of a cell between sorts, as
+    16-bit slot distances: the walk's bytes (hip.tile=0) for a single cell, the
+    lattice, cells with more than eight neighbours and cells whose neighbours'
+    slots are further off; after a change of radius and a second upload too."""
+    from openabl_amd import MEMBERS, Simulation, record_dtype
+    print(f"case life kept neighbours {case} {prec}", flush=True)
+    rng = np.random.default_rng(7)
+    size = {"one": 1, "lattice": 37, "crowded": 40, "far": 200}[case]
+    xy = np.stack(np.meshgrid(np.arange(size) + 0.5, np.arange(size) + 0.5), -1).reshape(-1, 2)
+    if case == "crowded":
+        xy = np.concatenate([xy, rng.uniform(0, size, (1500, 2))])
+    if case == "far":  # 40,000 cells in a strip between the lattice's rows
+        xy = np.concatenate([xy, rng.uniform((20, 90.5), (120, 91.5), (40000, 2))])
+    dt = record_dtype(MEMBERS["game_of_life"], prec)
+    recs = [np.zeros(len(xy), dt) for _ in range(2)]
+    for r in recs:
+        order = rng.permutation(len(xy))
+        r["pos"] = xy[order].astype(r["pos"].dtype)
+        r["alive"] = rng.random(len(xy)) < 0.4
+    outs = []
+    for tile in (1, 0):
+        sim = Simulation("game_of_life", prec, config={"hip.tile": tile},
+                         params=dict(game_of_life_params(num_agents=len(xy)), size=size))
+        got = []
+        for r, radius in ((recs[0], 1.5), (recs[0], 1.2), (recs[1], 1.5)):
+            sim.set_param("radius", radius)
+            sim.upload(r)
+            sim.simulate(5)
+            got.append(field_bytes(sim.download(dt)))
+            sim.simulate(2)
+            got.append(field_bytes(sim.download(dt)))
+        outs.append(got)
+        sim.close()
+    assert outs[0] == outs[1]
