@@ -1326,8 +1326,11 @@ std::string Gen::device_program() {
   }
   // the program description
   static const char *kKind[] = {"", "", "K_BOOL", "K_INT", "K_FLOAT", "", "K_FLOAT2", "K_FLOAT3"};
-  o << "\nconst ProgramDesc *program() {\n  static const ProgramDesc d = {\n    \"" << prog_name
-    << "\",\n    {";
+  std::string tiled;  // steps the launcher runs on the LDS tiles
+  for (size_t k = 0; k < steps.size(); k++)
+    if (tile_capable(*steps[k])) tiled += (tiled.empty() ? "" : ", ") + std::to_string(k);
+  o << "\nconst ProgramDesc *program() {\n  static const ProgramDesc d = "
+    << (tiled.empty() ? "{" : "with_tiles({") << "\n    \"" << prog_name << "\",\n    {";
   for (size_t t = 0; t < S.agents.size(); t++) {
     AgentDecl *ag = S.agents[t];
     o << (t ? ",\n     " : "") << "{\"" << ag->name << "\", {";
@@ -1348,11 +1351,11 @@ std::string Gen::device_program() {
       << (f->near_agent ? f->near_agent->index : -1) << ", nullptr, 0.0, " << w << "u, launch_"
       << f->name << ", " << (f->uses_removal ? "true" : "false") << ", " << adds << ", "
       << (list_capable(*f) ? "true" : "false") << ", "
-      << (f->near_agent ? "radius_" + f->name : std::string("nullptr")) << ", "
-      << (tile_capable(*f) ? "true" : "false") << "}";
+      << (f->near_agent ? "radius_" + f->name : std::string("nullptr")) << "}";
   }
   o << "},\n    env,\n    nullptr,\n    nullptr,\n    nullptr,\n    false,\n    "
-    << (S.simulate && S.simulate->seq_decl ? "seq_step" : "nullptr") << ",\n  };\n  return &d;\n}\n\n"
+    << (S.simulate && S.simulate->seq_decl ? "seq_step" : "nullptr") << ",\n  }"
+    << (tiled.empty() ? "" : ", {" + tiled + "})") << ";\n  return &d;\n}\n\n"
     << "const bool registered = register_program(program());\n\n}  // namespace " << ns << "\n";
   return o.str();
 }

@@ -11,6 +11,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <initializer_list>
 #include <string>
 #include <vector>
 
@@ -120,6 +121,12 @@ struct ProgramDesc {
   // instead of seq_step when set
   int (*seq_step_prec)(struct ::abl_sim *sim, int precision);
 };
+
+// The program with StepDesc::tiles set for these steps (generated programs).
+inline ProgramDesc with_tiles(ProgramDesc d, std::initializer_list<size_t> steps) {
+  for (const size_t k : steps) d.steps[k].tiles = true;
+  return d;
+}
 
 // Column pointers of one agent type (members in declaration order, vector
 // components expanded x, y, z).
