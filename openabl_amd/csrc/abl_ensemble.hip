@@ -80,6 +80,26 @@ __global__ void k_ens_bin(const P *__restrict__ px, const P *__restrict__ py, En
   atomicAdd(&count[k], 1u);
 }
 
+// The phases of the gated re-sort as launches of their own (issue_rebuild): the
+// slots of the members due are binned, and placed.
+template <typename P>
+__global__ __launch_bounds__(256) void k_ens_delta(DeltaArgs d, EnsTiles e, const uint32_t *gate,
+                                                   int parity, int phase) {
+  if (gate[parity] == 0u) return;
+  const int i = (int) (blockIdx.x * 256u + threadIdx.x);
+  if (i >= d.n) return;
+  const int m = member_of(e.off, e.members, (uint32_t) i);
+  if (e.mgate[parity * e.members + m] == 0u) return;
+  const uint32_t gen = gate[kGateGen];
+  if (phase == 0)
+    bin_delta_item(i, e.cell_base[m] + cell_key<P>(e.grids[m], (const P *) d.px, (const P *) d.py,
+                                                   (const P *) nullptr, i),
+                   d.skey, d.key, d.count, d.bsum, d.ml, gen);
+  else
+    place_item(i, d.key, d.skey, d.skey_out, d.start_old, d.start_new, d.ml, gen, d.gc, d.id_in,
+               d.id_out, d.n);
+}
+
 // slot s of member m back to record id within that member's output block
 __global__ void k_ens_unpermute(char *__restrict__ aos, ColSet cols, int elem, int ncols,
                                 const int32_t *__restrict__ id, uint32_t begin, int n) {
@@ -139,7 +159,12 @@ struct abl_ensemble {
   uint32_t *start_new = nullptr;           // the rebuild's cell offsets
   uint32_t *dirty = nullptr;               // MoverLists
   unsigned long long *mhead = nullptr, *mnext = nullptr;
-  uint32_t *h_error = nullptr;   // pinned copy of the error flag, as of the last simulate()
+  uint32_t *h_error = nullptr;   // pinned copy of the error flag and the generation, as of the
+                                 // last simulate()
+  // four launches per rebuild instead of one: most timesteps since the last look rebuilt
+  bool split = false;
+  uint32_t gen_seen = 1;
+  uint64_t step_seen = 0;
   // download workspace: one member's records, grown to the largest asked for
   std::mutex dl_lock;
   void *dl = nullptr;
@@ -381,7 +406,9 @@ static NListArgs ens_build_args(const abl_ensemble *e) {
   return nl;
 }
 
-// The gated rebuild of the current timestep (tiled_rebuild_multi).
+// The gated rebuild of the current timestep: one launch (tiled_rebuild_multi), or
+// four (ens_check), which cost a timestep without a rebuild about 10 us more and one
+// with a rebuild 50 us less; the same results.
 static int issue_rebuild(abl_ensemble *e) {
   DeltaArgs d{};
   const int b = e->cur;
@@ -407,9 +434,19 @@ static int issue_rebuild(abl_ensemble *e) {
   d.q_other = queues + (~e->timestep & 1u);
   d.error = e->nl_gate + kGateError;
   d.spins = kPhaseSpins;
-  const int rc = e->hooks->launch_multi_list(e->precision, e->d_build[b], ens_tiles(e), e->reach,
-                                             e->occupancy, e->tile, e->block, e->stream,
-                                             ens_build_args(e), &d, 3);
+  NListArgs nl = ens_build_args(e);
+  nl.gated = 1;
+  const EnsTiles t = ens_tiles(e);
+  if (e->split) {
+    const auto delta = e->elem == 8 ? k_ens_delta<double> : k_ens_delta<float>;
+    hipLaunchKernelGGL(delta, grid_blocks(d.n, 256), 256, 0, e->stream, d, t, nl.gate, nl.parity, 0);
+    hipLaunchKernelGGL(k_scan_apply, d.nscan, kScanBlock, 0, e->stream, e->count, e->bsum,
+                       e->start_new, d.ncells, nl.gate + nl.parity);
+    hipLaunchKernelGGL(delta, grid_blocks(d.n, 256), 256, 0, e->stream, d, t, nl.gate, nl.parity, 2);
+  }
+  const int rc = e->hooks->launch_multi_list(e->precision, e->d_build[b], t, e->reach,
+                                             e->occupancy, e->tile, e->block, e->stream, nl,
+                                             e->split ? nullptr : &d, e->split ? 1 : 3);
   return rc ? ens_fail(rc, "list rebuild: no launch size") : ABL_OK;
 }
 
@@ -440,8 +477,11 @@ static int init_lists(abl_ensemble *e) {
   ENS_TRY(hipMalloc(&e->mnext, N * 8));
   ENS_TRY(hipMemsetAsync(e->dirty, 0, e->ncells * 4, e->stream));
   ENS_TRY(hipMemsetAsync(e->mhead, 0, e->ncells * 8, e->stream));
-  ENS_TRY(hipHostMalloc((void **) &e->h_error, 4, hipHostMallocDefault));
-  *e->h_error = 0u;
+  ENS_TRY(hipHostMalloc((void **) &e->h_error, 8, hipHostMallocDefault));
+  e->h_error[0] = 0u;
+  e->h_error[1] = e->gen_seen = 1u;
+  e->step_seen = 0;
+  e->split = false;
   // The lists below are those of the initial state: no member is due at the
   // first timestep (an overflowed list sets its member's gate at that step).
   std::vector<uint32_t> words(kGateWords, 0u), none(2 * M, 0u);
@@ -720,14 +760,30 @@ extern "C" int abl_ens_simulate(abl_ensemble *e, int steps) {
   }
   ENS_TRY(hipEventRecord(e->ev1, e->stream));
   if (e->h_error)
-    ENS_TRY(hipMemcpyAsync(e->h_error, e->nl_gate + kGateError, 4, hipMemcpyDeviceToHost, e->stream));
+    ENS_TRY(hipMemcpyAsync(e->h_error, e->nl_gate + kGateError, 8, hipMemcpyDeviceToHost, e->stream));
   return ABL_OK;
 }
 
-// After a synchronisation: no rebuild of the timesteps so far gave up waiting.
-static int ens_check(const abl_ensemble *e) {
-  if (e->h_error && *(const volatile uint32_t *) e->h_error)
-    return ens_fail(ABL_ERR_DEVICE, "list rebuild: a phase did not finish");
+// After a synchronisation: no rebuild of the timesteps so far gave up waiting; and
+// the form of the rebuilds to come, by how many of these timesteps rebuilt.
+static int ens_check(abl_ensemble *e) {
+  if (!e->h_error) return ABL_OK;
+  const volatile uint32_t *h = e->h_error;
+  if (h[0]) return ens_fail(ABL_ERR_DEVICE, "list rebuild: a phase did not finish");
+  const uint64_t steps = e->timestep - e->step_seen;
+  if (steps >= 8) {
+    const bool split = (uint64_t) (h[1] - e->gen_seen) * 4u > steps;
+    e->gen_seen = h[1];
+    e->step_seen = e->timestep;
+    if (split != e->split) {
+      e->split = split;
+      ENS_TRY(hipMemsetAsync(e->nl_gate + kGateQueue, 0, (kGateWords - kGateQueue) * 4, e->stream));
+      if (e->exec) ENS_TRY(hipGraphExecDestroy(e->exec));
+      if (e->graph) ENS_TRY(hipGraphDestroy(e->graph));
+      e->exec = nullptr;
+      e->graph = nullptr;
+    }
+  }
   return ABL_OK;
 }
 

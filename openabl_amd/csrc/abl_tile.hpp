@@ -1224,16 +1224,20 @@ __global__ __launch_bounds__(256, policy_list_waves<M>::value) void tiled_step_l
 // members + m].  A member rebuilds exactly when a run of it alone would: when
 // one of its own agents strayed or overflowed.
 
-// Every member's first lists, after the full sort (records in the sorted buffers
-// args point at; copied back as in tiled_list_build).
+// Every member's first lists, after the full sort, or (nl.gated) those of the
+// members due (records in the sorted buffers args point at; copied back as in
+// tiled_list_build).
 template <class M, int TX, int TY, int TZ, int RM>
 __global__ __launch_bounds__(256) void tiled_list_build_multi(const typename M::Args *__restrict__ args,
                                                               const uint2 *__restrict__ tile_of,
-                                                              NListArgs nl) {
+                                                              int members, NListArgs nl,
+                                                              const uint32_t *__restrict__ mgate) {
   extern __shared__ __align__(16) unsigned char smem[];
+  if (nl.gated && nl.gate[nl.parity] == 0u) return;
   list_copy_starts(nl);
   const unsigned t = xcd_block(blockIdx.x, gridDim.x);
   const uint2 of = tile_of[t];
+  if (nl.gated && mgate[nl.parity * members + uniform((int) of.x)] == 0u) return;
   const uint32_t longest = list_build_tile<M, TX, TY, TZ, RM>(
       args[uniform((int) of.x)], nl, t - (unsigned) uniform((int) of.y), smem);
   list_longest(nl, longest);
@@ -1243,8 +1247,9 @@ __global__ __launch_bounds__(256) void tiled_list_build_multi(const typename M::
 // (tiled_rebuild), over the chunks of those members only.  30 members of 1,000 to
 // 65,536 boids: a timestep with no member due 37 us (of it 4.6 us for this launch
 // that returns) against 48 us with seven gated launches for the full sort and the list
-// build; with one to a few members due each step 64 against 69 us, with every
-// member due 230 us against 143: a skin that small is not worth its lists.
+// build.  Where members are due on most timesteps the ensemble takes the re-sort's
+// phases as launches of their own instead (ens_check): every member due on every
+// timestep 230 us this way, 130 with four launches.
 template <class M, int TX, int TY, int TZ, int RM>
 __global__ __launch_bounds__(256) void tiled_rebuild_multi(const typename M::Args *__restrict__ args,
                                                             EnsTiles e, NListArgs nl, DeltaArgs d) {

@@ -102,12 +102,14 @@ def test_rebuild_chunks_of_many_members(count, most, graph):
     ens = Ensemble("boids2d", "f64", ms, config=dict(cfg, **{"hip.graph": graph}))
     ens.init(0x1234, 0x5678)
     ens.simulate(9)
+    ens.synchronize()  # most timesteps rebuilt: four launches per rebuild from here on
+    ens.simulate(7)
     dt = record_dtype(MEMBERS["boids2d"], "f64")
     for m in sorted({0, count // 2, count - 1, *rng.integers(0, count, 3).tolist()}):
         load_library().abl_rng_seed(*member_seed(0x1234, 0x5678, m))
         sim = Simulation("boids2d", "f64", params=ms[m], config=cfg)
         sim.init_agents()
-        sim.simulate(9)
+        sim.simulate(16)
         assert field_bytes(ens.download(m)) == field_bytes(sim.download(dt)), m
         sim.close()
     ens.close()
