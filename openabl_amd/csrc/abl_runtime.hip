@@ -20,6 +20,8 @@
 // ascending id, which is independent of history: a run gives the same result
 // alone or beside other runs.
 #include <hip/hip_runtime.h>
+#include <sys/mman.h>
+#include <unistd.h>
 
 #include <algorithm>
 #include <atomic>
@@ -30,6 +32,7 @@
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "../../include/abl_hip.h"
@@ -1300,6 +1303,42 @@ extern "C" int abl_hip_count(abl_sim *sim, int t, size_t *count) {
 
 static int check_rebuild(abl_sim *sim);
 
+// Have the pages of a large download's destination ready while the device still
+// works: freshly allocated memory costs the copy a fault and a cleared page at a
+// time otherwise.  Contents stay as they are; where the kernel lacks the call
+// nothing happens.  1,048,576 boids (34 MB): 3.5 -> 2.6 ms where the device is idle
+// already, and 14.7 -> 13.5 ms from upload to download of 200 timesteps.
+static void populate_pages(void *p, size_t bytes) {
+#ifdef MADV_POPULATE_WRITE
+  constexpr size_t kLeast = (size_t) 16 << 20, kParts = 4, kAlign = (size_t) 2 << 20;
+  if (bytes < kLeast) return;
+  const uintptr_t page = (uintptr_t) sysconf(_SC_PAGESIZE);
+  const uintptr_t a = ((uintptr_t) p + page - 1) & ~(page - 1), z = ((uintptr_t) p + bytes) & ~(page - 1);
+  if (z <= a) return;
+  const uintptr_t part = ((z - a) / kParts + kAlign - 1) & ~(kAlign - 1);
+  auto fill = [](uintptr_t from, uintptr_t to) {
+    if (to > from) (void) madvise((void *) from, to - from, MADV_POPULATE_WRITE);
+  };
+  std::thread others[kParts - 1];
+  uintptr_t from = a;
+  try {
+    for (std::thread &o : others) {
+      const uintptr_t to = std::min(from + part, z);
+      o = std::thread(fill, from, to);
+      from = to;
+    }
+  } catch (const std::exception &) {  // no thread to be had: the rest is this one's
+  }
+  fill(from, z);
+  for (std::thread &o : others) {
+    if (o.joinable()) o.join();
+  }
+#else
+  (void) p;
+  (void) bytes;
+#endif
+}
+
 extern "C" int abl_hip_download(abl_sim *sim, int t, void *aos, size_t capacity, size_t *count) {
   CHECK_SIM(sim);
   if (t < 0 || t >= (int) sim->types.size()) return fail(ABL_ERR_ARG, "agent type out of range");
@@ -1307,6 +1346,7 @@ extern "C" int abl_hip_download(abl_sim *sim, int t, void *aos, size_t capacity,
   if (count) *count = s.n;
   if (s.n == 0) return ABL_OK;
   if (!aos || capacity < s.n) return fail(ABL_ERR_ARG, "download buffer too small");
+  populate_pages(aos, s.n * s.aos_size);
   HIP_TRY(hipStreamSynchronize(sim->stream));
   int rc = check_rebuild(sim);
   if (rc) return rc;
