@@ -1038,7 +1038,8 @@ __device__ __forceinline__ bool rebuild_phases(const DeltaArgs &d, uint32_t chun
 // scan tile, piece of the offsets and tile, each released by all four waves, a
 // rebuild took 1,840 us for 1,000,003 agents (the same phases as four launches
 // 125 us) and 102 us for 1,000; with one item per block and phase, released by
-// one thread, and the tiles not claimed at all it takes 310 us and 60 us.
+// one thread, and the tiles not claimed at all it takes 310 us and 60 us; with the
+// counters in shards 285 us for 1,048,576 boids and 36 for 1,000.
 template <class M, int TX, int TY, int TZ, int RM>
 __global__ __launch_bounds__(256) void tiled_rebuild(typename M::Args a, NListArgs nl,
                                                       DeltaArgs d) {
