@@ -212,6 +212,7 @@ struct AgentStore {
   // whether the agents crowd into tiles that do not fit LDS (probe_tiles),
   // looked at once per upload, parameter or configuration change
   bool dense = false, dense_known = false;
+  uint32_t crowd = 0;  // those agents, as last counted
   uint64_t nl_t_req = 0, nl_t_prev = 0;
   uint32_t nl_c_prev = 0;
   // run-time add/remove: ids stop being 0..n-1 once agents die or are born
@@ -1688,11 +1689,10 @@ static int probe_tiles(abl_sim *sim, AgentStore &b, const StepDesc &st, const St
 }
 
 static int read_crowd(abl_sim *sim, AgentStore &b) {
-  uint32_t crowd = 0;
-  const int rc = read_count(sim, crowd_word(sim, b), &crowd);
+  const int rc = read_count(sim, crowd_word(sim, b), &b.crowd);
   if (rc) return rc;
   b.dense_known = true;
-  b.dense = crowd >= crowd_limit(b);
+  b.dense = b.crowd >= crowd_limit(b);
   return ABL_OK;
 }
 
@@ -1872,6 +1872,7 @@ static int enter_lists(abl_sim *sim, AgentStore &b, const StepDesc &st, const St
     const uint32_t longest = words[0];
     b.dense_known = true;
     b.dense = nl.crowd && words[1] >= nl.crowd_limit;
+    if (nl.crowd) b.crowd = words[1];
     if (b.dense) return ABL_OK;
     // watched from here on (list_watch)
     b.nl_c_prev = words[2];
@@ -2309,6 +2310,22 @@ extern "C" int abl_hip_footprint(abl_sim *sim, size_t *bytes) {
   for (const AgentStore &s : sim->types) b += store_bytes(s);
   if (sim->dead) b += sim->fcap * (1 + 1 + 4 + 4) + (sim->fcap / kDeadTile + 2) * 4;
   *bytes = b;
+  return ABL_OK;
+}
+
+// What the runtime has decided for an agent type.
+extern "C" int abl_hip_inspect(abl_sim *sim, int t, const char *what, double *value) {
+  CHECK_SIM(sim);
+  if (t < 0 || t >= (int) sim->types.size()) return fail(ABL_ERR_ARG, "agent type out of range");
+  if (!what || !value) return fail(ABL_ERR_ARG, "null argument");
+  const AgentStore &s = sim->types[t];
+  const std::string k(what);
+  if (k == "lists") *value = s.nl_ok;
+  else if (k == "lists_given_up") *value = s.nl_off;
+  else if (k == "list_capacity") *value = s.nl_cap;
+  else if (k == "crowded") *value = s.dense_known && s.dense;
+  else if (k == "crowded_agents") *value = s.crowd;
+  else return fail(ABL_ERR_ARG, "unknown quantity " + k);
   return ABL_OK;
 }
 

@@ -1354,17 +1354,24 @@ __global__ __launch_bounds__(256) void tile_probe(GridView g, int cap, unsigned 
     halo += (uint32_t) __shfl_xor((int) halo, d, kWave);
     own += (uint32_t) __shfl_xor((int) own, d, kWave);
   }
-  if (lane == 0 && (int) halo >= cap && own) atomicAdd(&stats[publish ? kProbeSum : 1], own);
-  if (!publish) return;
+  // one add per block, by the thread that then takes the ticket: its fence orders
+  // the two, and the last block's fence orders its reading behind every ticket (a
+  // block barrier alone does not wait for adds of other waves still under way)
+  __shared__ uint32_t crowded;
+  if (threadIdx.x == 0) crowded = 0u;
   __syncthreads();
-  if (threadIdx.x == 0) {
+  if (lane == 0 && (int) halo >= cap && own) atomicAdd(&crowded, own);
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  if (crowded) atomicAdd(&stats[publish ? kProbeSum : 1], crowded);
+  if (!publish) return;
+  __threadfence();
+  if (atomicAdd(&stats[kProbeTicket], 1u) == gridDim.x - 1u) {
     __threadfence();
-    if (atomicAdd(&stats[kProbeTicket], 1u) == gridDim.x - 1u) {
-      const uint32_t sum = atomicExch(&stats[kProbeSum], 0u);
-      stats[kProbeTicket] = 0u;
-      stats[kProbeCount] = sum;
-      __hip_atomic_store(publish, sum, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-    }
+    const uint32_t sum = atomicExch(&stats[kProbeSum], 0u);
+    stats[kProbeTicket] = 0u;
+    stats[kProbeCount] = sum;
+    __hip_atomic_store(publish, sum, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
   }
 }
 

@@ -57,6 +57,7 @@ _SIGNATURES = {
     "abl_hip_synchronize": ([C.c_void_p], C.c_int),
     "abl_hip_neighbours": ([C.c_void_p, C.c_int, C.c_void_p, C.c_size_t, C.c_void_p], C.c_int),
     "abl_hip_footprint": ([C.c_void_p, C.c_void_p], C.c_int),
+    "abl_hip_inspect": ([C.c_void_p, C.c_int, C.c_char_p, C.c_void_p], C.c_int),
     "abl_hip_last_timing": ([C.c_void_p, C.c_void_p], C.c_int),
     "abl_hip_download_ids": ([C.c_void_p, C.c_int, C.c_void_p, C.c_size_t, C.c_void_p], C.c_int),
     "abl_hip_reduce_sum": ([C.c_void_p, C.c_int, C.c_char_p, C.c_void_p], C.c_int),
@@ -284,6 +285,12 @@ class Simulation:
         b = C.c_size_t()
         _check(self.lib.abl_hip_footprint(self.h, C.byref(b)))
         return b.value
+
+    def inspect(self, what: str, t: int = 0) -> float:
+        """What the runtime has decided for agent type t (abl_hip_inspect)."""
+        v = C.c_double()
+        _check(self.lib.abl_hip_inspect(self.h, t, what.encode(), C.byref(v)))
+        return v.value
 
     def last_timing(self):
         out = (C.c_double * 3)()

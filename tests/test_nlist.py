@@ -297,3 +297,29 @@ def test_tile_shapes_equal(n, density, cfg, prec):
     for b in runs[1:]:
         for t, x, y in zip(steps, runs[0], b):
             assert field_bytes(x) == field_bytes(y), t
+
+
+@pytest.mark.parametrize("prec", ["f64", "f32", "f32c"])
+@pytest.mark.parametrize("cfg", [{"hip.nlist": 0}, {}], ids=["tiles", "lists"])
+def test_crowded_agents_are_counted_exactly(prec, cfg):
+    """The agents of tiles beyond LDS, added up by many blocks and handed to the
+    host by the last one: all of them where no tile fits, none where every tile
+    does, upload after upload (the count's words are left clear)."""
+    from openabl_amd import MEMBERS, Simulation, record_dtype
+    print(f"case nlist crowd count {prec} {cfg}", flush=True)
+    dt = record_dtype(MEMBERS["boids2d"], prec)
+    rng = np.random.default_rng(11)
+    # 16,384 agents at 256 per cell, and 60,000 at 6.6 (some 1,000 blocks count)
+    for n, density, want in ((16384, 16384 / 6400.0, 16384), (60000, 0.065536, 0)):
+        params = boids2d_params(num_agents=n)
+        params["agent_density"] = density
+        sim = Simulation("boids2d", prec, params=params, config=cfg)
+        recs = np.zeros(n, dt)
+        for _ in range(3):
+            recs["pos"] = rng.uniform(0, sim.get_param("max_pos"), (n, 2))
+            sim.upload(recs)
+            sim.simulate(2)
+            assert sim.inspect("crowded_agents") == want
+            assert sim.inspect("crowded") == (want > 0)
+            assert sim.inspect("lists") == (want == 0 and not cfg)
+        sim.close()
