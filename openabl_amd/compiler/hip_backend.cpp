@@ -1356,7 +1356,7 @@ std::string Gen::device_program() {
   o << "},\n    env,\n    nullptr,\n    nullptr,\n    nullptr,\n    false,\n    "
     << (S.simulate && S.simulate->seq_decl ? "seq_step" : "nullptr") << ",\n  }"
     << (tiled.empty() ? "" : ", {" + tiled + "})") << ";\n  return &d;\n}\n\n"
-    << "const bool registered = register_program(program());\n\n}  // namespace " << ns << "\n";
+    << "const bool registered = register_program(program(), program_abi(), true);\n\n}  // namespace " << ns << "\n";
   return o.str();
 }
 
@@ -1413,9 +1413,15 @@ void HipBackend::generate(Script &script, const Analysis &analysis, const Backen
   std::ostringstream b;
   b << "#!/bin/sh\n# generated by openabl-hip: the device program, then the host program\n"
     << "set -e\nROOT=\"${ABL_HIP_ROOT:-" << root << "}\"\n"
-    << "# nothing to do when both outputs are newer than their sources\n"
-    << "if [ -f libsteps.so ] && [ -f main ] && [ libsteps.so -nt steps.hip ] && "
-    << "[ main -nt main.cpp ] && [ main -nt abl_gen.h ]; then exit 0; fi\n"
+    << "# nothing to do when both outputs are newer than their sources, the runtime's\n"
+    << "# headers among them\n"
+    << "fresh() {\n"
+    << "  [ -f libsteps.so ] && [ -f main ] && [ libsteps.so -nt steps.hip ] && "
+    << "[ main -nt main.cpp ] && [ main -nt abl_gen.h ] || return 1\n"
+    << "  for h in \"$ROOT\"/include/abl_hip.h \"$ROOT\"/openabl_amd/csrc/*.hpp; do\n"
+    << "    [ ! -e \"$h\" ] || { [ libsteps.so -nt \"$h\" ] && [ main -nt \"$h\" ]; } || return 1\n"
+    << "  done\n}\n"
+    << "if fresh; then exit 0; fi\n"
     << "hipcc --offload-arch=${ABL_HIP_ARCH:-gfx950} -O3 -std=c++17 -ffp-contract=off "
     << "-Wno-parentheses-equality "
     << "-Xclang -target-feature -Xclang -packed-fp32-ops -fPIC -shared "

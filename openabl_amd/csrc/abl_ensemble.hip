@@ -195,7 +195,7 @@ extern "C" int abl_ens_create(const char *program, int precision, int members,
     return ens_fail(ABL_ERR_ARG, "bad argument");
   *out = nullptr;
   const ProgramDesc *prog = find_program(program);
-  if (!prog) return ens_fail(ABL_ERR_ARG, std::string("unknown program ") + program);
+  if (!prog) return ens_fail(ABL_ERR_ARG, no_program(program));
   if (!prog->ensemble) return ens_fail(ABL_ERR_UNSUPPORTED, "program has no ensemble support");
   if (precision != ABL_PREC_F64 && precision != ABL_PREC_F32)
     return ens_fail(ABL_ERR_UNSUPPORTED, "precision not supported");

@@ -466,8 +466,31 @@ inline void seq_log(abl_sim *sim, const char *fmt, A... args) {
 
 }  // namespace gen
 
+// What a step library and the runtime have to agree on: the structures they
+// hand each other (their sizes, taken when either is compiled) and what the
+// members mean (kStepContract, counted up with every change that sizes do not
+// show).
+constexpr uint64_t kStepContract = 2;
+constexpr uint64_t program_abi() {
+  uint64_t h = kStepContract;
+  for (const uint64_t size : {(uint64_t) sizeof(ProgramDesc), (uint64_t) sizeof(StepDesc),
+                              (uint64_t) sizeof(StepLaunch), (uint64_t) sizeof(NListArgs),
+                              (uint64_t) sizeof(DeltaArgs)})
+    h = (h ^ size) * 0x100000001B3ull;
+  return h;
+}
+
 // Register a generated step program with the runtime (abl_runtime.hip); a
-// generated library calls it from a static initialiser.
-bool register_program(const ProgramDesc *desc);
+// generated library calls it from a static initialiser.  `abi` as the library was
+// compiled: a library built for other structures is refused, and creating its
+// program fails saying so.  `writes_flags`: steps that remove or add write every
+// agent's flag (StepLaunch::dead); for others the runtime clears the flags before
+// each step.
+bool register_program(const ProgramDesc *desc, uint64_t abi, bool writes_flags);
+
+// The form of step programs emitted earlier, which write a flag only to set it.
+static inline bool register_program(const ProgramDesc *desc) {
+  return register_program(desc, program_abi(), false);
+}
 
 }  // namespace abl

@@ -93,26 +93,48 @@ static const ProgramDesc *const *programs() {
 
 // Programs registered at load time by generated step libraries
 // (register_program), after the built-in ones; a registered program of an
-// existing name replaces it for later lookups.
+// existing name replaces it for later lookups, also where it was refused.
+namespace {
+struct Registered {
+  std::string name;
+  const ProgramDesc *desc;  // null: refused
+  bool writes_flags;
+};
+}  // namespace
 static std::mutex g_registry_mu;
-static std::vector<const ProgramDesc *> &registered() {
-  static std::vector<const ProgramDesc *> v;
+static std::vector<Registered> &registered() {
+  static std::vector<Registered> v;
   return v;
 }
 
-bool abl::register_program(const ProgramDesc *desc) {
-  if (!desc || !desc->name) return false;
+bool abl::register_program(const ProgramDesc *desc, uint64_t abi, bool writes_flags) {
+  if (!desc || !desc->name) return false;  // the name is where it has always been
+  const bool fits = abi == program_abi();
   std::lock_guard<std::mutex> g(g_registry_mu);
-  registered().push_back(desc);
-  return true;
+  registered().push_back({desc->name, fits ? desc : nullptr, writes_flags});
+  return fits;
+}
+
+// What step libraries built before register_program took `abi` call.
+extern "C" bool abl_register_unversioned(const ProgramDesc *desc)
+    __asm__("_ZN3abl16register_programEPKNS_11ProgramDescE");
+extern "C" bool abl_register_unversioned(const ProgramDesc *desc) {
+  return abl::register_program(desc, 0, false);
+}
+
+// The latest registration of a name, or nullptr (registry locked).
+static const Registered *lookup(const char *name) {
+  const auto &v = registered();
+  for (auto it = v.rbegin(); it != v.rend(); ++it)
+    if (it->name == name) return &*it;
+  return nullptr;
 }
 
 const ProgramDesc *abl::find_program(const char *name) {
   if (!name) return nullptr;
   {
     std::lock_guard<std::mutex> g(g_registry_mu);
-    for (auto it = registered().rbegin(); it != registered().rend(); ++it)
-      if (std::strcmp((*it)->name, name) == 0) return *it;
+    if (const Registered *r = lookup(name)) return r->desc;
   }
   for (int i = 0; programs()[i]; i++) {
     if (std::strcmp(programs()[i]->name, name) == 0) return programs()[i];
@@ -120,11 +142,28 @@ const ProgramDesc *abl::find_program(const char *name) {
   return nullptr;
 }
 
+std::string abl::no_program(const char *name) {
+  std::lock_guard<std::mutex> g(g_registry_mu);
+  if (const Registered *r = lookup(name); r && !r->desc)
+    return std::string("program ") + name + " was built for another version of this runtime: "
+           "delete its libsteps.so and run its build.sh";
+  return std::string("unknown program ") + name;
+}
+
+// Whether a program's steps write every agent's add() and removeCurrent() flag.
+static bool writes_flags(const ProgramDesc *desc) {
+  std::lock_guard<std::mutex> g(g_registry_mu);
+  for (const Registered &r : registered())
+    if (r.desc == desc) return r.writes_flags;
+  return true;
+}
+
 extern "C" int abl_hip_program_count(void) {
   int n = 0;
   while (programs()[n]) n++;
   std::lock_guard<std::mutex> g(g_registry_mu);
-  return n + (int) registered().size();
+  for (const Registered &r : registered()) n += r.desc != nullptr;
+  return n;
 }
 
 extern "C" const char *abl_hip_program_name(int index) {
@@ -132,7 +171,8 @@ extern "C" const char *abl_hip_program_name(int index) {
   while (programs()[n]) n++;
   if (index >= 0 && index < n) return programs()[index]->name;
   std::lock_guard<std::mutex> g(g_registry_mu);
-  if (index >= n && index < n + (int) registered().size()) return registered()[index - n]->name;
+  for (const Registered &r : registered())
+    if (r.desc && index == n++) return r.desc->name;
   return nullptr;
 }
 
@@ -229,6 +269,7 @@ struct AgentStore {
 
 struct abl_sim {
   const ProgramDesc *prog = nullptr;
+  bool clear_flags = false;  // the program's steps write a flag only to set it
   int precision = ABL_PREC_F64;
   std::vector<double> params;
   std::vector<AgentStore> types;
@@ -563,6 +604,12 @@ __global__ void k_bin(const P *__restrict__ px, const P *__restrict__ py, const 
 }
 
 // ---- kernels: run-time removal and birth -----------------------------------------
+
+// Flags of programs that do not clear them themselves (register_program).
+__global__ void k_zero_u8(uint8_t *__restrict__ p, int n) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) p[i] = 0;
+}
 
 static __device__ __forceinline__ void copy_cols(const GatherCols &g, uint32_t src, uint32_t dst) {
   for (int c = 0; c < g.ncols; c++) {
@@ -1042,11 +1089,12 @@ extern "C" int abl_hip_create(const char *program, int precision, abl_sim **out)
   if (precision != ABL_PREC_F64 && precision != ABL_PREC_F32 && precision != ABL_PREC_F32C)
     return fail(ABL_ERR_UNSUPPORTED, "unknown precision");
   const ProgramDesc *prog = find_program(program);
-  if (!prog) return fail(ABL_ERR_ARG, std::string("unknown program ") + program);
+  if (!prog) return fail(ABL_ERR_ARG, no_program(program));
   if (precision == ABL_PREC_F32C && !prog->f32c)
     return fail(ABL_ERR_UNSUPPORTED, std::string(program) + " has no FP32-compensated form");
   abl_sim *sim = new abl_sim();
   sim->prog = prog;
+  sim->clear_flags = !writes_flags(prog);
   sim->precision = precision;
   for (const ParamDesc &p : prog->params) sim->params.push_back(p.value);
   sim->types.resize(prog->agents.size());
@@ -2115,6 +2163,10 @@ static int launch_step(abl_sim *sim, const StepDesc &st, uint32_t ordinal) {
   if (n_step > 0 && (st.removes || st.adds)) {
     L.dead = sim->dead;
     L.born = sim->born;
+    if (sim->clear_flags) {
+      for (uint8_t *flags : {sim->dead, sim->born})
+        hipLaunchKernelGGL(k_zero_u8, grid_blocks(n_step, 256), 256, 0, sim->stream, flags, n_step);
+    }
     if (st.adds) {
       AgentStore &c = sim->types[st.adds - 1];
       for (size_t k = 0; k < c.cols.size(); k++) L.birth.c[k] = c.bmem[k];
@@ -2244,7 +2296,7 @@ extern "C" int abl_hip_estimate_footprint(const char *program, int precision, in
   if (!program || !bytes || num_params < 0 || (num_params && (!param_names || !param_values)))
     return fail(ABL_ERR_ARG, "null argument");
   const ProgramDesc *prog = find_program(program);
-  if (!prog) return fail(ABL_ERR_ARG, std::string("unknown program ") + program);
+  if (!prog) return fail(ABL_ERR_ARG, no_program(program));
   std::vector<double> params;
   for (const ParamDesc &p : prog->params) params.push_back(p.value);
   for (int k = 0; k < num_params; k++) {

@@ -170,7 +170,7 @@ struct StepLaunch {
   // run-time add()/removeCurrent() and random() inside steps
   const int32_t *self_id;  // ids of the stepping agents
   // removeCurrent() and add() flags: a step that removes, or adds, writes 0 or 1
-  // for each of its agents
+  // for each of its agents (or only the ones: register_program)
   uint8_t *dead;
   uint8_t *born;
   ColSet birth;            // newborn columns (the added type), per parent slot
@@ -212,8 +212,9 @@ const ProgramDesc *program_circle3d();
 const ProgramDesc *program_boids2d();
 const ProgramDesc *program_game_of_life();
 const ProgramDesc *program_predator_prey();
-// registered program by name, or nullptr (abl_runtime.hip)
+// registered program by name, or nullptr, and why there is none (abl_runtime.hip)
 const ProgramDesc *find_program(const char *name);
+std::string no_program(const char *name);
 
 inline double param_of(const StepLaunch &L, int idx) { return L.params[idx]; }
 
