@@ -322,6 +322,7 @@ int abl_server_destroy(abl_server *srv);
 /* What the runtime has decided for an agent type so far (it changes nothing and
  * waits for nothing): "lists" (1: its step walks neighbour lists),
  * "lists_given_up" (1: rebuilt too often), "list_capacity" (entries per list),
+ * "tiles" (1: its last step walked the stencil on LDS tiles),
  * "crowded" (1: stepped untiled because too many agents sit in tiles that do
  * not fit LDS), "crowded_agents" (their number when last counted). */
 int abl_hip_inspect(abl_sim *sim, int agent_type, const char *what, double *value);

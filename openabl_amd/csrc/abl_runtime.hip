@@ -253,6 +253,7 @@ struct AgentStore {
   // looked at once per upload, parameter or configuration change
   bool dense = false, dense_known = false;
   uint32_t crowd = 0;  // those agents, as last counted
+  bool on_tiles = false;  // the last step walked the stencil on tiles
   uint64_t nl_t_req = 0, nl_t_prev = 0;
   uint32_t nl_c_prev = 0;
   // run-time add/remove: ids stop being 0..n-1 once agents die or are born
@@ -2112,7 +2113,8 @@ static int launch_step(abl_sim *sim, const StepDesc &st, uint32_t ordinal) {
     // crowded tiles: one thread per agent instead (unless lists are asked for)
     if ((st.nlist || st.tiles) && st.near_agent == st.agent && sim->order == 0 &&
         sim->tile != 0 && !(sim->nlist_set && sim->nlist)) {
-      if (!b.dense_known && !(want_list && reach_for(b, rl) <= 4) && L.grid.reach <= 4) {
+      if (!b.dense_known && !(want_list && reach_for(b, rl) <= 4) && L.grid.reach <= 4 &&
+          (!st.walks_tiles || st.walks_tiles(L))) {
         b.dense = false;
         b.dense_known = b.n < kProbeAgents;
         if (!b.dense_known) {
@@ -2174,11 +2176,14 @@ static int launch_step(abl_sim *sim, const StepDesc &st, uint32_t ordinal) {
   }
   if (L.n > 0) {
     int sp = span_open(sim, 1);
+    a.on_tiles = (st.nlist || st.tiles) && L.nl_mode == 0 && L.tile != 0 && L.order == 0 &&
+                 L.grid.reach <= 4 && (!st.walks_tiles || st.walks_tiles(L));
     st.launch(L);
     if (probed) {
       int rc = read_crowd(sim, *probed);
       if (rc) return rc;
       if (probed->dense) {
+        a.on_tiles = false;
         L.tile = 0;
         L.nl = nullptr;
         st.launch(L);
@@ -2375,6 +2380,7 @@ extern "C" int abl_hip_inspect(abl_sim *sim, int t, const char *what, double *va
   if (k == "lists") *value = s.nl_ok;
   else if (k == "lists_given_up") *value = s.nl_off;
   else if (k == "list_capacity") *value = s.nl_cap;
+  else if (k == "tiles") *value = s.on_tiles;
   else if (k == "crowded") *value = s.dense_known && s.dense;
   else if (k == "crowded_agents") *value = s.crowd;
   else return fail(ABL_ERR_ARG, "unknown quantity " + k);

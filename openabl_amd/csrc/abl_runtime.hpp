@@ -97,6 +97,9 @@ struct StepDesc {
   // the near loop visits its own type, whose positions no step writes: the
   // launcher keeps each agent's neighbours between two sorts (StepLaunch::fixed)
   bool fixed;
+  // whether the launcher walks this stencil on the tiles (nl_mode 0); null: yes,
+  // wherever it tiles at all
+  bool (*walks_tiles)(const StepLaunch &);
 };
 
 struct ProgramDesc {
@@ -161,7 +164,8 @@ struct StepLaunch {
   float lds_slack;     // LDS records per expected halo agent
   // neighbour lists: 0 = stencil walk, 1 = build the lists, 2 = step through
   // them, 3 = gated re-sort and build in one launch (delta, abl_pipeline.hpp),
-  // 4 = count the agents of tiles whose halo does not fit LDS into nl->stats[1]
+  // 4 = count the agents of tiles whose halo does not fit LDS (nl->publish, or
+  // nl->stats[1])
   int nl_mode;
   const NListArgs *nl;
   const DeltaArgs *delta;

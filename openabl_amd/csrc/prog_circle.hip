@@ -43,7 +43,8 @@ const ProgramDesc *program_circle() {
       {{"Point", {{"pos", K_FLOAT2, true}}}},
       {{"num_timesteps", 100}, {"num_agents", 1000}, {"rho", 0.05}, {"k_rep", 0.05},
        {"k_att", 0.01}, {"r", 5.0}, {"W", 141.421}},
-      {{"move_point", 0, 0, "r", 2.0, 0x3u, launch_move_point<2>, false, 0, true}},
+      {{"move_point", 0, 0, "r", 2.0, 0x3u, launch_move_point<2>, false, 0, true, nullptr,
+        false, false, walks_tiles}},
       env2,
       host_init2,
       nullptr,

@@ -87,7 +87,8 @@ const ProgramDesc *program_circle3d() {
       {{"num_timesteps", 100}, {"num_agents", 1000}, {"rho", 0.05}, {"k_rep", 0.05},
        {"k_att", 0.01}, {"r", 5.0}, {"W", 27.1442}, {"num_clusters", 64},
        {"cluster_sigma", 20.0}, {"background_fraction", 0.2}},
-      {{"move_point", 0, 0, "r", 2.0, 0x7u, launch_move_point<3>, false, 0, true}},
+      {{"move_point", 0, 0, "r", 2.0, 0x7u, launch_move_point<3>, false, 0, true, nullptr,
+        false, false, walks_tiles}},
       env3,
       host_init3,
       nullptr,

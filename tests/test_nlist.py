@@ -28,7 +28,7 @@ from orclib import Oracle, boids2d_params, circle3d_params, circle_params, field
 pytestmark = pytest.mark.gpu
 
 
-def run(model, prec, params, steps, **cfg):
+def run(model, prec, params, steps, crowded=None, **cfg):
     from openabl_amd import MEMBERS, Simulation, load_library, record_dtype
     load_library().abl_rng_seed(0xDEADBEEF, 0xBEEFDEAD)
     sim = Simulation(model, prec, params=params, config=cfg)
@@ -39,6 +39,8 @@ def run(model, prec, params, steps, **cfg):
         sim.simulate(upto - done)
         done = upto
         out.append(sim.download(record_dtype(MEMBERS[model], prec)))
+        if crowded is not None:
+            assert sim.inspect("crowded") == crowded
     sim.close()
     return out
 
@@ -252,8 +254,9 @@ def test_crowded_tiles_equal_untiled(model, prec, params, cfg, cells):
     first timestep on: the bits of hip.tile=0 on the same cells."""
     print(f"case nlist crowded tiles {model} {prec} {cfg}", flush=True)
     steps = (1, 4)
-    a = run(model, prec, params, steps, **cfg)
-    b = run(model, prec, params, steps, **dict(cfg, **{"hip.tile": 0, "hip.cell_inflate": cells}))
+    a = run(model, prec, params, steps, crowded=params["num_agents"] >= 8192, **cfg)
+    b = run(model, prec, params, steps, crowded=False,
+            **dict(cfg, **{"hip.tile": 0, "hip.cell_inflate": cells}))
     for t, x, y in zip(steps, a, b):
         assert field_bytes(x) == field_bytes(y), t
 
@@ -323,3 +326,24 @@ def test_crowded_agents_are_counted_exactly(prec, cfg):
             assert sim.inspect("crowded") == (want > 0)
             assert sim.inspect("lists") == (want == 0 and not cfg)
         sim.close()
+
+
+@pytest.mark.parametrize("prec", ["f64", "f32", "f32c"])
+def test_crowd_is_counted_only_for_steps_on_tiles(prec):
+    """circle3d walks its stencil untiled (but in FP32-compensated): then there is nothing to count, and crowded or not, each
+    timestep is one launch.  The same bits either way in FP64 and FP32."""
+    from openabl_amd import MEMBERS, Simulation, load_library, record_dtype
+    print(f"case nlist crowd count {prec} circle3d", flush=True)
+    params = circle3d_params(num_agents=20011, rho=20011 / 1e9, r=4.0, num_clusters=4, cluster_sigma=12.0)
+    outs = []
+    for cfg in ({}, {"hip.tile": 1}, {"hip.tile": 0, "hip.cell_inflate": 1}):
+        load_library().abl_rng_seed(0xDEADBEEF, 0xBEEFDEAD)
+        sim = Simulation("circle3d", prec, params=params, config=dict(cfg, **{"hip.nlist": 0}))
+        sim.init_agents()
+        sim.simulate(3)
+        counted = prec == "f32c" and cfg.get("hip.tile", 1) == 1
+        assert (sim.inspect("crowded_agents") > 20011 / 4) == counted, cfg
+        assert sim.inspect("crowded") == counted and sim.inspect("tiles") == 0
+        outs.append(field_bytes(sim.download(record_dtype(MEMBERS["circle3d"], prec))))
+        sim.close()
+    assert outs[0] == outs[1] == outs[2]
