@@ -131,7 +131,12 @@ int abl_hip_get_param(abl_sim *sim, const char *name, double *value);
 /* `-C key=value` runtime options: "hip.block" (threads per block),
  * "hip.cell_scale" (cells per granularity, 1..4), "hip.order" ("cell" or
  * "index": visit neighbours in cell order or in the reference's index
- * order), "hip.tile" (LDS tile shape, 0 = untiled), "hip.lds_slack" (LDS
+ * order), "hip.tile" (LDS tile shape of steps that run on tiles: 0 = one thread
+ * per agent; in 2-D 1 = sized by the agents per cell, 2 = 8 x 8 and 3 = 32 x 8
+ * cells; 1 by default, except that circle and circle3d then walk their stencil
+ * untiled, and that a type most of whose agents crowd into tiles that do not fit
+ * LDS is stepped untiled, see abl_hip_inspect; game_of_life keeps its neighbours
+ * instead, whatever shape is named), "hip.lds_slack" (LDS
  * records per tile as a multiple of the expected halo), "hip.grid" ("delta"
  * or "full" re-sort), "hip.nlist" (1: neighbour lists with a skin for tiled
  * near loops over the agent's own type, 0: walk the stencil every step;

@@ -5,7 +5,8 @@ candidate runtime configuration -- threads per block ("hip.block"), cells per
 granularity ("hip.cell_scale", i.e. cell edge = granularity / scale with a
 (2*scale+1)^d stencil), LDS tile shape ("hip.tile", 0 = untiled) and LDS
 budget ("hip.lds_slack") -- on a private copy of the state, and returns the
-fastest.  Every candidate computes the same neighbour sets (the near test is
+fastest.  (A tile shape that is named is used for the stencil walk too where the
+default is to walk untiled; 3-D models have one shape, and game_of_life none.)  Every candidate computes the same neighbour sets (the near test is
 exact whatever the cell size), and tile shape and LDS budget do not change
 results at all, so tuning never changes results beyond the summation order
 of the default cell-ordered visit (which depends on the cell size).

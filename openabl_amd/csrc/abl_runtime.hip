@@ -280,6 +280,7 @@ struct abl_sim {
   int cell_scale = 1;
   int order = 0;
   int tile = 1;
+  bool tile_set = false;   // "hip.tile" given
   bool grid_delta = true;  // "hip.grid": delta re-sort when the stored order allows it
   float lds_slack = 2.0f;  // "hip.lds_slack": LDS tile records per expected halo agent
   bool nlist = true;       // "hip.nlist": neighbour lists for steps that support them
@@ -1204,6 +1205,7 @@ extern "C" int abl_hip_set_config(abl_sim *sim, const char *key, const char *val
     int t = std::atoi(value);
     if (t < 0 || t > 3) return fail(ABL_ERR_ARG, "hip.tile must be 0..3");
     sim->tile = t;
+    sim->tile_set = true;
   } else if (k == "hip.nlist") {
     if (v == "1" || v == "true") sim->nlist = true;
     else if (v == "0" || v == "false") sim->nlist = false;
@@ -2105,6 +2107,7 @@ static int launch_step(abl_sim *sim, const StepDesc &st, uint32_t ordinal) {
     L.grid.reach = reach_for(b, r);
     L.near_t = sqrtf_le_threshold(r);
     L.tile = sim->tile;
+    L.tile_given = sim->tile_set;
     L.lds_slack = sim->lds_slack;
     L.occupancy = b.ncells ? (float) ((double) b.n / (double) b.ncells) : 0.f;
     L.rc = (float) (r / b.cell * (1.0 + 1.0 / 1048576.0));

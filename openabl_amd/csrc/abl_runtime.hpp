@@ -160,6 +160,7 @@ struct StepLaunch {
   int block;           // threads per block
   int order;           // 0 = cell order, 1 = reference index order
   int tile;            // LDS tile variant (0: untiled thread-per-agent kernel)
+  bool tile_given;     // asked for by the caller, not the default
   float occupancy;     // near-type agents per cell (sizes the LDS tile budget)
   float lds_slack;     // LDS records per expected halo agent
   // neighbour lists: 0 = stencil walk, 1 = build the lists, 2 = step through

@@ -375,12 +375,13 @@ void launch_c(const StepLaunch &L) {
 // candidate hides its reads, and it has as many blocks as the agents fill.  FP64,
 // circle with 1,000 / 64,000 / 1,000,003 agents 25.6 / 37.7 / 114 us per timestep
 // (tiles 50 / 74 / 142), circle3d with 2,000 / 200,003 agents 337 / 593 us (tiles
-// 1,654 / 605); FP32 alike.  (Its buffer offsets end at 2^31 bytes.)  Not for FP32-compensated, whose tiles round
+// 1,654 / 605); FP32 alike.  (Its buffer offsets end at 2^31 bytes.)  A caller that
+// asks for a tile shape gets it.  Not for FP32-compensated, whose tiles round
 // offsets from the tile's own origin: lists and stencil would no longer agree to
 // the bit.
 inline bool on_tiles(const StepLaunch &L, size_t elem) {
   return L.tile != 0 && L.grid.reach <= 4 &&
-         (L.nl_mode != 0 || (size_t) L.n * elem >= ((size_t) 1 << 31));
+         (L.nl_mode != 0 || L.tile_given || (size_t) L.n * elem >= ((size_t) 1 << 31));
 }
 
 // StepDesc::walks_tiles

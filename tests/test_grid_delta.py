@@ -10,7 +10,7 @@ from orclib import boids2d_params, circle3d_params, circle_params, field_bytes
 pytestmark = pytest.mark.gpu
 
 
-def run(model, prec, params, steps, grid, **cfg):
+def run(model, prec, params, steps, grid, tiles=None, **cfg):
     from openabl_amd import MEMBERS, Simulation, load_library, record_dtype
     load_library().abl_rng_seed(0xDEADBEEF, 0xBEEFDEAD)
     sim = Simulation(model, prec, params=params, config=dict(cfg, **{"hip.grid": grid}))
@@ -21,6 +21,8 @@ def run(model, prec, params, steps, grid, **cfg):
         sim.simulate(upto - done)
         done = upto
         out.append((sim.download(record_dtype(MEMBERS[model], prec)), sim.neighbours(0)))
+        if tiles is not None:  # the walk that the case is about
+            assert sim.inspect("tiles") == tiles
     sim.close()
     return out
 
@@ -77,11 +79,13 @@ def test_delta_after_upload_and_param_change():
     assert field_bytes(outs[0]) == field_bytes(outs[1])
 
 
+# below the population from which a type is stepped untiled for its tiles beyond
+# LDS, which the smaller budget and the clusters make
 TILE_CASES = [
-    ("boids2d", boids2d_params(num_agents=20000), 1),
-    ("boids2d", boids2d_params(num_agents=20000), 2),
+    ("boids2d", boids2d_params(num_agents=8191), 1),
+    ("boids2d", boids2d_params(num_agents=8191), 2),
     ("circle", circle_params(num_agents=4096), 1),
-    ("circle3d", circle3d_params(num_agents=32768, rho=32768 / 1e9, r=4.0, num_clusters=2,
+    ("circle3d", circle3d_params(num_agents=8191, rho=8191 / 1e9, r=4.0, num_clusters=2,
                                  cluster_sigma=20.0), 1),
 ]
 
@@ -95,10 +99,11 @@ def test_tiled_kernels_equal_untiled(model, params, cs, prec):
     row of the stencil, cell-sorted order inside a row; narrowing only skips
     cells that cannot hold a neighbour), so runs are bit-identical."""
     print(f"case tiles {model} {prec} cs={cs}", flush=True)
-    ref = run(model, prec, params, (1, 5), "delta", **{"hip.tile": 0, "hip.cell_scale": cs})
+    ref = run(model, prec, params, (1, 5), "delta", tiles=0,
+              **{"hip.tile": 0, "hip.cell_scale": cs, "hip.nlist": 0})
     for tile in (1, 2, 3):
         for slack in (2.0, 1.0):
-            got = run(model, prec, params, (1, 5), "delta",
+            got = run(model, prec, params, (1, 5), "delta", tiles=1,
                       **{"hip.tile": tile, "hip.cell_scale": cs, "hip.lds_slack": slack,
                          "hip.nlist": 0})
             for (x, _), (y, _) in zip(got, ref):

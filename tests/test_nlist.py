@@ -330,7 +330,8 @@ def test_crowded_agents_are_counted_exactly(prec, cfg):
 
 @pytest.mark.parametrize("prec", ["f64", "f32", "f32c"])
 def test_crowd_is_counted_only_for_steps_on_tiles(prec):
-    """circle3d walks its stencil untiled (but in FP32-compensated): then there is nothing to count, and crowded or not, each
+    """circle3d walks its stencil untiled unless a tile shape is named (or in
+    FP32-compensated): then there is nothing to count, and crowded or not, each
     timestep is one launch.  The same bits either way in FP64 and FP32."""
     from openabl_amd import MEMBERS, Simulation, load_library, record_dtype
     print(f"case nlist crowd count {prec} circle3d", flush=True)
@@ -341,7 +342,7 @@ def test_crowd_is_counted_only_for_steps_on_tiles(prec):
         sim = Simulation("circle3d", prec, params=params, config=dict(cfg, **{"hip.nlist": 0}))
         sim.init_agents()
         sim.simulate(3)
-        counted = prec == "f32c" and cfg.get("hip.tile", 1) == 1
+        counted = cfg.get("hip.tile", 1 if prec == "f32c" else 0) == 1
         assert (sim.inspect("crowded_agents") > 20011 / 4) == counted, cfg
         assert sim.inspect("crowded") == counted and sim.inspect("tiles") == 0
         outs.append(field_bytes(sim.download(record_dtype(MEMBERS["circle3d"], prec))))
