@@ -259,11 +259,11 @@ int abl_hip_log_text(abl_sim *sim, char *buf, size_t capacity, size_t *len);
  * timestep is replayed as a captured HIP graph ("hip.graph", default on).
  * Member m's initialisation starts from abl_ens_member_seed(s0, s1, m); each
  * member's result is bit-identical to a run of it alone from that state with
- * the same "hip.cell_scale", "hip.tile", "hip.nlist", "hip.skin" and
- * "hip.list_cap".  Neighbour lists ("hip.nlist", default 1, when every member
+ * the same "hip.cell_scale", "hip.tile", "hip.nlist" (given, not left at its
+ * default), "hip.skin" and "hip.list_cap".  Neighbour lists ("hip.nlist", default 1, when every member
  * has the same near radius): one set over all members' agents, and a rebuild
- * gate per member, so a member re-sorts and rebuilds its lists on exactly the
- * timesteps a run of it alone does.  Programs: boids2d. */
+ * gate and list capacity per member, so a member re-sorts, rebuilds and grows its
+ * lists on exactly the timesteps a run of it alone does.  Programs: boids2d. */
 typedef struct abl_ensemble abl_ensemble;
 const char *abl_ens_last_error(void);
 int abl_ens_member_seed(uint64_t s0, uint64_t s1, int member, uint64_t out[2]);
@@ -277,6 +277,11 @@ int abl_ens_simulate(abl_ensemble *ens, int timesteps);
 int abl_ens_synchronize(abl_ensemble *ens, double *ms);
 int abl_ens_member_count(abl_ensemble *ens, int member, size_t *count);
 int abl_ens_agents(abl_ensemble *ens, size_t *total);
+/* What the ensemble has decided so far, for a member: "lists" (1: its step walks
+ * neighbour lists), "list_capacity" (entries per list); for all: "rebuild_launches"
+ * (1, or 4 where many timesteps rebuild), "rebuilds" (timesteps on which some
+ * member rebuilt, as last looked at). */
+int abl_ens_inspect(abl_ensemble *ens, int member, const char *what, double *value);
 int abl_ens_download(abl_ensemble *ens, int member, void *aos, size_t capacity, size_t *count);
 int abl_ens_destroy(abl_ensemble *ens);
 

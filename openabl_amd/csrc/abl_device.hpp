@@ -165,6 +165,8 @@ struct EnsTiles {
   const uint32_t *cell_base;  // [members + 1] first cells
   const GridView *grids;      // [members]
   uint32_t *mgate;            // [2][members] rebuild flags by timestep parity (lists)
+  const uint32_t *mcap;       // [members] list entries per agent, at most NListArgs::cap
+  uint32_t *mlong;            // [members] longest list beyond that since the lists were entered
   int members;
   unsigned total;             // tiles
 };

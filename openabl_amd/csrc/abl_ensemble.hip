@@ -66,6 +66,9 @@ struct Member {
   uint32_t cell_base = 0, tile_base = 0, ntiles = 0;
   double cell = 0.0;
   float near_t = 0.f, rc = 0.f;
+  // lists: estimated entries per agent, the capacity, and when to look at them
+  int est = 0, cap = 0;
+  ListWatch watch;
 };
 
 // Every slot's cell key.
@@ -147,31 +150,40 @@ struct abl_ensemble {
   int list_cap = 0;            // "hip.list_cap": entries per list (0: sized from the data)
   bool lists = false;          // in use (decided by abl_ens_init)
   double r = 0.0, rl = 0.0, cell = 0.0;
-  int nl_cap = 0;
+  int nl_cap = 0;              // entries per agent allocated: the largest member's capacity
   uint16_t *nl_idx = nullptr, *nl_len = nullptr;
   uint32_t *nl_perm = nullptr;
   uint4 *nl_prow0 = nullptr;
   double *nl_pos0 = nullptr;
-  uint32_t *nl_gate = nullptr;   // [0..1] some member due, by parity; [2] longest list;
-                                 // error flag, generation and queues (abl_pipeline.hpp)
+  uint32_t *nl_gate = nullptr;   // [0..1] some member due, by parity; error flag, generation
+                                 // and queues (abl_pipeline.hpp)
   uint32_t *nl_mgate = nullptr;  // [2][members] member due, by parity
+  uint32_t *nl_mcap = nullptr;   // [members] capacities; [members] lists to be entered anew
+  uint32_t *nl_mlong = nullptr;  // [members] EnsTiles::mlong
   uint32_t *skey[2] = {nullptr, nullptr};  // each slot's cell key at the last sort; the rebuild's
   uint32_t *start_new = nullptr;           // the rebuild's cell offsets
   uint32_t *dirty = nullptr;               // MoverLists
   unsigned long long *mhead = nullptr, *mnext = nullptr;
-  uint32_t *h_error = nullptr;   // pinned copy of the error flag and the generation, as of the
-                                 // last simulate()
-  // four launches per rebuild instead of one: most timesteps since the last look rebuilt
+  uint32_t *h_error = nullptr;   // pinned copy of the error flag as of the last simulate()
+  // what look() asked for: pinned copies of the generation and of nl_mlong after a
+  // timestep, in the slot of that timestep (answers are read kListSample later)
+  static constexpr uint64_t kSlots = 2 * kListSample;
+  uint32_t *h_look = nullptr;    // [kSlots][1 + members]
+  hipEvent_t look_ev[kSlots] = {};
+  uint64_t next_look = 0;        // the timestep after which look() has something to do
+  ListWatch watch;               // the ensemble's own: the number of rebuilds
+  std::vector<int> entering;     // members whose lists are entered anew at the next timestep
+  // four launches per rebuild instead of one: many timesteps rebuild
   bool split = false;
   uint32_t gen_seen = 1;
-  uint64_t step_seen = 0;
   // download workspace: one member's records, grown to the largest asked for
   std::mutex dl_lock;
   void *dl = nullptr;
   size_t dl_bytes = 0;
   hipStream_t stream = nullptr;
-  hipGraphExec_t exec = nullptr;
-  hipGraph_t graph = nullptr;
+  // two timesteps, captured with one launch per rebuild and with four
+  hipGraphExec_t exec[2] = {nullptr, nullptr};
+  hipGraph_t graph[2] = {nullptr, nullptr};
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   double last_ms = 0.0;
 };
@@ -266,6 +278,15 @@ extern "C" int abl_ens_set_config(abl_ensemble *e, const char *key, const char *
   return ABL_OK;
 }
 
+static void drop_graphs(abl_ensemble *e) {
+  for (int k = 0; k < 2; k++) {
+    if (e->exec[k]) (void) hipGraphExecDestroy(e->exec[k]);
+    if (e->graph[k]) (void) hipGraphDestroy(e->graph[k]);
+    e->exec[k] = nullptr;
+    e->graph[k] = nullptr;
+  }
+}
+
 static void free_all(abl_ensemble *e) {
   for (int b = 0; b < 2; b++) {
     for (int c = 0; c < kMaxCols; c++) {
@@ -299,6 +320,8 @@ static void free_all(abl_ensemble *e) {
   drop(e->nl_pos0);
   drop(e->nl_gate);
   drop(e->nl_mgate);
+  drop(e->nl_mcap);
+  drop(e->nl_mlong);
   drop(e->skey[0]);
   drop(e->skey[1]);
   drop(e->start_new);
@@ -308,11 +331,13 @@ static void free_all(abl_ensemble *e) {
   drop(e->dl);
   e->dl_bytes = 0;
   if (e->h_error) (void) hipHostFree(e->h_error);
-  e->h_error = nullptr;
-  if (e->exec) (void) hipGraphExecDestroy(e->exec);
-  if (e->graph) (void) hipGraphDestroy(e->graph);
-  e->exec = nullptr;
-  e->graph = nullptr;
+  if (e->h_look) (void) hipHostFree(e->h_look);
+  e->h_error = e->h_look = nullptr;
+  for (hipEvent_t &ev : e->look_ev) {
+    if (ev) (void) hipEventDestroy(ev);
+    ev = nullptr;
+  }
+  drop_graphs(e);
 }
 
 // The list arguments of the current timestep (as a run alone forms them).
@@ -345,6 +370,8 @@ static EnsTiles ens_tiles(const abl_ensemble *e) {
   t.cell_base = e->d_cell_base;
   t.grids = e->d_grids;
   t.mgate = e->nl_mgate;
+  t.mcap = e->nl_mcap;
+  t.mlong = e->nl_mlong;
   t.members = (int) e->mem.size();
   t.total = e->total_tiles;
   return t;
@@ -406,8 +433,17 @@ static NListArgs ens_build_args(const abl_ensemble *e) {
   return nl;
 }
 
+// The gated list build of the members due, their agents sorted already.
+static int issue_build(abl_ensemble *e) {
+  NListArgs nl = ens_build_args(e);
+  nl.gated = 1;
+  const int rc = e->hooks->launch_multi_list(e->precision, e->d_build[e->cur], ens_tiles(e), e->reach,
+                                             e->occupancy, e->tile, e->block, e->stream, nl, nullptr, 1);
+  return rc ? ens_fail(rc, "list build") : ABL_OK;
+}
+
 // The gated rebuild of the current timestep: one launch (tiled_rebuild_multi), or
-// four (ens_check), which cost a timestep without a rebuild about 10 us more and one
+// four (look), which cost a timestep without a rebuild about 10 us more and one
 // with a rebuild 50 us less; the same results.
 static int issue_rebuild(abl_ensemble *e) {
   DeltaArgs d{};
@@ -443,71 +479,162 @@ static int issue_rebuild(abl_ensemble *e) {
     hipLaunchKernelGGL(k_scan_apply, d.nscan, kScanBlock, 0, e->stream, e->count, e->bsum,
                        e->start_new, d.ncells, nl.gate + nl.parity);
     hipLaunchKernelGGL(delta, grid_blocks(d.n, 256), 256, 0, e->stream, d, t, nl.gate, nl.parity, 2);
+    return issue_build(e);
   }
-  const int rc = e->hooks->launch_multi_list(e->precision, e->d_build[b], t, e->reach,
-                                             e->occupancy, e->tile, e->block, e->stream, nl,
-                                             e->split ? nullptr : &d, e->split ? 1 : 3);
+  const int rc = e->hooks->launch_multi_list(e->precision, e->d_build[b], t, e->reach, e->occupancy,
+                                             e->tile, e->block, e->stream, nl, &d, 3);
   return rc ? ens_fail(rc, "list rebuild: no launch size") : ABL_OK;
 }
 
-// List buffers, and every member's first sort and lists (as a run alone
-// enters list mode: capacity "hip.list_cap", or from the expected population
-// of the list radius, grown once to the longest list, at most four times the
-// estimate).
+// Entry lists for the largest capacity; those of members that keep theirs stay
+// (rows of eight entries of all agents, so more rows go behind).  The captured
+// timesteps hold the address.
+static int reserve_entries(abl_ensemble *e) {
+  int cap = 0;
+  for (const Member &mb : e->mem) cap = std::max(cap, mb.cap);
+  if (cap <= e->nl_cap) return ABL_OK;
+  uint16_t *idx = nullptr;
+  ENS_TRY(hipMalloc(&idx, (size_t) cap * e->n * 2));
+  if (e->nl_idx) {
+    hipError_t err = hipMemcpyAsync(idx, e->nl_idx, (size_t) e->nl_cap * e->n * 2,
+                                    hipMemcpyDeviceToDevice, e->stream);
+    if (err == hipSuccess) err = hipStreamSynchronize(e->stream);
+    if (err != hipSuccess) {
+      (void) hipFree(idx);
+      ENS_TRY(err);
+    }
+    ENS_TRY(hipFree(e->nl_idx));
+  }
+  e->nl_idx = idx;
+  e->nl_cap = cap;
+  drop_graphs(e);
+  return ABL_OK;
+}
+
+// The capacities, and which members enter their lists anew, to the device.
+static int put_capacities(abl_ensemble *e) {
+  const size_t M = e->mem.size();
+  std::vector<uint32_t> words(2 * M, 0u);
+  for (size_t m = 0; m < M; m++) words[m] = (uint32_t) e->mem[m].cap;
+  for (const int m : e->entering) words[M + (size_t) m] = 1u;
+  ENS_TRY(hipMemcpyAsync(e->nl_mcap, words.data(), 2 * M * 4, hipMemcpyHostToDevice, e->stream));
+  ENS_TRY(hipStreamSynchronize(e->stream));
+  return ABL_OK;
+}
+
+// More room for the lists of member m, as a run alone makes it (enter_lists);
+// whether there is any.
+static bool grow_lists(const abl_ensemble *e, Member &mb, uint32_t longest) {
+  const int room = list_room(mb.est, longest);
+  if (e->list_cap || (int64_t) longest <= mb.cap || room <= mb.cap || mb.cap >= kListMost) return false;
+  mb.cap = list_capacity(room);
+  return true;
+}
+
+// Sets the members entering their lists due, nothing counted of them yet.
+__global__ void k_ens_enter(const uint32_t *__restrict__ enter, int members, int parity,
+                            uint32_t *__restrict__ gate, uint32_t *__restrict__ mgate,
+                            uint32_t *__restrict__ mlong) {
+  const int m = blockIdx.x * blockDim.x + threadIdx.x;
+  if (m >= members || !enter[m]) return;
+  gate[parity] = 1u;
+  mgate[parity * members + m] = 1u;
+  mlong[m] = 0u;
+}
+
+// The rebuild of the current timestep where some members enter their lists anew
+// (look): those are due whatever their agents did, get the capacity that look()
+// gave them, and once more room if their lists have outgrown that meanwhile.  A
+// run alone enters list mode like that, so its lists, and the order it adds its
+// neighbours in, stay the member's.
+static int enter_members(abl_ensemble *e) {
+  const int M = (int) e->mem.size();
+  int rc = reserve_entries(e);
+  if (!rc) rc = put_capacities(e);
+  if (rc) return rc;
+  const int parity = (int) (e->timestep & 1u);
+  hipLaunchKernelGGL(k_ens_enter, grid_blocks(M, 256), 256, 0, e->stream, e->nl_mcap + M, M, parity,
+                     e->nl_gate, e->nl_mgate, e->nl_mlong);
+  rc = issue_rebuild(e);
+  if (rc) return rc;
+  std::vector<uint32_t> longest((size_t) M);
+  ENS_TRY(hipMemcpyAsync(longest.data(), e->nl_mlong, (size_t) M * 4, hipMemcpyDeviceToHost, e->stream));
+  ENS_TRY(hipStreamSynchronize(e->stream));
+  bool again = false;
+  for (const int m : e->entering) {
+    Member &mb = e->mem[(size_t) m];
+    again = grow_lists(e, mb, longest[(size_t) m]) || again;
+    mb.watch.entered(e->timestep);
+    e->next_look = std::min(e->next_look, mb.watch.next());
+  }
+  if (again) {
+    rc = reserve_entries(e);
+    if (!rc) rc = put_capacities(e);
+    if (!rc) rc = issue_build(e);
+  }
+  e->entering.clear();
+  return rc;
+}
+
+// List buffers, and every member's first sort and lists, as a run alone enters
+// list mode: capacity "hip.list_cap", or from the expected population of the
+// list radius, grown once to the longest list.
 static int init_lists(abl_ensemble *e) {
   const size_t N = e->n;
   const size_t M = e->mem.size();
-  int want = 16;
-  for (const Member &mb : e->mem) {
-    const double env = (double) mb.g.n[0] * (double) mb.g.n[1] * mb.cell * mb.cell;
-    const double expect = env > 0 ? M_PI * e->rl * e->rl * (double) mb.n / env : 0.0;
-    want = std::max(want, (int) (1.5 * expect) + 16);
+  for (Member &mb : e->mem) {
+    mb.est = list_estimate(2, (size_t) mb.g.n[0] * (size_t) mb.g.n[1], mb.cell, (size_t) mb.n, e->rl);
+    mb.cap = list_capacity(e->list_cap ? e->list_cap : mb.est);
+    mb.watch.entered(0);
   }
-  if (e->list_cap) want = e->list_cap;
-  int cap = std::min((want + 7) & ~7, 65528);
+  e->watch.entered(0);
+  e->next_look = e->watch.next();
+  e->entering.clear();
+  e->nl_cap = 0;
   ENS_TRY(hipMalloc(&e->nl_len, N * 2));
   ENS_TRY(hipMalloc(&e->nl_perm, N * 4));
   ENS_TRY(hipMalloc(&e->nl_prow0, N * 16));
   ENS_TRY(hipMalloc(&e->nl_pos0, 2 * N * 8));
   ENS_TRY(hipMalloc(&e->nl_gate, kGateWords * 4));
   ENS_TRY(hipMalloc(&e->nl_mgate, 2 * M * 4));
+  ENS_TRY(hipMalloc(&e->nl_mcap, 2 * M * 4));
+  ENS_TRY(hipMalloc(&e->nl_mlong, M * 4));
   for (uint32_t *&k : e->skey) ENS_TRY(hipMalloc(&k, N * 4));
   ENS_TRY(hipMalloc(&e->dirty, e->ncells * 4));
   ENS_TRY(hipMalloc(&e->mhead, e->ncells * 8));
   ENS_TRY(hipMalloc(&e->mnext, N * 8));
   ENS_TRY(hipMemsetAsync(e->dirty, 0, e->ncells * 4, e->stream));
   ENS_TRY(hipMemsetAsync(e->mhead, 0, e->ncells * 8, e->stream));
-  ENS_TRY(hipHostMalloc((void **) &e->h_error, 8, hipHostMallocDefault));
-  e->h_error[0] = 0u;
-  e->h_error[1] = e->gen_seen = 1u;
-  e->step_seen = 0;
+  ENS_TRY(hipHostMalloc((void **) &e->h_error, 4, hipHostMallocDefault));
+  ENS_TRY(hipHostMalloc((void **) &e->h_look, e->kSlots * (1 + M) * 4, hipHostMallocDefault));
+  for (hipEvent_t &ev : e->look_ev) ENS_TRY(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+  *e->h_error = 0u;
+  e->gen_seen = 1u;
   e->split = false;
   // The lists below are those of the initial state: no member is due at the
   // first timestep (an overflowed list sets its member's gate at that step).
-  std::vector<uint32_t> words(kGateWords, 0u), none(2 * M, 0u);
+  std::vector<uint32_t> words(kGateWords, 0u), longest(M), none(2 * M, 0u);
   words[kGateGen] = 1u;
   ENS_TRY(hipMemcpy(e->nl_mgate, none.data(), 2 * M * 4, hipMemcpyHostToDevice));
+  ENS_TRY(hipMemcpy(e->nl_mlong, none.data(), M * 4, hipMemcpyHostToDevice));
+  ENS_TRY(hipMemcpy(e->nl_gate, words.data(), kGateWords * 4, hipMemcpyHostToDevice));
   const int ntiles = ((int) e->ncells + kScanTile - 1) / kScanTile;
-  for (int attempt = 0;; attempt++) {
-    if (e->nl_idx) ENS_TRY(hipFree(e->nl_idx));
-    e->nl_idx = nullptr;
-    ENS_TRY(hipMalloc(&e->nl_idx, (size_t) cap * N * 2));
-    e->nl_cap = cap;
-    ENS_TRY(hipMemcpy(e->nl_gate, words.data(), kGateWords * 4, hipMemcpyHostToDevice));
-    ENS_TRY(hipMemsetAsync(e->count, 0, (e->ncells + 1) * 4, e->stream));
-    issue_sort(e, e->start_new, e->skey[1], e->count);
-    hipLaunchKernelGGL(k_tile_totals, ntiles, kScanBlock, 0, e->stream, e->count, e->bsum,
-                       (int) e->ncells);
+  ENS_TRY(hipMemsetAsync(e->count, 0, (e->ncells + 1) * 4, e->stream));
+  issue_sort(e, e->start_new, e->skey[1], e->count);
+  hipLaunchKernelGGL(k_tile_totals, ntiles, kScanBlock, 0, e->stream, e->count, e->bsum,
+                     (int) e->ncells);
+  for (bool again = true; again;) {
+    int rc = reserve_entries(e);
+    if (!rc) rc = put_capacities(e);
+    if (rc) return rc;
     e->hooks->launch_multi_list(e->precision, e->d_build[e->cur], ens_tiles(e), e->reach,
                                 e->occupancy, e->tile, e->block, e->stream, ens_build_args(e),
                                 nullptr, 1);
     ENS_TRY(hipGetLastError());
     ENS_TRY(hipStreamSynchronize(e->stream));
-    uint32_t longest = 0;
-    ENS_TRY(hipMemcpy(&longest, e->nl_gate + 2, 4, hipMemcpyDeviceToHost));
-    const int grow = std::min((int) (1.25 * longest) + 16, 4 * want);
-    if (attempt > 0 || (int) longest <= cap || grow <= cap || cap >= 65528 || e->list_cap) break;
-    cap = std::min((grow + 7) & ~7, 65528);
+    ENS_TRY(hipMemcpy(longest.data(), e->nl_mlong, M * 4, hipMemcpyDeviceToHost));
+    again = false;
+    for (size_t m = 0; m < M; m++) again = grow_lists(e, e->mem[m], longest[m]) || again;
   }
   return ABL_OK;
 }
@@ -700,7 +827,7 @@ static int issue_step(abl_ensemble *e) {
   const int b = e->cur;
   if (e->lists) {
     if (n > 0) {
-      const int rc = issue_rebuild(e);
+      const int rc = e->entering.empty() ? issue_rebuild(e) : enter_members(e);
       if (rc) return rc;
       // the step reads buffer b: the arguments whose input is 1 - (1 - b)
       e->hooks->launch_multi_list(e->precision, e->d_args[1 - b], ens_tiles(e), e->reach,
@@ -724,66 +851,123 @@ static int issue_step(abl_ensemble *e) {
   return ABL_OK;
 }
 
+// What follows from how the lists fare, after the timestep that next_look names has
+// been issued.  Asked and read at fixed timesteps (ListWatch), whatever the pace of
+// host and device and however simulate() is called.
+//
+// Lists grown: a member whose lists have outgrown their capacity enters them anew
+// at the next timestep, which is the one a run of it alone does that at
+// (list_watch, enter_lists).  One overflowed list makes its member rebuild on
+// every timestep: 30 members of up to 8,192 boids, FP32, 18 us per timestep, and
+// 90 from the first list that outgrew its capacity on.
+//
+// One launch per rebuild or four: one above a quarter of the timesteps, back below
+// an eighth, so that a rate in between does not switch to and fro.
+static int look(abl_ensemble *e) {
+  const uint64_t t = e->timestep - 1;
+  const size_t M = e->mem.size();
+  bool ask = false;
+  auto slot = [&](uint64_t t_req) { return e->h_look + (t_req % e->kSlots) * (1 + M); };
+  // an answer is there: waits, for what was asked kListSample timesteps ago
+  auto answer = [&](ListWatch &w, const uint32_t **words) -> hipError_t {
+    const hipError_t err = hipEventSynchronize(e->look_ev[w.t_req % e->kSlots]);
+    *words = slot(w.t_req);
+    w.read();
+    return err;
+  };
+  const uint32_t *words = nullptr;
+  uint64_t next = ~0ull;
+  for (size_t m = 0; m < M; m++) {
+    Member &mb = e->mem[m];
+    if (mb.watch.next() == t) {
+      if (mb.watch.pending) {
+        ENS_TRY(answer(mb.watch, &words));
+        if (grow_lists(e, mb, words[1 + m])) e->entering.push_back((int) m);
+      } else {
+        ask = true;
+        mb.watch.asked(t);
+      }
+    }
+    next = std::min(next, mb.watch.next());
+  }
+  if (e->watch.next() == t) {
+    if (e->watch.pending) {
+      const uint64_t steps = e->watch.t_req - e->watch.t_prev;
+      ENS_TRY(answer(e->watch, &words));
+      const uint64_t rebuilt = words[0] - e->gen_seen;
+      e->gen_seen = words[0];
+      const bool split = e->split ? rebuilt * 8u >= steps : rebuilt * 4u > steps;
+      if (split != e->split) {
+        e->split = split;
+        ENS_TRY(hipMemsetAsync(e->nl_gate + kGateQueue, 0, (kGateWords - kGateQueue) * 4, e->stream));
+      }
+    } else {
+      ask = true;
+      e->watch.asked(t);
+    }
+  }
+  e->next_look = std::min(next, e->watch.next());
+  if (ask) {
+    uint32_t *w = slot(t);
+    ENS_TRY(hipMemcpyAsync(w, e->nl_gate + kGateGen, 4, hipMemcpyDeviceToHost, e->stream));
+    ENS_TRY(hipMemcpyAsync(w + 1, e->nl_mlong, M * 4, hipMemcpyDeviceToHost, e->stream));
+    ENS_TRY(hipEventRecord(e->look_ev[t % e->kSlots], e->stream));
+  }
+  return ABL_OK;
+}
+
+// Two timesteps as a graph, in the form the rebuilds have.
+static int capture(abl_ensemble *e) {
+  const int k = e->split ? 1 : 0;
+  if (e->exec[k]) return ABL_OK;
+  const uint64_t t0 = e->timestep;
+  ENS_TRY(hipStreamBeginCapture(e->stream, hipStreamCaptureModeThreadLocal));
+  int rc = issue_step(e);
+  if (!rc) rc = issue_step(e);
+  hipError_t ce = hipStreamEndCapture(e->stream, &e->graph[k]);
+  e->timestep = t0;  // captured, not run
+  if (rc) return rc;
+  ENS_TRY(ce);
+  ENS_TRY(hipGraphInstantiate(&e->exec[k], e->graph[k], nullptr, nullptr, 0));
+  return ABL_OK;
+}
+
 extern "C" int abl_ens_simulate(abl_ensemble *e, int steps) {
   if (!e || steps < 0) return ens_fail(ABL_ERR_ARG, "bad argument");
   if (!e->ready) return ens_fail(ABL_ERR_STATE, "abl_ens_init first");
   ENS_TRY(hipEventRecord(e->ev0, e->stream));
-  int t = 0;
-  if (e->use_graph && steps > 0) {
+  const uint64_t end = e->timestep + (uint64_t) steps;
+  const bool watched = e->lists && e->n > 0;
+  while (e->timestep < end) {
     // the id buffer (without lists) or the column buffers and the gates'
     // parity (with lists) alternate per step: two timesteps, captured from
     // an even start, end where they start
-    auto even = [&] { return e->lists ? (e->timestep & 1u) == 0 : (e->id_cur & 1) == 0; };
-    if (!e->exec) {
-      if (even() && steps >= 2) {
-        const uint64_t t0 = e->timestep;
-        ENS_TRY(hipStreamBeginCapture(e->stream, hipStreamCaptureModeThreadLocal));
-        int rc = issue_step(e);
-        if (!rc) rc = issue_step(e);
-        hipError_t ce = hipStreamEndCapture(e->stream, &e->graph);
-        e->timestep = t0;  // captured, not run
-        if (rc) return rc;
-        ENS_TRY(ce);
-        ENS_TRY(hipGraphInstantiate(&e->exec, e->graph, nullptr, nullptr, 0));
-      }
+    const bool even = e->lists ? (e->timestep & 1u) == 0 : (e->id_cur & 1) == 0;
+    const bool plain = !watched || (e->entering.empty() && e->next_look != e->timestep);
+    if (e->use_graph && even && plain && e->timestep + 2 <= end) {
+      const int rc = capture(e);
+      if (rc) return rc;
+      ENS_TRY(hipGraphLaunch(e->exec[e->split ? 1 : 0], e->stream));
+      e->timestep += 2;
+    } else {
+      const int rc = issue_step(e);
+      if (rc) return rc;
     }
-    if (e->exec && even()) {
-      for (; t + 2 <= steps; t += 2) {
-        ENS_TRY(hipGraphLaunch(e->exec, e->stream));
-        e->timestep += 2;
-      }
+    if (watched && e->next_look == e->timestep - 1) {
+      const int rc = look(e);
+      if (rc) return rc;
     }
-  }
-  for (; t < steps; t++) {
-    int rc = issue_step(e);
-    if (rc) return rc;
   }
   ENS_TRY(hipEventRecord(e->ev1, e->stream));
   if (e->h_error)
-    ENS_TRY(hipMemcpyAsync(e->h_error, e->nl_gate + kGateError, 8, hipMemcpyDeviceToHost, e->stream));
+    ENS_TRY(hipMemcpyAsync(e->h_error, e->nl_gate + kGateError, 4, hipMemcpyDeviceToHost, e->stream));
   return ABL_OK;
 }
 
-// After a synchronisation: no rebuild of the timesteps so far gave up waiting; and
-// the form of the rebuilds to come, by how many of these timesteps rebuilt.
-static int ens_check(abl_ensemble *e) {
-  if (!e->h_error) return ABL_OK;
-  const volatile uint32_t *h = e->h_error;
-  if (h[0]) return ens_fail(ABL_ERR_DEVICE, "list rebuild: a phase did not finish");
-  const uint64_t steps = e->timestep - e->step_seen;
-  if (steps >= 8) {
-    const bool split = (uint64_t) (h[1] - e->gen_seen) * 4u > steps;
-    e->gen_seen = h[1];
-    e->step_seen = e->timestep;
-    if (split != e->split) {
-      e->split = split;
-      ENS_TRY(hipMemsetAsync(e->nl_gate + kGateQueue, 0, (kGateWords - kGateQueue) * 4, e->stream));
-      if (e->exec) ENS_TRY(hipGraphExecDestroy(e->exec));
-      if (e->graph) ENS_TRY(hipGraphDestroy(e->graph));
-      e->exec = nullptr;
-      e->graph = nullptr;
-    }
-  }
+// After a synchronisation: no rebuild of the timesteps so far gave up waiting.
+static int ens_check(const abl_ensemble *e) {
+  if (e->h_error && *(const volatile uint32_t *) e->h_error)
+    return ens_fail(ABL_ERR_DEVICE, "list rebuild: a phase did not finish");
   return ABL_OK;
 }
 
@@ -833,6 +1017,20 @@ extern "C" int abl_ens_download(abl_ensemble *e, int member, void *aos, size_t c
   ENS_TRY(hipMemcpyAsync(aos, e->dl, bytes, hipMemcpyDeviceToHost, e->stream));
   ENS_TRY(hipStreamSynchronize(e->stream));
   return ens_check(e);
+}
+
+// What the ensemble has decided for a member.
+extern "C" int abl_ens_inspect(abl_ensemble *e, int member, const char *what, double *value) {
+  if (!e || member < 0 || member >= (int) e->mem.size() || !what || !value)
+    return ens_fail(ABL_ERR_ARG, "bad argument");
+  const Member &mb = e->mem[(size_t) member];
+  const std::string k(what);
+  if (k == "lists") *value = e->lists && mb.n > 0;
+  else if (k == "list_capacity") *value = mb.cap;
+  else if (k == "rebuild_launches") *value = e->split ? 4 : 1;
+  else if (k == "rebuilds") *value = e->gen_seen - 1u;
+  else return ens_fail(ABL_ERR_ARG, "unknown quantity " + k);
+  return ABL_OK;
 }
 
 extern "C" int abl_ens_agents(abl_ensemble *e, size_t *total) {

@@ -246,7 +246,8 @@ struct AgentStore {
   // previous sample
   uint32_t *nl_host = nullptr;
   hipEvent_t nl_ev = nullptr;
-  bool nl_pending = false, nl_watched = false;
+  ListWatch nl_watch;
+  uint32_t nl_c_prev = 0;
   bool nl_off = false;          // lists given up for this type (rebuilt nearly every step)
   bool nl_kept = false;         // the rebuild rate was measured and the lists kept
   // whether the agents crowd into tiles that do not fit LDS (probe_tiles),
@@ -254,8 +255,6 @@ struct AgentStore {
   bool dense = false, dense_known = false;
   uint32_t crowd = 0;  // those agents, as last counted
   bool on_tiles = false;  // the last step walked the stencil on tiles
-  uint64_t nl_t_req = 0, nl_t_prev = 0;
-  uint32_t nl_c_prev = 0;
   // run-time add/remove: ids stop being 0..n-1 once agents die or are born
   int64_t next_id = 0;
   bool ids_dense = true;
@@ -398,7 +397,7 @@ static void free_store(AgentStore &s) {
   if (s.nl_host) (void) hipHostFree(s.nl_host);
   s.nl_ev = nullptr;
   s.nl_host = nullptr;
-  s.nl_pending = false;
+  s.nl_watch = ListWatch{};
   for (int c = 0; c < kMaxCols; c++) {
     if (s.bmem[c]) (void) hipFree(s.bmem[c]);
     s.bmem[c] = nullptr;
@@ -1675,13 +1674,6 @@ static int apply_births(abl_sim *sim, AgentStore &parent, AgentStore &child, int
 
 // ---- neighbour lists ---------------------------------------------------------------
 
-// Capacity for lists of up to `longest` entries: a quarter more, but at most
-// four times the estimate (an agent in a dense cluster with a longer list walks
-// the stencil instead).
-static int list_room(const AgentStore &b, uint32_t longest) {
-  return (int) std::min(1.25 * (double) longest + 16.0, 4.0 * (double) b.nl_est);
-}
-
 // The gate block of an agent type.
 static int reserve_gate(abl_sim *sim, AgentStore &s) {
   if (s.nl_gate) return ABL_OK;
@@ -1778,10 +1770,10 @@ static void keep_neighbours(AgentStore &b, StepLaunch &L) {
 
 // What the host looks at while a type walks lists: the longest list built and
 // the number of rebuilds run since the lists were entered (NListArgs::stats).
-// It copies them to pinned memory behind an event, the first time kListSample
-// timesteps after entry and then every kListWatch, and reads the copy when it
-// has issued another kListSample timesteps (waiting for the event if need be:
-// the device still has those timesteps queued, so the wait costs it nothing).
+// It copies them to pinned memory behind an event at the timesteps ListWatch
+// names, and reads the copy when it has issued another kListSample timesteps
+// (waiting for the event if need be: the device still has those timesteps queued,
+// so the wait costs it nothing).
 // What follows from them is thus decided at a fixed timestep, whatever the
 // host's and the device's pace, and runs give the same bits alone, batched or
 // served.
@@ -1798,48 +1790,42 @@ static void keep_neighbours(AgentStore &b, StepLaunch &L) {
 // list mode anew, with room for the longest list (list_room's bound).  boids2d,
 // 65,536 agents at ten times the time step, 300 timesteps: 29 us per timestep,
 // 54 without growing.
-constexpr uint64_t kListSample = 8, kListWatch = 64;
 static int list_watch(abl_sim *sim, AgentStore &b) {
-  if (b.nl_off) return ABL_OK;
+  ListWatch &w = b.nl_watch;
+  if (b.nl_off || sim->timestep < w.next()) return ABL_OK;
   if (!b.nl_host) {
     HIP_TRY(hipHostMalloc((void **) &b.nl_host, 3 * 4, hipHostMallocDefault));
     HIP_TRY(hipEventCreateWithFlags(&b.nl_ev, hipEventDisableTiming));
   }
-  if (b.nl_pending) {
-    if (sim->timestep - b.nl_t_req < kListSample) return ABL_OK;
-    HIP_TRY(hipEventSynchronize(b.nl_ev));
-    b.nl_pending = false;
-    const uint32_t longest = b.nl_host[0], c = b.nl_host[2];
-    const uint64_t dt = b.nl_t_req - b.nl_t_prev;
-    if (!sim->nlist_set && !b.nl_kept) {
-      if (2 * (uint64_t) (c - b.nl_c_prev) > dt) {
-        b.nl_off = true;
-        b.sorted = false;  // the stencil walk starts from a full sort
-        return ABL_OK;
-      }
-      b.nl_kept = true;
-    }
-    b.nl_c_prev = c;
-    b.nl_t_prev = b.nl_t_req;
-    if (!sim->list_cap && (int64_t) longest > b.nl_cap && list_room(b, longest) > b.nl_cap) {
-      b.nl_want = list_room(b, longest);
-      b.nl_ok = false;
-      b.sorted = false;
-    }
-    return ABL_OK;
-  }
-  if (sim->timestep - b.nl_t_prev >= (b.nl_watched ? kListWatch : kListSample)) {
+  if (!w.pending) {
     HIP_TRY(hipMemcpyAsync(b.nl_host, b.nl_gate + 2, 3 * 4, hipMemcpyDeviceToHost, sim->stream));
     HIP_TRY(hipEventRecord(b.nl_ev, sim->stream));
-    b.nl_t_req = sim->timestep;
-    b.nl_pending = b.nl_watched = true;
+    w.asked(sim->timestep);
+    return ABL_OK;
+  }
+  HIP_TRY(hipEventSynchronize(b.nl_ev));
+  const uint32_t longest = b.nl_host[0], c = b.nl_host[2];
+  const uint64_t dt = w.t_req - w.t_prev;
+  w.read();
+  if (!sim->nlist_set && !b.nl_kept) {
+    if (2 * (uint64_t) (c - b.nl_c_prev) > dt) {
+      b.nl_off = true;
+      b.sorted = false;  // the stencil walk starts from a full sort
+      return ABL_OK;
+    }
+    b.nl_kept = true;
+  }
+  b.nl_c_prev = c;
+  if (!sim->list_cap && (int64_t) longest > b.nl_cap && list_room(b.nl_est, longest) > b.nl_cap) {
+    b.nl_want = list_room(b.nl_est, longest);
+    b.nl_ok = false;
+    b.sorted = false;
   }
   return ABL_OK;
 }
 
 static int reserve_lists(abl_sim *sim, AgentStore &s, int cap) {
-  cap = (cap + 7) & ~7;  // whole 16-byte rows of entries
-  if (cap > 65528) cap = 65528;
+  cap = list_capacity(cap);
   if (s.nl_idx && s.nl_cap >= cap && s.nl_ncap >= s.n) return ABL_OK;
   void *ptrs[] = {s.nl_idx, s.nl_len, s.nl_pos0, s.nl_perm, s.nl_prow0};
   HIP_TRY(hipStreamSynchronize(sim->stream));
@@ -1882,22 +1868,13 @@ static NListArgs list_args(const abl_sim *sim, const AgentStore &s, double r, do
   return nl;
 }
 
-// List entries of an agent: half again the expected population of the list
-// radius rl.
-static int list_estimate(const AgentStore &b, double rl) {
-  const double vol = b.dim == 3 ? 4.0 / 3.0 * M_PI * rl * rl * rl : M_PI * rl * rl;
-  const double env = (double) b.ncells * std::pow(b.cell, (double) b.dim);
-  const double expect = env > 0 ? vol * (double) b.n / env : 0.0;
-  return (int) (1.5 * expect) + 16;
-}
-
 // Enter list mode on a fresh grid: build the lists from the current buffers,
 // grow them once if the longest list did not fit (one host wait per entry).
 // Not entered (nl_ok stays false) when the agents turn out to crowd into tiles
 // that do not fit LDS.
 static int enter_lists(abl_sim *sim, AgentStore &b, const StepDesc &st, const StepLaunch &Lb,
                        double r, double rl) {
-  b.nl_est = list_estimate(b, rl);
+  b.nl_est = list_estimate(b.dim, b.ncells, b.cell, b.n, rl);
   const int want = sim->list_cap ? sim->list_cap : std::max(std::max(b.nl_cap, b.nl_est), b.nl_want);
   b.nl_want = 0;
   if (sim->list_cap && b.nl_cap != ((sim->list_cap + 7) & ~7)) b.nl_cap = 0;  // size requested
@@ -1927,10 +1904,9 @@ static int enter_lists(abl_sim *sim, AgentStore &b, const StepDesc &st, const St
     if (b.dense) return ABL_OK;
     // watched from here on (list_watch)
     b.nl_c_prev = words[2];
-    b.nl_t_prev = sim->timestep;
-    b.nl_pending = b.nl_watched = false;
-    const int grow = list_room(b, longest);
-    if ((int) longest <= b.nl_cap || grow <= b.nl_cap || b.nl_cap >= 65528 || sim->list_cap) break;
+    b.nl_watch.entered(sim->timestep);
+    const int grow = list_room(b.nl_est, longest);
+    if ((int) longest <= b.nl_cap || grow <= b.nl_cap || b.nl_cap >= kListMost || sim->list_cap) break;
     rc = reserve_lists(sim, b, grow);
     if (rc) return rc;
   }

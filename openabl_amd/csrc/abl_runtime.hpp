@@ -11,6 +11,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
+#include <cmath>
 #include <initializer_list>
 #include <string>
 #include <vector>
@@ -50,6 +52,48 @@ struct NListArgs;
 
 // Default neighbour-list skin, as a fraction of the near radius.
 constexpr double kDefaultSkin = 0.05;
+
+// Neighbour-list capacities, in entries per agent (runs alone and ensembles).
+// From the expected population of the list radius rl, and half again, at first:
+inline int list_estimate(int dim, size_t ncells, double cell, size_t n, double rl) {
+  const double vol = dim == 3 ? 4.0 / 3.0 * M_PI * rl * rl * rl : M_PI * rl * rl;
+  const double env = (double) ncells * std::pow(cell, (double) dim);
+  const double expect = env > 0 ? vol * (double) n / env : 0.0;
+  return (int) (1.5 * expect) + 16;
+}
+// for lists of up to `longest` entries a quarter more, but at most four times the
+// estimate (an agent in a dense cluster with a longer list walks the stencil
+// instead);
+inline int list_room(int estimate, uint32_t longest) {
+  return (int) std::min(1.25 * (double) longest + 16.0, 4.0 * (double) estimate);
+}
+// in whole 16-byte rows of 16-bit entries.
+inline int list_capacity(int want) { return std::min((want + 7) & ~7, 65528); }
+constexpr int kListMost = 65528;
+
+// When the host looks at how lists fare (list_watch in abl_runtime.hip, look in
+// abl_ensemble.hip): what it reads is copied kListSample timesteps after the lists
+// were entered and then every kListWatch, and acted on another kListSample later,
+// by when it has long arrived.
+constexpr uint64_t kListSample = 8, kListWatch = 64;
+struct ListWatch {
+  uint64_t t_prev = 0, t_req = 0;
+  bool pending = false, watched = false;
+  // the timestep after which there is something to do: to read where pending,
+  // else to ask
+  uint64_t next() const {
+    return pending ? t_req + kListSample : t_prev + (watched ? kListWatch : kListSample);
+  }
+  void entered(uint64_t t) { *this = ListWatch{t, 0, false, false}; }
+  void asked(uint64_t t) {
+    t_req = t;
+    pending = watched = true;
+  }
+  void read() {
+    t_prev = t_req;
+    pending = false;
+  }
+};
 
 // Hooks a single-type, single-step program provides so many independent runs
 // of it can be batched into one launch per kernel (abl_ensemble.hip).

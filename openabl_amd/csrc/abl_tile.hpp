@@ -865,7 +865,8 @@ __device__ __forceinline__ void tiled_body(const typename M::Args &a, unsigned t
 // Build the lists of one tile's agents; returns the longest list.
 template <class M, int TX, int TY, int TZ, int RM>
 __device__ __forceinline__ uint32_t list_build_tile(const typename M::Args &a, const NListArgs &nl,
-                                                    unsigned tile, unsigned char *smem) {
+                                                    uint32_t cap, unsigned tile,
+                                                    unsigned char *smem) {
   using F = typename M::F;
   constexpr int DIM = M::DIM;
   constexpr int NS = M::NS;
@@ -902,14 +903,14 @@ __device__ __forceinline__ uint32_t list_build_tile(const typename M::Args &a, c
         d2 += e * e;
       }
       if (d2 <= nl.r2_list) {
-        if (cnt < (uint32_t) nl.cap) {
+        if (cnt < cap) {
           put(cnt & 7u, l);
           if ((cnt & 7u) == 7u) store_row(cnt >> 3);
         }
         cnt++;
       }
     });
-    const bool fits = tile_lists && cnt <= (uint32_t) nl.cap && cnt < kListOverflow;
+    const bool fits = tile_lists && cnt <= cap && cnt < kListOverflow;
     nl.len[gi] = fits ? (uint16_t) cnt : kListOverflow;
     if (fits && (cnt & 7u)) {
       // pad the last row with the far-away record (index total)
@@ -999,7 +1000,8 @@ __global__ __launch_bounds__(256) void tiled_list_build(typename M::Args a, NLis
   }
   list_copy_starts(nl);
   const uint32_t longest =
-      list_build_tile<M, TX, TY, TZ, RM>(a, nl, xcd_block(blockIdx.x, gridDim.x), smem);
+      list_build_tile<M, TX, TY, TZ, RM>(a, nl, (uint32_t) nl.cap,
+                                         xcd_block(blockIdx.x, gridDim.x), smem);
   list_longest(nl, longest);
 }
 
@@ -1057,7 +1059,8 @@ __global__ __launch_bounds__(256) void tiled_rebuild(typename M::Args a, NListAr
   list_copy_starts(nl);
   uint32_t longest = 0;
   for (unsigned t = blockIdx.x; t < nt; t += gridDim.x) {
-    longest = max(longest, list_build_tile<M, TX, TY, TZ, RM>(a, nl, xcd_block(t, nt), smem));
+    longest = max(longest, list_build_tile<M, TX, TY, TZ, RM>(a, nl, (uint32_t) nl.cap,
+                                                              xcd_block(t, nt), smem));
     __syncthreads();  // the next tile's tables go where this one's are read
   }
   list_longest(nl, longest);
@@ -1222,26 +1225,36 @@ __global__ __launch_bounds__(256, policy_list_waves<M>::value) void tiled_step_l
 // tiled_step_multi) over one set of lists indexed by the members'
 // concatenated slots.  Besides the ensemble's gate (nl.gate: some member is
 // due a rebuild) every member has its own, by timestep parity: mgate[p *
-// members + m].  A member rebuilds exactly when a run of it alone would: when
-// one of its own agents strayed or overflowed.
+// members + m], and its own list capacity.  A member rebuilds exactly when a run
+// of it alone would: when one of its own agents strayed or overflowed.
+
+// Lists of a member that did not fit (the host looks at them now and then): one
+// atomic per wave that built one, which is none at all in nearly every build.
+__device__ __forceinline__ void member_longest(uint32_t *word, uint32_t longest, uint32_t cap) {
+  if (__builtin_amdgcn_ballot_w64(longest > cap) == 0) return;
+#pragma unroll
+  for (int d = 1; d < kWave; d <<= 1) longest = max(longest, (uint32_t) __shfl_xor((int) longest, d, kWave));
+  if (threadIdx.x % kWave == 0) atomicMax(word, longest);
+}
 
 // Every member's first lists, after the full sort, or (nl.gated) those of the
 // members due (records in the sorted buffers args point at; copied back as in
 // tiled_list_build).
 template <class M, int TX, int TY, int TZ, int RM>
 __global__ __launch_bounds__(256) void tiled_list_build_multi(const typename M::Args *__restrict__ args,
-                                                              const uint2 *__restrict__ tile_of,
-                                                              int members, NListArgs nl,
-                                                              const uint32_t *__restrict__ mgate) {
+                                                              EnsTiles e, NListArgs nl) {
   extern __shared__ __align__(16) unsigned char smem[];
   if (nl.gated && nl.gate[nl.parity] == 0u) return;
   list_copy_starts(nl);
   const unsigned t = xcd_block(blockIdx.x, gridDim.x);
-  const uint2 of = tile_of[t];
-  if (nl.gated && mgate[nl.parity * members + uniform((int) of.x)] == 0u) return;
-  const uint32_t longest = list_build_tile<M, TX, TY, TZ, RM>(
-      args[uniform((int) of.x)], nl, t - (unsigned) uniform((int) of.y), smem);
-  list_longest(nl, longest);
+  const uint2 of = e.tile_of[t];
+  const int m = uniform((int) of.x);
+  if (nl.gated && e.mgate[nl.parity * e.members + m] == 0u) return;
+  const uint32_t cap = e.mcap[m];
+  member_longest(e.mlong + m,
+                 list_build_tile<M, TX, TY, TZ, RM>(args[m], nl, cap,
+                                                    t - (unsigned) uniform((int) of.y), smem),
+                 cap);
 }
 
 // The gated re-sort and list build of the members due, in one launch
@@ -1249,7 +1262,7 @@ __global__ __launch_bounds__(256) void tiled_list_build_multi(const typename M::
 // 65,536 boids: a timestep with no member due 37 us (of it 4.6 us for this launch
 // that returns) against 48 us with seven gated launches for the full sort and the list
 // build.  Where members are due on most timesteps the ensemble takes the re-sort's
-// phases as launches of their own instead (ens_check): every member due on every
+// phases as launches of their own instead (look): every member due on every
 // timestep 230 us this way, 130 with four launches.
 template <class M, int TX, int TY, int TZ, int RM>
 __global__ __launch_bounds__(256) void tiled_rebuild_multi(const typename M::Args *__restrict__ args,
@@ -1269,17 +1282,18 @@ __global__ __launch_bounds__(256) void tiled_rebuild_multi(const typename M::Arg
       }))
     return;
   list_copy_starts(nl);
-  uint32_t longest = 0;
   for (unsigned t = blockIdx.x; t < e.total; t += gridDim.x) {
     const unsigned tile = xcd_block(t, e.total);
     const uint2 of = e.tile_of[tile];
     const int m = uniform((int) of.x);
     if (due[m] == 0u) continue;
-    longest = max(longest, list_build_tile<M, TX, TY, TZ, RM>(
-                               args[m], nl, tile - (unsigned) uniform((int) of.y), smem));
+    const uint32_t cap = e.mcap[m];
+    member_longest(e.mlong + m,
+                   list_build_tile<M, TX, TY, TZ, RM>(args[m], nl, cap,
+                                                      tile - (unsigned) uniform((int) of.y), smem),
+                   cap);
     __syncthreads();  // the next tile's tables go where this one's are read
   }
-  list_longest(nl, longest);
 }
 
 // One timestep of every member through the lists; clears this parity's gates

@@ -535,8 +535,8 @@ int ens_launch_list(const void *args, const EnsTiles &e, float occupancy, int bl
   const int threads = block > 256 ? 256 : block;
   const BoidArgs<F> *ma = (const BoidArgs<F> *) args;
   if (mode == 1) {
-    hipLaunchKernelGGL((tiled_list_build_multi<M, TX, TY, 1, RM>), e.total, threads, smem, st, ma,
-                       e.tile_of, e.members, nl, e.mgate);
+    hipLaunchKernelGGL((tiled_list_build_multi<M, TX, TY, 1, RM>), e.total, threads, smem, st, ma, e,
+                       nl);
   } else if (mode == 2) {
     hipLaunchKernelGGL((tiled_step_list_multi<M, TX, TY, 1, RM>), e.total, threads, smem, st, ma,
                        e.tile_of, e.members, nl, e.mgate);

@@ -65,6 +65,12 @@ class Ensemble:
         _check(self.lib.abl_ens_agents(self.h, C.byref(n)))
         return n.value
 
+    def inspect(self, what: str, member: int = 0) -> float:
+        """What the ensemble has decided for a member (abl_ens_inspect)."""
+        v = C.c_double()
+        _check(self.lib.abl_ens_inspect(self.h, member, what.encode(), C.byref(v)))
+        return v.value
+
     def download(self, member: int) -> np.ndarray:
         dt = record_dtype(AGENTS[self.program][0][1], self.precision)
         n = C.c_size_t()

@@ -89,6 +89,7 @@ _SIGNATURES = {
     "abl_ens_synchronize": ([C.c_void_p, C.c_void_p], C.c_int),
     "abl_ens_member_count": ([C.c_void_p, C.c_int, C.c_void_p], C.c_int),
     "abl_ens_agents": ([C.c_void_p, C.c_void_p], C.c_int),
+    "abl_ens_inspect": ([C.c_void_p, C.c_int, C.c_char_p, C.c_void_p], C.c_int),
     "abl_ens_download": ([C.c_void_p, C.c_int, C.c_void_p, C.c_size_t, C.c_void_p], C.c_int),
     "abl_ens_destroy": ([C.c_void_p], C.c_int),
 }

@@ -26,8 +26,7 @@ def members(k, seed=5):
 
 
 LISTS = {"stencil": {"hip.nlist": 0},
-         # a fixed list capacity, so a list that outgrows it overflows in the
-         # ensemble exactly when it does in the run alone
+         # a fixed list capacity: lists that outgrow it overflow
          "lists": {"hip.nlist": 1, "hip.list_cap": 96},
          # a skin a boid at full speed crosses in three steps: rebuilds
          "lists-skin": {"hip.nlist": 1, "hip.list_cap": 96, "hip.skin": 0.0005}}
@@ -101,15 +100,85 @@ def test_rebuild_chunks_of_many_members(count, most, graph):
     cfg = {"hip.cell_scale": 2, "hip.tile": 1, "hip.nlist": 1, "hip.list_cap": 96, "hip.skin": 0.001}
     ens = Ensemble("boids2d", "f64", ms, config=dict(cfg, **{"hip.graph": graph}))
     ens.init(0x1234, 0x5678)
-    ens.simulate(9)
-    ens.synchronize()  # most timesteps rebuilt: four launches per rebuild from here on
+    assert ens.inspect("rebuild_launches") == 1
+    ens.simulate(17)
+    assert ens.inspect("rebuild_launches") == 4  # most of the first timesteps rebuilt
     ens.simulate(7)
     dt = record_dtype(MEMBERS["boids2d"], "f64")
     for m in sorted({0, count // 2, count - 1, *rng.integers(0, count, 3).tolist()}):
         load_library().abl_rng_seed(*member_seed(0x1234, 0x5678, m))
         sim = Simulation("boids2d", "f64", params=ms[m], config=cfg)
         sim.init_agents()
-        sim.simulate(16)
+        sim.simulate(24)
         assert field_bytes(ens.download(m)) == field_bytes(sim.download(dt)), m
+        sim.close()
+    ens.close()
+
+
+@pytest.mark.parametrize("prec", ["f64", "f32"])
+@pytest.mark.parametrize("graph,chunks", [(1, (90, 110, 141)), (0, (341,)), (1, (17, 1, 71, 252))])
+def test_lists_grow_as_in_runs_alone(prec, graph, chunks):
+    """Members whose agents draw together until their lists outgrow the capacity
+    sized from their density: each enters its lists anew, with more room, on the
+    timestep a run of it alone does, so capacities and bits stay the run's,
+    however simulate() is called.  One member stays as it is."""
+    from openabl_amd import MEMBERS, Simulation, load_library, record_dtype
+    from openabl_amd.ensemble import Ensemble, member_seed
+    print(f"case ensemble growing lists {prec} graph={graph} {chunks}", flush=True)
+    ms = [{"num_agents": n, "agent_density": 0.065536, "max_pos": fold6(math.sqrt(n / 0.065536)),
+           "time_scale": t, "steer_scale": s, "collision_scale": 1.5}
+          for n, t, s in ((3001, 0.05, 3.0), (1500, 0.02, 3.0), (700, 0.0005, 1.0), (2000, 0.2, 2.0))]
+    cfg = {"hip.cell_scale": 1, "hip.tile": 1, "hip.nlist": 1}
+    ens = Ensemble("boids2d", prec, ms, config=dict(cfg, **{"hip.graph": graph}))
+    ens.init(0x1234, 0x5678)
+    first = [ens.inspect("list_capacity", m) for m in range(len(ms))]
+    sims = []
+    for m, p in enumerate(ms):
+        load_library().abl_rng_seed(*member_seed(0x1234, 0x5678, m))
+        sims.append(Simulation("boids2d", prec, params=p, config=cfg))
+        sims[m].init_agents()
+    dt = record_dtype(MEMBERS["boids2d"], prec)
+    for n in chunks:
+        ens.simulate(n)
+        for m, sim in enumerate(sims):
+            sim.simulate(n)
+            assert field_bytes(ens.download(m)) == field_bytes(sim.download(dt)), (n, m)
+    last = [ens.inspect("list_capacity", m) for m in range(len(ms))]
+    assert last == [sim.inspect("list_capacity") for sim in sims]
+    grown = [b > a for a, b in zip(first, last)]
+    assert sum(grown) >= 2 and not grown[2], (first, last)
+    for sim in sims:
+        sim.close()
+    ens.close()
+
+
+def test_members_equal_alone_runs_while_the_rebuild_changes_form():
+    """A batch whose rebuild rate goes above and below what one launch per rebuild
+    is for, several times, with lists growing meanwhile: both captured graphs in
+    turn, and still every member's run alone."""
+    from openabl_amd import MEMBERS, Simulation, load_library, record_dtype
+    from openabl_amd.ensemble import Ensemble, member_seed
+    print("case ensemble rebuild forms in turn", flush=True)
+    rng = np.random.default_rng(3)
+    ms = [{"num_agents": int(n), "agent_density": 0.065536, "max_pos": fold6(math.sqrt(n / 0.065536)),
+           "time_scale": 0.002} for n in rng.integers(300, 2000, 12)]
+    cfg = {"hip.cell_scale": 1, "hip.tile": 1, "hip.nlist": 1}
+    ens = Ensemble("boids2d", "f32", ms, config=cfg)
+    ens.init(1, 2)
+    forms = [ens.inspect("rebuild_launches")]
+    for _ in range(90):
+        ens.simulate(10)
+        now = ens.inspect("rebuild_launches")
+        if now != forms[-1]:
+            forms.append(now)
+    assert forms[:3] == [1, 4, 1]
+    dt = record_dtype(MEMBERS["boids2d"], "f32")
+    for m, p in enumerate(ms):
+        load_library().abl_rng_seed(*member_seed(1, 2, m))
+        sim = Simulation("boids2d", "f32", params=p, config=cfg)
+        sim.init_agents()
+        sim.simulate(900)
+        assert field_bytes(ens.download(m)) == field_bytes(sim.download(dt)), m
+        assert ens.inspect("list_capacity", m) == sim.inspect("list_capacity"), m
         sim.close()
     ens.close()
