@@ -150,7 +150,7 @@ struct abl_ensemble {
   int list_cap = 0;            // "hip.list_cap": entries per list (0: sized from the data)
   bool lists = false;          // in use (decided by abl_ens_init)
   double r = 0.0, rl = 0.0, cell = 0.0;
-  int nl_cap = 0;              // entries per agent allocated: the largest member's capacity
+  int nl_cap = 0;              // entries per agent allocated, at least the largest member's capacity
   uint16_t *nl_idx = nullptr, *nl_len = nullptr;
   uint32_t *nl_perm = nullptr;
   uint4 *nl_prow0 = nullptr;
@@ -487,12 +487,15 @@ static int issue_rebuild(abl_ensemble *e) {
 }
 
 // Entry lists for the largest capacity; those of members that keep theirs stay
-// (rows of eight entries of all agents, so more rows go behind).  The captured
-// timesteps hold the address.
+// (rows of eight entries of all agents, so more rows go behind).  Twice the rows
+// asked for, where lists may grow: an allocation and captures anew, since the
+// captured timesteps hold the address, cost 4 ms for 470,000 agents, as much as
+// 100 timesteps.
 static int reserve_entries(abl_ensemble *e) {
   int cap = 0;
   for (const Member &mb : e->mem) cap = std::max(cap, mb.cap);
   if (cap <= e->nl_cap) return ABL_OK;
+  if (!e->list_cap) cap = list_capacity(2 * cap);
   uint16_t *idx = nullptr;
   ENS_TRY(hipMalloc(&idx, (size_t) cap * e->n * 2));
   if (e->nl_idx) {
@@ -574,6 +577,15 @@ static int enter_members(abl_ensemble *e) {
   }
   e->entering.clear();
   return rc;
+}
+
+// The generation and the members' longest lists to pinned memory: a copy command
+// between kernels holds the stream up for some 20 us, twice what this launch takes.
+__global__ void k_ens_tell(const uint32_t *__restrict__ gen, const uint32_t *__restrict__ mlong,
+                           int members, uint32_t *__restrict__ out) {
+  const int m = blockIdx.x * blockDim.x + threadIdx.x;
+  if (m == 0) __hip_atomic_store(out, *gen, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  if (m < members) __hip_atomic_store(out + 1 + m, mlong[m], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // List buffers, and every member's first sort and lists, as a run alone enters
@@ -909,8 +921,9 @@ static int look(abl_ensemble *e) {
   e->next_look = std::min(next, e->watch.next());
   if (ask) {
     uint32_t *w = slot(t);
-    ENS_TRY(hipMemcpyAsync(w, e->nl_gate + kGateGen, 4, hipMemcpyDeviceToHost, e->stream));
-    ENS_TRY(hipMemcpyAsync(w + 1, e->nl_mlong, M * 4, hipMemcpyDeviceToHost, e->stream));
+    hipLaunchKernelGGL(k_ens_tell, grid_blocks((int) M, 256), 256, 0, e->stream, e->nl_gate + kGateGen,
+                       e->nl_mlong, (int) M, w);
+    ENS_TRY(hipGetLastError());
     ENS_TRY(hipEventRecord(e->look_ev[t % e->kSlots], e->stream));
   }
   return ABL_OK;

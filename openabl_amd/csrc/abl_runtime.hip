@@ -2328,7 +2328,7 @@ extern "C" int abl_hip_estimate_footprint(const char *program, int precision, in
         // estimate of a uniform population grown at most four times
         const double rl = r * (1.0 + kDefaultSkin);
         const double ball = s.dim == 3 ? 4.0 / 3.0 * M_PI * rl * rl * rl : M_PI * rl * rl;
-        const double want = 1.5 * ball * (double) agents / vol + 16.0;
+        const double want = 1.5 * ball * (double) agents / vol + kListSpare;
         list_entries = std::max(list_entries, std::min(4.0 * want + 8.0, 65528.0));
       }
     }

@@ -54,12 +54,17 @@ struct NListArgs;
 constexpr double kDefaultSkin = 0.05;
 
 // Neighbour-list capacities, in entries per agent (runs alone and ensembles).
-// From the expected population of the list radius rl, and half again, at first:
+// From the expected population of the list radius rl, half again and kListSpare, at
+// first.  (A list that does not fit makes every timestep rebuild until the host
+// looks, up to 80 timesteps; with 16 to spare, members of 1,000 to 65,536 boids,
+// each with its own capacity, met the first of those after some 2,000 timesteps,
+// 5 ms in all.)
+constexpr int kListSpare = 24;
 inline int list_estimate(int dim, size_t ncells, double cell, size_t n, double rl) {
   const double vol = dim == 3 ? 4.0 / 3.0 * M_PI * rl * rl * rl : M_PI * rl * rl;
   const double env = (double) ncells * std::pow(cell, (double) dim);
   const double expect = env > 0 ? vol * (double) n / env : 0.0;
-  return (int) (1.5 * expect) + 16;
+  return (int) (1.5 * expect) + kListSpare;
 }
 // for lists of up to `longest` entries a quarter more, but at most four times the
 // estimate (an agent in a dense cluster with a longer list walks the stencil
