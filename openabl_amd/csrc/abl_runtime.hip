@@ -2304,10 +2304,19 @@ extern "C" int abl_hip_estimate_footprint(const char *program, int precision, in
     layout_agent(s, prog->agents[t], precision);
     const size_t cb = col_bytes(s);
     // columns, ids, sort scratch, upload/download staging
-    size_t per_agent = 2 * cb + 8 + 32 + s.aos_size;
-    if (adds) per_agent += 3 * cb + 16;  // a parent's newborn staging, the child store's growth
-    // flags, birth lists (2 per agent and spare), the download's table of ids
-    if (adds || removes) per_agent += 2 * 14 + 20;
+    const size_t stored = 2 * cb + 8 + 32;
+    size_t per_agent = stored + s.aos_size;
+    bool added = false, fixed = false;
+    for (const StepDesc &st : prog->steps) {
+      added = added || st.adds == (int) t + 1;
+      fixed = fixed || (st.fixed && st.near_agent == (int) t);
+    }
+    // room for a newborn of every parent, an eighth to spare, and the newborns'
+    // staging likewise (launch_step, reserve_births)
+    if (added) per_agent += stored * 5 / 4 + 1 + cb * 9 / 8 + 1;
+    // flags and birth lists (2 per agent and an eighth), the download's table of ids
+    if (adds || removes) per_agent += 24 + 21;
+    if (fixed) per_agent += 17;  // kept neighbours
     // the grid of this type, at the finest cell size a near loop over it uses
     size_t ncells = cells;
     double list_entries = 0.0;

@@ -122,6 +122,41 @@ def test_estimate_bounds_live_footprint(prog, prec, params, steps):
     assert live <= est
 
 
+@pytest.mark.parametrize("case", ["births", "life"])
+def test_estimate_bounds_what_a_type_may_come_to_hold(case):
+    """The parts of the footprint that the cases above hide behind a grid much
+    finer than theirs: a single type that bears its own newborns, its stores and
+    flags grown with room to spare; kept neighbours, on few cells."""
+    import ctypes as C
+    from openabl_amd import MEMBERS, Simulation, codegen, load_library, record_dtype
+    print(f"case footprint {case}", flush=True)
+    params = {}
+    if case == "births":
+        codegen.load_program(codegen.program_dir("model_births"))
+        prog, dt = "model_births", record_dtype([("pos", "float2"), ("life", "int"), ("age", "int")])
+    else:
+        prog, dt = "game_of_life", record_dtype(MEMBERS["game_of_life"])
+        params = {"num_agents": 400.0, "size": 20.0, "radius": 0.2}
+    n = 300000 if case == "births" else 1000000
+    rec = np.zeros(n, dt)
+    rec["pos"] = np.random.default_rng(1).uniform(0, 20, (n, 2))
+    if case == "births":
+        rec["life"], rec["age"] = 50, np.arange(n) % 4
+    sim = Simulation(prog, "f64", params=params)
+    sim.upload(rec)
+    names = (C.c_char_p * len(params))(*[k.encode() for k in params])
+    vals = (C.c_double * len(params))(*params.values())
+    for _ in range(6):
+        sim.simulate(1)
+        sim.download(dt)
+        est = C.c_size_t()
+        assert load_library().abl_hip_estimate_footprint(prog.encode(), 0, len(params), names, vals,
+                                                         sim.count(), 1, C.byref(est)) == 0
+        print(f"  {sim.count()} agents: live {sim.footprint()} estimate {est.value}", flush=True)
+        assert sim.footprint() <= est.value
+    sim.close()
+
+
 def test_status_polling_while_runs_finish():
     """One thread polls status, run times and stats while runs start and
     finish on the server's threads: every run seen DONE already has its end
