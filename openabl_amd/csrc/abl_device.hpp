@@ -337,7 +337,9 @@ __device__ __forceinline__ void for_each_candidate_row(const GridView &g, double
 
 // Visit the candidates of an agent's stencil, narrowed to the cells within rc
 // cell units of (px, py, pz), in the order of for_each_candidate:
-// visit(j, q), q the candidate's position, until it returns false.
+// visit(j, q), q the candidate's position, until it returns false.  The stencil's
+// first cells along an axis are always among them: a coordinate that is NaN is
+// binned there, and a near test accepts NaN.
 //
 // A lane's walk is a chain of reads, each waited for before the next test, so
 // AHEAD positions of a row are read together, and the next row's cell offsets
@@ -363,9 +365,16 @@ __device__ __forceinline__ void for_each_candidate_pos(const GridView &g, const 
     *a = *b = 0u;
     const int y = cy + dy, z = cz + dz;
     int xa, xb;
-    if (dz > zr || y < 0 || y >= g.n[1] || z < 0 || (g.dim == 3 && z >= g.n[2]) ||
-        !row_interval(ux, uy, uz, dy, dz, rc, R, &xa, &xb))
-      return;
+    if (dz > zr || y < 0 || y >= g.n[1] || z < 0 || (g.dim == 3 && z >= g.n[2])) return;
+    if (y == 0 || (g.dim == 3 && z == 0)) {
+      xa = -R;
+      xb = R;
+    } else if (!row_interval(ux, uy, uz, dy, dz, rc, R, &xa, &xb)) {
+      if (cx > R) return;
+      xa = xb = -cx;
+    } else if (cx <= R) {
+      xa = -cx;
+    }
     const int x0 = max(cx + xa, 0), x1 = min(cx + xb, g.n[0] - 1);
     if (x0 > x1) return;
     const uint32_t base = ((uint32_t) z * (uint32_t) g.n[1] + (uint32_t) y) * (uint32_t) g.n[0];

@@ -56,3 +56,43 @@ def test_small_sort_equals_full(model, prec, params, cfg):
         sim.close()
     assert out[0][0] == out[1][0]
     assert all(np.array_equal(x, y) for x, y in zip(out[0][1], out[1][1]))
+
+
+@pytest.mark.parametrize("prec", ["f64", "f32"])
+def test_near_loops_reach_agents_at_nan(prec):
+    """A near test accepts an agent whose position is NaN, and such agents are
+    binned to an axis' first cells: the near loops narrowed to the radius still
+    visit every one that the stencil holds (what index order does, whose sums
+    are added in another order: 1e-4 and 1e-10 of a value or of 1 after one
+    timestep, some 1,000 addends of 6e-8 and 1e-16)."""
+    from openabl_amd import AGENTS, Simulation, record_dtype
+    print(f"case population nan {prec}", flush=True)
+    rng = np.random.default_rng(2)
+    params = predator_prey_params(num_agents=6000)
+    dts = [record_dtype(m, prec) for _, m in AGENTS["predator_prey"]]
+    recs = [np.zeros(n, dt) for n, dt in zip((300, 2000, 3700), dts)]
+    for rec in recs:
+        rec["pos"] = rng.uniform(0, params["env_size"], rec["pos"].shape)
+    for rec in recs[:2]:
+        rec["dir"] = rng.uniform(-0.7, 0.7, rec["dir"].shape)
+        rec["life"] = 40
+        k = rng.choice(len(rec), 24, False)
+        rec["pos"][k[:8], 0] = rec["pos"][k[8:16], 1] = rec["pos"][k[16:]] = np.nan
+    outs = []
+    for order in ("cell", "index"):
+        sim = Simulation("predator_prey", prec, params=params, config={"hip.order": order})
+        for t, rec in enumerate(recs):
+            sim.upload(rec, t)
+        sim.simulate(1)
+        outs.append([sim.download(dt, t) for t, dt in enumerate(dts)])
+        sim.close()
+    tol = 1e-10 if prec == "f64" else 1e-4
+    assert np.isnan(outs[0][1]["steer"]).any() and not np.isnan(outs[0][1]["steer"]).all()
+    for a, b in zip(*outs):
+        assert len(a) == len(b)
+        for f in a.dtype.names:
+            if a[f].dtype.kind == "f":
+                assert np.array_equal(np.isnan(a[f]), np.isnan(b[f])), f
+                assert np.allclose(a[f], b[f], rtol=tol, atol=tol, equal_nan=True), f
+            else:
+                assert np.array_equal(a[f], b[f]), f
