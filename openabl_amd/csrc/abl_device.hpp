@@ -53,7 +53,16 @@ struct GridView {
   int reach;
   int dim;
   const uint32_t *start;  // ncells + 1 offsets into the cell-sorted order
+  uint32_t *nan;          // null, or a word that is set if a coordinate sorted is NaN (kept
+                          // for near loops by for_each_candidate_pos)
 };
+
+// Such coordinates are binned to cell 0 of their axis (cell_coord), and near tests
+// accept them whatever their distance.
+template <typename P>
+__device__ __forceinline__ void note_nan(const GridView &g, P x, P y, P z) {
+  if (g.nan && (x != x || y != y || z != z)) *g.nan = 1u;
+}
 
 __device__ __forceinline__ int cell_coord(double p, double lo, double inv, int n) {
   double q = floor((p - lo) * inv);
@@ -337,9 +346,9 @@ __device__ __forceinline__ void for_each_candidate_row(const GridView &g, double
 
 // Visit the candidates of an agent's stencil, narrowed to the cells within rc
 // cell units of (px, py, pz), in the order of for_each_candidate:
-// visit(j, q), q the candidate's position, until it returns false.  The stencil's
-// first cells along an axis are always among them: a coordinate that is NaN is
-// binned there, and a near test accepts NaN.
+// visit(j, q), q the candidate's position, until it returns false.  Where there are
+// agents at NaN (GridView::nan) the stencil's first cells along each axis, which
+// hold them, are among them too.
 //
 // A lane's walk is a chain of reads, each waited for before the next test, so
 // AHEAD positions of a row are read together, and the next row's cell offsets
@@ -360,21 +369,23 @@ __device__ __forceinline__ void for_each_candidate_pos(const GridView &g, const 
   const float uz = g.dim == 3 ? (float) ((pz - g.lo[2]) * g.inv_cell - (double) cz) : 0.f;
   const int R = g.reach;
   const int zr = g.dim == 3 ? R : 0;
+  const bool nan = g.nan && *g.nan != 0u;
   // the slots [a, b) of the stencil row (dy, dz), none past the last row
   auto fetch = [&](int dy, int dz, uint32_t *a, uint32_t *b) {
     *a = *b = 0u;
     const int y = cy + dy, z = cz + dz;
     int xa, xb;
     if (dz > zr || y < 0 || y >= g.n[1] || z < 0 || (g.dim == 3 && z >= g.n[2])) return;
-    if (y == 0 || (g.dim == 3 && z == 0)) {
-      xa = -R;
-      xb = R;
-    } else if (!row_interval(ux, uy, uz, dy, dz, rc, R, &xa, &xb)) {
-      if (cx > R) return;
-      xa = xb = -cx;
-    } else if (cx <= R) {
-      xa = -cx;
+    bool near = row_interval(ux, uy, uz, dy, dz, rc, R, &xa, &xb);
+    if (__builtin_expect(nan, 0)) {
+      const bool first = y == 0 || (g.dim == 3 && z == 0);
+      if (first || cx <= R) {
+        xb = first ? R : near ? xb : -cx;
+        xa = first ? -R : -cx;
+        near = true;
+      }
     }
+    if (!near) return;
     const int x0 = max(cx + xa, 0), x1 = min(cx + xb, g.n[0] - 1);
     if (x0 > x1) return;
     const uint32_t base = ((uint32_t) z * (uint32_t) g.n[1] + (uint32_t) y) * (uint32_t) g.n[0];

@@ -159,7 +159,8 @@ constexpr int kSmallAgents = 4096;
 constexpr int kSmallCells = 8192;
 constexpr int kSmallBlock = 1024;
 
-template <typename P>
+// NAN_NOTED: notes coordinates that are NaN (GridView::nan).
+template <typename P, bool NAN_NOTED>
 static __global__ __launch_bounds__(kSmallBlock) void k_sort_small(
     const P *__restrict__ px, const P *__restrict__ py, const P *__restrict__ pz, GridView g, int ncells,
     int n, const int32_t *__restrict__ id, GatherCols gc, int32_t *__restrict__ id_out,
@@ -184,7 +185,10 @@ static __global__ __launch_bounds__(kSmallBlock) void k_sort_small(
   for (int u = 0; u < kItems; u++) {
     const int i = tid + u * kSmallBlock;
     key[u] = i < n ? key_of(i) : 0u;
-    if (i < n) atomicAdd(&cell[key[u]], 1u);
+    if (i < n) {
+      atomicAdd(&cell[key[u]], 1u);
+      if constexpr (NAN_NOTED) note_nan<P>(g, px[i], py[i], g.dim == 3 ? pz[i] : (P) 0);
+    }
   }
   __syncthreads();
   // each thread's run of cells: counts out, offsets out and into LDS
@@ -388,6 +392,7 @@ static __global__ void k_bin_delta(const P *__restrict__ px, const P *__restrict
   if (gate && *gate == 0u) return;  // neighbour-list mode: no rebuild this timestep
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
+  note_nan<P>(g, px[i], py[i], g.dim == 3 ? pz[i] : (P) 0);
   bin_delta_item(i, cell_key<P>(g, px, py, pz, i), skey, key, count, bsum, ml, gen);
 }
 

@@ -598,8 +598,8 @@ __global__ void k_bin(const P *__restrict__ px, const P *__restrict__ py, const 
                       GridView g, uint32_t *__restrict__ key, uint32_t *__restrict__ count, int n) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  int3 c = cell_of<P>(g, px[i], py[i], g.dim == 3 ? pz[i] : (P) 0);
-  uint32_t k = ((uint32_t) c.z * (uint32_t) g.n[1] + (uint32_t) c.y) * (uint32_t) g.n[0] + (uint32_t) c.x;
+  const uint32_t k = cell_key<P>(g, px, py, pz, i);
+  note_nan<P>(g, px[i], py[i], g.dim == 3 ? pz[i] : (P) 0);
   key[i] = k;
   atomicAdd(&count[k], 1u);
 }
@@ -904,6 +904,10 @@ static int setup_grid(abl_sim *sim, AgentStore &s) {
   }
   s.ncells = ncells;
   g.start = s.startb[s.start_cur];
+  // behind the cells' counts: cleared with them, and else left set (a full sort
+  // clears it)
+  for (const StepDesc &st : sim->prog->steps)
+    if (st.nan && &sim->types[st.near_agent] == &s) g.nan = s.count + ncells;
   s.gv = g;
   return ABL_OK;
 }
@@ -937,7 +941,8 @@ template <typename P>
 static void launch_sort_small(abl_sim *sim, AgentStore &s, int n, int nc, uint32_t *start_new,
                               const GatherCols &gc) {
   const int pc = s.pos_col;
-  hipLaunchKernelGGL(k_sort_small<P>, 1, kSmallBlock, 0, sim->stream, (const P *) col_cur(s, pc),
+  const auto kernel = s.gv.nan ? k_sort_small<P, true> : k_sort_small<P, false>;
+  hipLaunchKernelGGL(kernel, 1, kSmallBlock, 0, sim->stream, (const P *) col_cur(s, pc),
                      (const P *) col_cur(s, pc + 1),
                      (const P *) (s.dim == 3 ? col_cur(s, pc + 2) : nullptr), s.gv, nc, n,
                      s.id[s.id_cur], gc, s.id[1 - s.id_cur], s.skey[1 - s.skey_cur], start_new, s.count,

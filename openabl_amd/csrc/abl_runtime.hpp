@@ -149,6 +149,8 @@ struct StepDesc {
   // whether the launcher walks this stencil on the tiles (nl_mode 0); null: yes,
   // wherever it tiles at all
   bool (*walks_tiles)(const StepLaunch &);
+  // the near loop looks at GridView::nan
+  bool nan;
 };
 
 struct ProgramDesc {

@@ -537,45 +537,49 @@ const ProgramDesc *program_predator_prey() {
        {"life", K_INT, false}}};
   static const AgentDesc grass = {
       "Grass", {{"pos", K_FLOAT2, true}, {"dead_cycles", K_INT, false}, {"avail", K_BOOL, false}}};
-  static const ProgramDesc d = {
-      "predator_prey",
-      {mover_pred, mover_prey, grass},
-      {{"SPACE_MULT", 1.0}, {"REPRODUCE_PREY_PROB", 0.005}, {"REPRODUCE_PREDATOR_PROB", 0.001},
-       {"GAIN_FROM_FOOD_PREDATOR", 35}, {"GAIN_FROM_FOOD_PREY", 60}, {"GRASS_REGROW_CYCLES", 60},
-       {"PRED_PREY_INTERACTION_RADIUS", 0.1}, {"PREY_GROUP_COHESION_RADIUS", 0.12},
-       {"SAME_SPECIES_AVOIDANCE_RADIUS", 0.035}, {"GRASS_EAT_DISTANCE", 0.02},
-       {"PRED_KILL_DISTANCE", 0.02}, {"DELTA_TIME", 0.0015}, {"PRED_SPEED_ADVANTAGE", 2.0},
-       {"prey_fraction", 0.35}, {"predator_fraction", 0.025}, {"agent_density", 1600.0},
-       {"num_agents", 3200}, {"num_timesteps", 100}, {"env_size", 1.41421}},
-      {
-          {"pred_follow_prey", T_PREDATOR, T_PREY, "PRED_PREY_INTERACTION_RADIUS", 1.0, W_STEER,
-           launch_pred_follow_prey, false, 0},
-          {"prey_avoid_pred", T_PREY, T_PREDATOR, "PRED_PREY_INTERACTION_RADIUS", 1.0, W_STEER,
-           launch_prey_avoid_pred, false, 0},
-          {"prey_flock", T_PREY, T_PREY, "PREY_GROUP_COHESION_RADIUS", 1.0, W_STEER,
-           launch_prey_flock, false, 0},
-          {"pred_avoid", T_PREDATOR, T_PREDATOR, "SAME_SPECIES_AVOIDANCE_RADIUS", 1.0, W_STEER,
-           launch_pred_avoid, false, 0},
-          {"prey_move", T_PREY, -1, nullptr, 0.0, W_MOVE, launch_prey_move, false, 0},
-          {"pred_move", T_PREDATOR, -1, nullptr, 0.0, W_MOVE, launch_pred_move, false, 0},
-          {"prey_eat_or_starve", T_PREY, T_GRASS, "GRASS_EAT_DISTANCE", 1.0, W_LIFE,
-           launch_prey_eat_or_starve, true, 0},
-          {"pred_eat_or_starve", T_PREDATOR, T_PREY, "PRED_KILL_DISTANCE", 1.0, W_LIFE,
-           launch_pred_eat_or_starve, true, 0},
-          {"grass_eaten", T_GRASS, T_PREY, "GRASS_EAT_DISTANCE", 1.0, W_GRASS,
-           launch_grass_eaten, false, 0},
-          {"prey_eaten", T_PREY, T_PREDATOR, "PRED_KILL_DISTANCE", 1.0, 0u, launch_prey_eaten,
-           true, 0},
-          {"pred_reproduction", T_PREDATOR, -1, nullptr, 0.0, W_LIFE, launch_pred_reproduction,
-           false, 1 + T_PREDATOR},
-          {"prey_reproduction", T_PREY, -1, nullptr, 0.0, W_LIFE, launch_prey_reproduction,
-           false, 1 + T_PREY},
-          {"grass_growth", T_GRASS, -1, nullptr, 0.0, W_GRASS, launch_grass_growth, false, 0},
-      },
-      env,
-      host_init,
-      gather_stats,
-  };
+  static const ProgramDesc d = [&] {
+    ProgramDesc desc = {
+        "predator_prey",
+        {mover_pred, mover_prey, grass},
+        {{"SPACE_MULT", 1.0}, {"REPRODUCE_PREY_PROB", 0.005}, {"REPRODUCE_PREDATOR_PROB", 0.001},
+         {"GAIN_FROM_FOOD_PREDATOR", 35}, {"GAIN_FROM_FOOD_PREY", 60}, {"GRASS_REGROW_CYCLES", 60},
+         {"PRED_PREY_INTERACTION_RADIUS", 0.1}, {"PREY_GROUP_COHESION_RADIUS", 0.12},
+         {"SAME_SPECIES_AVOIDANCE_RADIUS", 0.035}, {"GRASS_EAT_DISTANCE", 0.02},
+         {"PRED_KILL_DISTANCE", 0.02}, {"DELTA_TIME", 0.0015}, {"PRED_SPEED_ADVANTAGE", 2.0},
+         {"prey_fraction", 0.35}, {"predator_fraction", 0.025}, {"agent_density", 1600.0},
+         {"num_agents", 3200}, {"num_timesteps", 100}, {"env_size", 1.41421}},
+        {
+            {"pred_follow_prey", T_PREDATOR, T_PREY, "PRED_PREY_INTERACTION_RADIUS", 1.0, W_STEER,
+             launch_pred_follow_prey, false, 0},
+            {"prey_avoid_pred", T_PREY, T_PREDATOR, "PRED_PREY_INTERACTION_RADIUS", 1.0, W_STEER,
+             launch_prey_avoid_pred, false, 0},
+            {"prey_flock", T_PREY, T_PREY, "PREY_GROUP_COHESION_RADIUS", 1.0, W_STEER,
+             launch_prey_flock, false, 0},
+            {"pred_avoid", T_PREDATOR, T_PREDATOR, "SAME_SPECIES_AVOIDANCE_RADIUS", 1.0, W_STEER,
+             launch_pred_avoid, false, 0},
+            {"prey_move", T_PREY, -1, nullptr, 0.0, W_MOVE, launch_prey_move, false, 0},
+            {"pred_move", T_PREDATOR, -1, nullptr, 0.0, W_MOVE, launch_pred_move, false, 0},
+            {"prey_eat_or_starve", T_PREY, T_GRASS, "GRASS_EAT_DISTANCE", 1.0, W_LIFE,
+             launch_prey_eat_or_starve, true, 0},
+            {"pred_eat_or_starve", T_PREDATOR, T_PREY, "PRED_KILL_DISTANCE", 1.0, W_LIFE,
+             launch_pred_eat_or_starve, true, 0},
+            {"grass_eaten", T_GRASS, T_PREY, "GRASS_EAT_DISTANCE", 1.0, W_GRASS,
+             launch_grass_eaten, false, 0},
+            {"prey_eaten", T_PREY, T_PREDATOR, "PRED_KILL_DISTANCE", 1.0, 0u, launch_prey_eaten,
+             true, 0},
+            {"pred_reproduction", T_PREDATOR, -1, nullptr, 0.0, W_LIFE, launch_pred_reproduction,
+             false, 1 + T_PREDATOR},
+            {"prey_reproduction", T_PREY, -1, nullptr, 0.0, W_LIFE, launch_prey_reproduction,
+             false, 1 + T_PREY},
+            {"grass_growth", T_GRASS, -1, nullptr, 0.0, W_GRASS, launch_grass_growth, false, 0},
+        },
+        env,
+        host_init,
+        gather_stats,
+    };
+    for (StepDesc &st : desc.steps) st.nan = st.near_agent >= 0;
+    return desc;
+  }();
   return &d;
 }
 
