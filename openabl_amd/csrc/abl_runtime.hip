@@ -248,6 +248,7 @@ struct AgentStore {
   hipEvent_t nl_ev = nullptr;
   ListWatch nl_watch;
   uint32_t nl_c_prev = 0;
+  bool nl_unchecked = false;    // one-launch rebuilds issued since the error flag was read
   bool nl_off = false;          // lists given up for this type (rebuilt nearly every step)
   bool nl_kept = false;         // the rebuild rate was measured and the lists kept
   // whether the agents crowd into tiles that do not fit LDS (probe_tiles),
@@ -1994,7 +1995,10 @@ static int gated_rebuild(abl_sim *sim, AgentStore &b, const StepDesc &st, const 
     L.delta = &d;
     st.launch(L);
     HIP_TRY(hipGetLastError());
-    if (launched) return ABL_OK;
+    if (launched) {
+      b.nl_unchecked = true;
+      return ABL_OK;
+    }
     launch_delta(sim, b, gate, start_cur, start_other, placed);
   }
   L.nl_mode = 1;
@@ -2012,7 +2016,7 @@ static int gated_rebuild(abl_sim *sim, AgentStore &b, const StepDesc &st, const 
 // scratch with the split launches from then on.
 static int check_rebuild(abl_sim *sim) {
   for (AgentStore &s : sim->types) {
-    if (!s.nl_gate) continue;
+    if (!s.nl_gate || !s.nl_unchecked) continue;
     uint32_t err = 0;
     HIP_TRY(hipMemcpy(&err, s.nl_gate + kGateError, 4, hipMemcpyDeviceToHost));
     if (err) {
@@ -2026,6 +2030,7 @@ static int check_rebuild(abl_sim *sim) {
       return fail(ABL_ERR_DEVICE, "one-launch neighbour-list rebuild ran past its spin limit; "
                                   "results since the last synchronisation are invalid");
     }
+    s.nl_unchecked = false;
   }
   return ABL_OK;
 }

@@ -348,3 +348,28 @@ def test_crowd_is_counted_only_for_steps_on_tiles(prec):
         outs.append(field_bytes(sim.download(record_dtype(MEMBERS["circle3d"], prec))))
         sim.close()
     assert outs[0] == outs[1] == outs[2]
+
+
+def test_rebuild_errors_are_looked_for_after_every_rebuild():
+    """The error flag of one-launch rebuilds is read where such a rebuild was
+    issued since: a spin limit forced after quiet downloads is still reported, at
+    the next download, and the one after that goes on."""
+    from openabl_amd import MEMBERS, AblError, Simulation, load_library, record_dtype
+    print("case nlist error after quiet downloads", flush=True)
+    load_library().abl_rng_seed(0xDEADBEEF, 0xBEEFDEAD)
+    dt = record_dtype(MEMBERS["boids2d"], "f64")
+    sim = Simulation("boids2d", "f64", params=boids2d_params(num_agents=20000),
+                     config={"hip.nlist": 1, "hip.skin": 1e-9})
+    sim.init_agents()
+    sim.download(dt)  # nothing issued yet
+    sim.simulate(4)
+    sim.download(dt)  # rebuilds, none abandoned
+    sim.download(dt)
+    sim.set_config("hip.barrier_spins", 0)
+    sim.simulate(4)
+    with pytest.raises(AblError, match="spin limit"):
+        sim.download(dt)
+    sim.download(dt)
+    sim.simulate(2)
+    assert np.isfinite(sim.download(dt)["pos"]).all()
+    sim.close()
