@@ -16,31 +16,23 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "abl_root_rcp.hpp"
+
 namespace abl {
 
 constexpr int kMaxCols = 32;
 constexpr int kWave = 64;
 
-// Correctly rounded sqrtf.  The instruction's root s is within one unit in the
-// last place u; d = s - u is nearer exactly when f <= s * d: the midpoint's
-// square is s * d + u^2 / 4, and f and s * d are multiples of u^2 (an ulp of f
-// is at least 2^23 u^2).  Likewise s + u is nearer exactly when f > s * (s + u).
-// Each product is compared through the sign of one fma.  f is a square sum: not
-// negative.  Zero, infinity and NaN come through as they are.  For values so small that a product could
-// underflow the double root is taken: it is correctly rounded, and rounding it
-// again to float is exact because 53 >= 2*24 + 2.  (The double root everywhere
-// is 1.5 times as many issue slots in the circle models' force path.)
+// Correctly rounded sqrtf (root_from), for a square sum f: not negative.  For values
+// so small that a product could underflow the double root is taken: it is correctly
+// rounded, and rounding it again to float is exact because 53 >= 2*24 + 2.  (The
+// double root everywhere is 1.5 times as many issue slots in the circle models'
+// force path.)
 __device__ __forceinline__ float sqrt_rn_f32(float f) {
   const uint32_t bits = __builtin_bit_cast(uint32_t, f);
   constexpr uint32_t tiny = 0x0F800000u;  // 2^-96
   if (__builtin_expect(bits - 1u < tiny - 1u, 0)) return (float) __builtin_sqrt((double) f);
-  const float s = __builtin_amdgcn_sqrtf(f);
-  const uint32_t sb = __builtin_bit_cast(uint32_t, s);
-  const float below = __builtin_bit_cast(float, sb - 1u), above = __builtin_bit_cast(float, sb + 1u);
-  float r = s;
-  if (__builtin_fmaf(-below, s, f) <= 0.f) r = below;
-  if (__builtin_fmaf(-above, s, f) > 0.f) r = above;
-  return r;
+  return root_from(f, __builtin_amdgcn_sqrtf(f));
 }
 
 // Uniform grid of one agent type: cell edge = granularity / cell_scale,
@@ -482,19 +474,10 @@ __device__ __forceinline__ F div_by_recip(F a, F b, F y) {
 __device__ __forceinline__ double least_mag(double m, double x) { return __builtin_fmin(m, __builtin_fabs(x)); }
 __device__ __forceinline__ float least_mag(float m, float x) { return __builtin_fminf(m, __builtin_fabsf(x)); }
 
-// 1 / b correctly rounded for a float b with 2^-100 <= |b| <= 2^100.  Two Newton
-// steps in double from the float reciprocal (relative error 2^-22, then 2^-44,
-// then the rounding): 1 - b y is exact in the fma for a 24-bit b, so the last
-// step rounds (1/b)(1 - 2^-88), and 1/b is no nearer than 2^-77 to a midpoint of
-// doubles (b m - 1 is a non-zero multiple of 2^-76 for a midpoint m) and no
-// nearer than 2^-48 to one of floats, so the float result is right too.
+// 1 / b correctly rounded for a float b with 2^-100 <= |b| <= 2^100 (rcp_from).
 template <typename F>
 __device__ __forceinline__ F rcp_rn(float b) {
-  const double B = (double) b;
-  double y = (double) __builtin_amdgcn_rcpf(b);
-  y = __builtin_fma(y, __builtin_fma(-B, y, 1.0), y);
-  y = __builtin_fma(y, __builtin_fma(-B, y, 1.0), y);
-  return (F) y;
+  return (F) rcp_from(b, __builtin_amdgcn_rcpf(b));
 }
 
 // Same candidates in ascending id order (the reference's visiting order):
