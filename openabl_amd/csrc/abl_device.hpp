@@ -45,15 +45,14 @@ struct GridView {
   int reach;
   int dim;
   const uint32_t *start;  // ncells + 1 offsets into the cell-sorted order
-  uint32_t *nan;          // null, or a word that is set if a coordinate sorted is NaN (kept
-                          // for near loops by for_each_candidate_pos)
 };
 
-// Such coordinates are binned to cell 0 of their axis (cell_coord), and near tests
-// accept them whatever their distance.
+// Sets *nan (kept for near loops by for_each_candidate_pos, else null) if a
+// coordinate sorted is NaN: it is binned to cell 0 of its axis (cell_coord), and near
+// tests accept it whatever the distance.
 template <typename P>
-__device__ __forceinline__ void note_nan(const GridView &g, P x, P y, P z) {
-  if (g.nan && (x != x || y != y || z != z)) *g.nan = 1u;
+__device__ __forceinline__ void note_nan(uint32_t *nan, P x, P y, P z) {
+  if (nan && (x != x || y != y || z != z)) *nan = 1u;
 }
 
 __device__ __forceinline__ int cell_coord(double p, double lo, double inv, int n) {
@@ -339,7 +338,7 @@ __device__ __forceinline__ void for_each_candidate_row(const GridView &g, double
 // Visit the candidates of an agent's stencil, narrowed to the cells within rc
 // cell units of (px, py, pz), in the order of for_each_candidate:
 // visit(j, q), q the candidate's position, until it returns false.  Where there are
-// agents at NaN (GridView::nan) the stencil's first cells along each axis, which
+// agents at NaN (*noted, note_nan) the stencil's first cells along each axis, which
 // hold them, are among them too.
 //
 // A lane's walk is a chain of reads, each waited for before the next test, so
@@ -352,7 +351,7 @@ __device__ __forceinline__ void for_each_candidate_row(const GridView &g, double
 template <int AHEAD, typename F, typename Visit>
 __device__ __forceinline__ void for_each_candidate_pos(const GridView &g, const F *const *p, double px,
                                                        double py, double pz, float rc,
-                                                       Visit &&visit) {
+                                                       const uint32_t *noted, Visit &&visit) {
   const int cx = cell_coord(px, g.lo[0], g.inv_cell, g.n[0]);
   const int cy = cell_coord(py, g.lo[1], g.inv_cell, g.n[1]);
   const int cz = g.dim == 3 ? cell_coord(pz, g.lo[2], g.inv_cell, g.n[2]) : 0;
@@ -361,7 +360,7 @@ __device__ __forceinline__ void for_each_candidate_pos(const GridView &g, const 
   const float uz = g.dim == 3 ? (float) ((pz - g.lo[2]) * g.inv_cell - (double) cz) : 0.f;
   const int R = g.reach;
   const int zr = g.dim == 3 ? R : 0;
-  const bool nan = g.nan && *g.nan != 0u;
+  const bool nan = noted && *noted != 0u;
   // the slots [a, b) of the stencil row (dy, dz), none past the last row
   auto fetch = [&](int dy, int dz, uint32_t *a, uint32_t *b) {
     *a = *b = 0u;

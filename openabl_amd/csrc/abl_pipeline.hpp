@@ -80,9 +80,7 @@ static __global__ __launch_bounds__(kScanBlock) void k_scan_tiles(const uint32_t
 
 // Exclusive scan of the tile totals (one block, any number of tiles).
 static __global__ __launch_bounds__(1024) void k_scan_totals(uint32_t *__restrict__ bsum, int ntiles,
-                                                     uint32_t *__restrict__ start, int ncells,
-                                                     const uint32_t *__restrict__ gate = nullptr) {
-  if (gate && *gate == 0u) return;
+                                                     uint32_t *__restrict__ start, int ncells) {
   __shared__ uint32_t lds[kWave + 1];
   uint32_t carry = 0;
   for (int base = 0; base < ntiles; base += blockDim.x) {
@@ -97,17 +95,14 @@ static __global__ __launch_bounds__(1024) void k_scan_totals(uint32_t *__restric
 }
 
 static __global__ void k_scan_add(uint32_t *__restrict__ start, const uint32_t *__restrict__ bsum,
-                           int ncells, const uint32_t *__restrict__ gate = nullptr) {
-  if (gate && *gate == 0u) return;
+                           int ncells) {
   const int c = blockIdx.x * blockDim.x + threadIdx.x;
   if (c < ncells) start[c] += bsum[c / kScanTile];
 }
 
 static __global__ void k_scatter(const uint32_t *__restrict__ key, uint32_t *__restrict__ count,
                           const uint32_t *__restrict__ start, const int32_t *__restrict__ id,
-                          uint32_t *__restrict__ tmp_idx, int32_t *__restrict__ tmp_id, int n,
-                          const uint32_t *__restrict__ gate = nullptr) {
-  if (gate && *gate == 0u) return;
+                          uint32_t *__restrict__ tmp_idx, int32_t *__restrict__ tmp_id, int n) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   const uint32_t k = key[i];
@@ -124,9 +119,7 @@ static __global__ void k_rank_gather(const uint32_t *__restrict__ tmp_idx, const
                               const uint32_t *__restrict__ key, const uint32_t *__restrict__ start,
                               GatherCols g, int32_t *__restrict__ id_out, int n,
                               uint32_t *__restrict__ skey_out = nullptr,
-                              uint32_t *__restrict__ count_out = nullptr,
-                              const uint32_t *__restrict__ gate = nullptr) {
-  if (gate && *gate == 0u) return;
+                              uint32_t *__restrict__ count_out = nullptr) {
   const int s = blockIdx.x * blockDim.x + threadIdx.x;
   if (s >= n) return;
   const uint32_t src = tmp_idx[s];
@@ -159,13 +152,13 @@ constexpr int kSmallAgents = 4096;
 constexpr int kSmallCells = 8192;
 constexpr int kSmallBlock = 1024;
 
-// NAN_NOTED: notes coordinates that are NaN (GridView::nan).
+// NAN_NOTED: coordinates that are NaN are noted (note_nan).
 template <typename P, bool NAN_NOTED>
 static __global__ __launch_bounds__(kSmallBlock) void k_sort_small(
     const P *__restrict__ px, const P *__restrict__ py, const P *__restrict__ pz, GridView g, int ncells,
     int n, const int32_t *__restrict__ id, GatherCols gc, int32_t *__restrict__ id_out,
     uint32_t *__restrict__ skey_out, uint32_t *__restrict__ start, uint32_t *__restrict__ count,
-    uint32_t *__restrict__ bsum) {
+    uint32_t *__restrict__ bsum, uint32_t *nan) {
   __shared__ uint32_t cell[kSmallCells];
   __shared__ int32_t sid[kSmallAgents];
   __shared__ uint16_t ssrc[kSmallAgents];
@@ -176,8 +169,11 @@ static __global__ __launch_bounds__(kSmallBlock) void k_sort_small(
   const int tid = (int) threadIdx.x;
   for (int c = tid; c < ncells; c += kSmallBlock) cell[c] = 0u;
   __syncthreads();
+  bool bad = false;  // a coordinate that is NaN
   auto key_of = [&](int i) {
-    const int3 c = cell_of<P>(g, px[i], py[i], g.dim == 3 ? pz[i] : (P) 0);
+    const P x = px[i], y = py[i], z = g.dim == 3 ? pz[i] : (P) 0;
+    if constexpr (NAN_NOTED) bad = bad || x != x || y != y || z != z;
+    const int3 c = cell_of<P>(g, x, y, z);
     return ((uint32_t) c.z * (uint32_t) g.n[1] + (uint32_t) c.y) * (uint32_t) g.n[0] + (uint32_t) c.x;
   };
   uint32_t key[kItems];
@@ -185,11 +181,9 @@ static __global__ __launch_bounds__(kSmallBlock) void k_sort_small(
   for (int u = 0; u < kItems; u++) {
     const int i = tid + u * kSmallBlock;
     key[u] = i < n ? key_of(i) : 0u;
-    if (i < n) {
-      atomicAdd(&cell[key[u]], 1u);
-      if constexpr (NAN_NOTED) note_nan<P>(g, px[i], py[i], g.dim == 3 ? pz[i] : (P) 0);
-    }
+    if (i < n) atomicAdd(&cell[key[u]], 1u);
   }
+  if (NAN_NOTED && bad) *nan = 1u;
   __syncthreads();
   // each thread's run of cells: counts out, offsets out and into LDS
   uint32_t v[kCells], sum = 0;
@@ -387,12 +381,12 @@ static __global__ void k_bin_delta(const P *__restrict__ px, const P *__restrict
                                    const P *__restrict__ pz, GridView g,
                                    const uint32_t *__restrict__ skey, uint32_t *__restrict__ key,
                                    uint32_t *__restrict__ count, uint32_t *__restrict__ bsum,
-                                   MoverLists ml, uint32_t gen, int n,
+                                   MoverLists ml, uint32_t gen, int n, uint32_t *nan,
                                    const uint32_t *__restrict__ gate = nullptr) {
   if (gate && *gate == 0u) return;  // neighbour-list mode: no rebuild this timestep
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  note_nan<P>(g, px[i], py[i], g.dim == 3 ? pz[i] : (P) 0);
+  note_nan<P>(nan, px[i], py[i], g.dim == 3 ? pz[i] : (P) 0);
   bin_delta_item(i, cell_key<P>(g, px, py, pz, i), skey, key, count, bsum, ml, gen);
 }
 

@@ -210,6 +210,7 @@ struct AgentStore {
   size_t ncells = 0, cells_cap = 0;
   bool grid_valid = false;
   GridView gv{};
+  uint32_t *nan = nullptr;  // note_nan
   double cell = 0.0;
   // delta re-sort (abl_pipeline.hpp): sorted keys of the stored order, mover
   // lists, and whether the stored order is the (cell, id) order of the last
@@ -596,11 +597,12 @@ __global__ __launch_bounds__(256) void k_ids_to_aos(char *__restrict__ aos, ColX
 
 template <typename P>
 __global__ void k_bin(const P *__restrict__ px, const P *__restrict__ py, const P *__restrict__ pz,
-                      GridView g, uint32_t *__restrict__ key, uint32_t *__restrict__ count, int n) {
+                      GridView g, uint32_t *__restrict__ key, uint32_t *__restrict__ count, int n,
+                      uint32_t *nan) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   const uint32_t k = cell_key<P>(g, px, py, pz, i);
-  note_nan<P>(g, px[i], py[i], g.dim == 3 ? pz[i] : (P) 0);
+  note_nan<P>(nan, px[i], py[i], g.dim == 3 ? pz[i] : (P) 0);
   key[i] = k;
   atomicAdd(&count[k], 1u);
 }
@@ -905,10 +907,11 @@ static int setup_grid(abl_sim *sim, AgentStore &s) {
   }
   s.ncells = ncells;
   g.start = s.startb[s.start_cur];
-  // behind the cells' counts: cleared with them, and else left set (a full sort
-  // clears it)
+  // the word behind the cells' counts: cleared with them by a full sort, else left
+  // set
+  s.nan = nullptr;
   for (const StepDesc &st : sim->prog->steps)
-    if (st.nan && &sim->types[st.near_agent] == &s) g.nan = s.count + ncells;
+    if (st.nan && &sim->types[st.near_agent] == &s) s.nan = s.count + ncells;
   s.gv = g;
   return ABL_OK;
 }
@@ -930,10 +933,10 @@ static void launch_bin(abl_sim *sim, AgentStore &s, bool delta, int n,
   if (delta) {
     MoverLists ml{s.dirty, s.mhead, s.mnext};
     hipLaunchKernelGGL(k_bin_delta<P>, grid_blocks(n, 256), 256, 0, sim->stream, px, py, pz, s.gv,
-                       s.skey[s.skey_cur], s.key, s.count, s.bsum, ml, s.gen, n, gate);
+                       s.skey[s.skey_cur], s.key, s.count, s.bsum, ml, s.gen, n, s.nan, gate);
   } else {
     hipLaunchKernelGGL(k_bin<P>, grid_blocks(n, 256), 256, 0, sim->stream, px, py, pz, s.gv, s.key,
-                       s.count, n);
+                       s.count, n, s.nan);
   }
 }
 
@@ -942,12 +945,12 @@ template <typename P>
 static void launch_sort_small(abl_sim *sim, AgentStore &s, int n, int nc, uint32_t *start_new,
                               const GatherCols &gc) {
   const int pc = s.pos_col;
-  const auto kernel = s.gv.nan ? k_sort_small<P, true> : k_sort_small<P, false>;
+  const auto kernel = s.nan ? k_sort_small<P, true> : k_sort_small<P, false>;
   hipLaunchKernelGGL(kernel, 1, kSmallBlock, 0, sim->stream, (const P *) col_cur(s, pc),
                      (const P *) col_cur(s, pc + 1),
                      (const P *) (s.dim == 3 ? col_cur(s, pc + 2) : nullptr), s.gv, nc, n,
                      s.id[s.id_cur], gc, s.id[1 - s.id_cur], s.skey[1 - s.skey_cur], start_new, s.count,
-                     s.bsum);
+                     s.bsum, s.nan);
 }
 
 // The delta re-sort's kernels into the other buffers (start_new, skey, ids,
@@ -2089,6 +2092,7 @@ static int launch_step(abl_sim *sim, const StepDesc &st, uint32_t ordinal) {
     L.nb_n = (int) b.n;
     for (size_t c = 0; c < b.cols.size(); c++) L.nb.c[c] = col_cur(b, (int) c);
     L.nb_id = b.id[b.id_cur];
+    L.nan = b.nan;
     L.grid = b.gv;
     L.grid.reach = reach_for(b, r);
     L.near_t = sqrtf_le_threshold(r);

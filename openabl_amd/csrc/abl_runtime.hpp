@@ -149,7 +149,7 @@ struct StepDesc {
   // whether the launcher walks this stencil on the tiles (nl_mode 0); null: yes,
   // wherever it tiles at all
   bool (*walks_tiles)(const StepLaunch &);
-  // the near loop looks at GridView::nan
+  // the near loop looks at StepLaunch::nan
   bool nan;
 };
 
@@ -205,6 +205,7 @@ struct StepLaunch {
   int nb_n;            // agents of the near type
   ColSet nb;           // near type, cell-sorted
   const int32_t *nb_id;
+  const uint32_t *nan;   // StepDesc::nan: set if a position of the near type is NaN
   GridView grid;
   float near_t;        // T = max{f : sqrtf(f) <= radius}
   const double *params;  // host copy, indexed as ProgramDesc::params

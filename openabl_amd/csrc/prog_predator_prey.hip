@@ -49,6 +49,7 @@ struct Args {
   uint8_t *born;
   GridView g;
   float near_t, rc;
+  const uint32_t *nan;
   int n;
   uint64_t seed, t;
   uint32_t ordinal;
@@ -89,7 +90,7 @@ __device__ __forceinline__ void near_loop(const Args<F> &a, F x, F y, const F *q
                              [&](uint32_t j) { visit(j, qx[j], qy[j]); });
   } else {
     const F *const p[3] = {qx, qy, nullptr};
-    for_each_candidate_pos<8, F>(a.g, p, (double) x, (double) y, 0.0, a.rc, [&](uint32_t j, const F *q) {
+    for_each_candidate_pos<8, F>(a.g, p, (double) x, (double) y, 0.0, a.rc, a.nan, [&](uint32_t j, const F *q) {
       visit(j, q[0], q[1]);
       return true;
     });
@@ -357,6 +358,7 @@ Args<F> make_args(const StepLaunch &L) {
   a.g = L.grid;
   a.near_t = L.near_t;
   a.rc = L.rc;
+  a.nan = L.nan;
   a.n = L.n;
   a.seed = L.seed;
   a.t = L.timestep;
