@@ -139,7 +139,8 @@ def kernel_name(precision: str) -> str:
 # the sources the neighbour kernel is compiled from: a committed profile
 # figure is used only while these hash as they did when it was measured
 KERNEL_SOURCES = ("openabl_amd/csrc/abl_tile.hpp", "openabl_amd/csrc/abl_device.hpp",
-                  "openabl_amd/csrc/abl_pipeline.hpp", "openabl_amd/csrc/abl_runtime.hpp",
+                  "openabl_amd/csrc/abl_root_rcp.hpp", "openabl_amd/csrc/abl_pipeline.hpp",
+                  "openabl_amd/csrc/abl_runtime.hpp",
                   "openabl_amd/csrc/prog_boids2d.hip")
 
 

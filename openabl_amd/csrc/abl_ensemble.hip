@@ -16,7 +16,8 @@
 // radius): one set of lists over the concatenated slots, built after a sort
 // and walked while no agent of the member has moved more than skin / 2 since
 // (abl_tile.hpp).  Each member has its own rebuild gate, set by its own
-// agents, so it rebuilds on exactly the timesteps a run of it alone would.
+// agents, and its own list capacity, so it rebuilds, and enters its lists anew with
+// more room, on exactly the timesteps a run of it alone would.
 // Re-sort and list build are one launch that returns at once when no member is
 // due (tiled_rebuild_multi); it re-sorts the agents of the members due by the
 // delta method into the other buffers, and the list build copies them back, so
@@ -444,7 +445,7 @@ static int issue_build(abl_ensemble *e) {
 
 // The gated rebuild of the current timestep: one launch (tiled_rebuild_multi), or
 // four (look), which cost a timestep without a rebuild about 10 us more and one
-// with a rebuild 50 us less; the same results.
+// on which all members rebuild half (tiled_rebuild_multi); the same results.
 static int issue_rebuild(abl_ensemble *e) {
   DeltaArgs d{};
   const int b = e->cur;
@@ -873,8 +874,8 @@ static int issue_step(abl_ensemble *e) {
 // every timestep: 30 members of up to 8,192 boids, FP32, 18 us per timestep, and
 // 90 from the first list that outgrew its capacity on.
 //
-// One launch per rebuild or four: one above a quarter of the timesteps, back below
-// an eighth, so that a rate in between does not switch to and fro.
+// One launch per rebuild or four: four from a quarter of the timesteps on, back
+// below an eighth, so that a rate in between does not switch to and fro.
 static int look(abl_ensemble *e) {
   const uint64_t t = e->timestep - 1;
   const size_t M = e->mem.size();

@@ -1052,7 +1052,10 @@ __device__ __forceinline__ bool rebuild_phases(const DeltaArgs &d, uint32_t chun
 // rebuild took 1,840 us for 1,000,003 agents (the same phases as four launches
 // 125 us) and 102 us for 1,000; with one item per block and phase, released by
 // one thread, and the tiles not claimed at all it takes 310 us and 60 us; with the
-// counters in shards 285 us for 1,048,576 boids and 36 for 1,000.
+// counters in shards 270 us for 1,048,576 boids and 34 for 1,000.  A timestep of
+// boids2d that rebuilds, and one that does not, with one launch 328 and 55 us for
+// 1,048,576 agents, 71 and 15 for 65,536; with four launches (hip.rebuild=split) 197
+// and 60, 51 and 19.
 template <class M, int TX, int TY, int TZ, int RM>
 __global__ __launch_bounds__(256) void tiled_rebuild(typename M::Args a, NListArgs nl,
                                                       DeltaArgs d) {
@@ -1270,11 +1273,11 @@ __global__ __launch_bounds__(256) void tiled_list_build_multi(const typename M::
 
 // The gated re-sort and list build of the members due, in one launch
 // (tiled_rebuild), over the chunks of those members only.  30 members of 1,000 to
-// 65,536 boids: a timestep with no member due 37 us (of it 4.6 us for this launch
-// that returns) against 48 us with seven gated launches for the full sort and the list
-// build.  Where members are due on most timesteps the ensemble takes the re-sort's
+// 65,536 boids: a timestep with no member due 35 us (of it 4.6 us for this launch
+// that returns) against 46 us with seven gated launches for the full sort and the list
+// build.  Where members are due on many timesteps the ensemble takes the re-sort's
 // phases as launches of their own instead (look): every member due on every
-// timestep 230 us this way, 130 with four launches.
+// timestep 217 us this way, 109 with four launches.
 template <class M, int TX, int TY, int TZ, int RM>
 __global__ __launch_bounds__(256) void tiled_rebuild_multi(const typename M::Args *__restrict__ args,
                                                             EnsTiles e, NListArgs nl, DeltaArgs d) {
@@ -1426,8 +1429,6 @@ inline void launch_tiled(typename M::Args a, const StepLaunch &L) {
 
 constexpr unsigned kRebuildBlocks = 1024;
 
-// Launch the neighbour-list build (mode 1) or the step through the lists
-// (mode 2) for a tile shape; same tiles and LDS budget as tiled_step.
 // Blocks of a one-launch rebuild, 0 if the device cannot tell: a block per two
 // chunks of agents and per tile, a multiple of the 8 XCDs, at most kRebuildBlocks
 // and what the CUs hold at once (the work queue does not need them resident
@@ -1457,6 +1458,9 @@ inline unsigned rebuild_grid(const void *kernel, size_t smem, int n, unsigned nt
   return std::min(std::min(grid, kRebuildBlocks), (std::max(chunks, ntiles) + 7u) & ~7u);
 }
 
+// Launch the neighbour-list build (mode 1), the step through the lists (mode 2) or
+// the gated rebuild in one launch (mode 3, *delta) for a tile shape; same tiles and
+// LDS budget as tiled_step.
 template <class M, int TX, int TY, int TZ, int RM>
 inline void launch_list(typename M::Args a, const GridView &g, float occupancy, int block,
                         hipStream_t stream, float slack, const NListArgs &nl, int mode,

@@ -373,9 +373,9 @@ void launch_c(const StepLaunch &L) {
 // By default the LDS tiles serve the lists alone and the stencil is walked by the
 // untiled kernel, which is the faster one at every size measured: a force per
 // candidate hides its reads, and it has as many blocks as the agents fill.  FP64,
-// circle with 1,000 / 64,000 / 1,000,003 agents 25.6 / 37.7 / 114 us per timestep
-// (tiles 50 / 74 / 142), circle3d with 2,000 / 200,003 agents 337 / 593 us (tiles
-// 1,654 / 605); FP32 alike.  (Its buffer offsets end at 2^31 bytes.)  A caller that
+// circle with 1,000 / 64,000 / 1,000,003 agents 26.6 / 37.5 / 107 us per timestep
+// with its re-sort (tiles 27.5 / 40.8 / 130), FP32 with 1,000,003 91 (110), circle3d
+// with 2,000 agents 387 us (1,867).  (Its buffer offsets end at 2^31 bytes.)  A caller that
 // asks for a tile shape gets it.  Not for FP32-compensated, whose tiles round
 // offsets from the tile's own origin: lists and stencil would no longer agree to
 // the bit.

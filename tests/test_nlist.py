@@ -28,7 +28,9 @@ from orclib import Oracle, boids2d_params, circle3d_params, circle_params, field
 pytestmark = pytest.mark.gpu
 
 
-def run(model, prec, params, steps, crowded=None, **cfg):
+def run(model, prec, params, steps, crowded=None, seen=None, **cfg):
+    """The agents after each of `steps` timesteps; `seen`: a dict of what
+    Simulation.inspect() names, whose lists take the values then."""
     from openabl_amd import MEMBERS, Simulation, load_library, record_dtype
     load_library().abl_rng_seed(0xDEADBEEF, 0xBEEFDEAD)
     sim = Simulation(model, prec, params=params, config=cfg)
@@ -41,6 +43,8 @@ def run(model, prec, params, steps, crowded=None, **cfg):
         out.append(sim.download(record_dtype(MEMBERS[model], prec)))
         if crowded is not None:
             assert sim.inspect("crowded") == crowded
+        for what, values in (seen or {}).items():
+            values.append(sim.inspect(what))
     sim.close()
     return out
 
@@ -226,13 +230,17 @@ def test_lists_given_up_when_rebuilt_every_step():
     walk bit for bit.  With hip.nlist=1 given, the lists stay (same bytes)."""
     print("case nlist given up: circle 65536, 120 steps", flush=True)
     params = circle_params(num_agents=65536, rho=0.1024, r=2.5)
-    steps = (20, 60, 120)
     cells = {"hip.cell_inflate": 1.0 + 0.05}  # the list mode's cells in both runs
-    a = run("circle", "f64", params, steps, **cells)
+    steps = (16, 20, 60, 120)
+    seen = {"lists": [], "lists_given_up": []}
+    a = run("circle", "f64", params, steps, seen=seen, **cells)
+    assert seen == {"lists": [1, 0, 0, 0], "lists_given_up": [0, 1, 1, 1]}
     b = run("circle", "f64", params, steps, **dict(cells, **{"hip.nlist": 0}))
     for t, x, y in zip(steps, a, b):
         assert field_bytes(x) == field_bytes(y), t
-    c = run("circle", "f64", params, (40,), **dict(cells, **{"hip.nlist": 1}))
+    seen = {"lists": [], "lists_given_up": []}
+    c = run("circle", "f64", params, (40,), seen=seen, **dict(cells, **{"hip.nlist": 1}))
+    assert seen == {"lists": [1], "lists_given_up": [0]}
     assert field_bytes(c[0]) == field_bytes(run("circle", "f64", params, (40,),
                                                 **dict(cells, **{"hip.nlist": 0}))[0])
 
@@ -269,9 +277,12 @@ def test_lists_grown_while_agents_draw_together(prec):
     bits."""
     print(f"case nlist growing {prec}", flush=True)
     params = dict(boids2d_params(num_agents=3001), time_scale=0.05, steer_scale=3.0)
-    steps = (60, 200)
-    a = run("boids2d", prec, params, steps,
+    steps = (1, 60, 200)
+    seen = {"list_capacity": []}
+    a = run("boids2d", prec, params, steps, seen=seen,
             **{"hip.nlist": 1, "hip.skin": 1e-9, "hip.cell_inflate": 1})
+    first, _, last = seen["list_capacity"]
+    assert last > first
     b = run("boids2d", prec, params, steps, **{"hip.nlist": 0})
     for t, x, y in zip(steps, a, b):
         assert field_bytes(x) == field_bytes(y), t
