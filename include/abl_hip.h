@@ -260,7 +260,8 @@ int abl_hip_log_text(abl_sim *sim, char *buf, size_t capacity, size_t *len);
  * Member m's initialisation starts from abl_ens_member_seed(s0, s1, m); each
  * member's result is bit-identical to a run of it alone from that state with
  * the same "hip.cell_scale", "hip.tile", "hip.nlist" (given, not left at its
- * default), "hip.skin" and "hip.list_cap".  Neighbour lists ("hip.nlist", default 1, when every member
+ * default), "hip.skin" and "hip.list_cap" (but for tiles whose halo holds 65,535
+ * agents or more, which keep no lists: a run alone may cut its tiles smaller).  Neighbour lists ("hip.nlist", default 1, when every member
  * has the same near radius): one set over all members' agents, and a rebuild
  * gate and list capacity per member, so a member re-sorts, rebuilds and grows its
  * lists on exactly the timesteps a run of it alone does.  Programs: boids2d. */
